@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../../include/cholespy_amd.h"
+#include "block_inverse.hpp"
 #include "block_plan.hpp"
 #include "common.hpp"
 #include "launchers.hpp"
@@ -224,8 +225,9 @@ struct cholespy_gpu_solver {
     std::vector<int> host_levels[2], host_row_level[2];
     // Pattern of the uploaded factor, kept for cholespy_solver_refactor:
     // column form of L, for each position of the row form the column-form
-    // position it copies, and the block plan's structure (values cleared).
-    std::vector<int> host_colptr, host_rowidx, csr_src;
+    // position it copies (device), and the block plan's structure.
+    std::vector<int> host_colptr, host_rowidx;
+    int *csr_src = nullptr;
     BlockPlan host_plan;
 };
 
@@ -282,8 +284,9 @@ std::vector<int> device_tasks(const BlockPlan &P, const std::vector<int> &tasks,
     return out;
 }
 
-// Copies a (possibly merged) block plan to the device in the handle's
-// precision; blk_sys maps blocks to systems for a batch.
+// Copies the structure of a (possibly merged) block plan to the device and
+// allocates its values, which fill_plan_values forms there; blk_sys maps
+// blocks to systems for a batch.
 int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<int> *blk_sys) {
     DeviceBlockPlan &d = s->plan;
     d.release();
@@ -326,66 +329,65 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
         HIP_TRY(upload(&d.ftask_wide, fw.data(), fw.size()));
         HIP_TRY(upload(&d.btask_wide, bw.data(), bw.size()));
     }
-    const size_t me = (size_t)d.m_entries;
-    if (s->fbytes == 4) {
-        std::vector<float> f(me), b(me);
-        for (size_t i = 0; i < me; ++i) {
-            f[i] = (float)P.mfwd[i];
-            b[i] = (float)P.mbwd[i];
-        }
-        HIP_TRY(upload(reinterpret_cast<float **>(&d.mfwd), f.data(), me));
-        HIP_TRY(upload(reinterpret_cast<float **>(&d.mbwd), b.data(), me));
-    } else {
-        HIP_TRY(upload(reinterpret_cast<double **>(&d.mfwd), P.mfwd.data(), me));
-        HIP_TRY(upload(reinterpret_cast<double **>(&d.mbwd), P.mbwd.data(), me));
-    }
+    const size_t me = (size_t)d.m_entries, fb = (size_t)s->fbytes;
+    HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mfwd), me * fb));
+    HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mbwd), me * fb));
     for (auto &row : s->grid_blocks)
         for (int &g : row) g = 0;
     s->buffers_path = -1;
     return CHOLESPY_OK;
 }
 
-// Copies the values of L (column form, in the order of host_rowidx) into the
-// row and column forms on the device, in the handle's precision.
-int upload_factor_values(cholespy_gpu_solver *s, const double *val) {
-    const int64_t nnz = s->nnz;
-    const size_t fb = (size_t)s->fbytes;
-    std::vector<char> lv((size_t)nnz * fb), uv((size_t)nnz * fb);
-    if (s->fbytes == 4) {
-        float *l = reinterpret_cast<float *>(lv.data()), *u = reinterpret_cast<float *>(uv.data());
-        for (int64_t p = 0; p < nnz; ++p) {
-            l[p] = (float)val[s->csr_src[(size_t)p]];
-            u[p] = (float)val[p];
-        }
-    } else {
-        double *l = reinterpret_cast<double *>(lv.data());
-        for (int64_t p = 0; p < nnz; ++p) l[p] = val[s->csr_src[(size_t)p]];
-        std::memcpy(uv.data(), val, (size_t)nnz * 8);
+// Device memory freed at the end of a scope.
+struct DeviceTemp {
+    void *p = nullptr;
+    ~DeviceTemp() { dev_free(p); }
+    template <typename T>
+    hipError_t put(const T *src, size_t count) {
+        T *q = nullptr;
+        const hipError_t e = upload(&q, src, count);
+        p = q;
+        return e;
     }
-    HIP_TRY(hipMemcpy(s->lvals, lv.data(), (size_t)nnz * fb, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(s->uvals, uv.data(), (size_t)nnz * fb, hipMemcpyHostToDevice));
+    template <typename T>
+    const T *as() const { return static_cast<const T *>(p); }
+};
+
+// Forms the plan's dense values on the device (block_inverse.hip) from L in
+// compressed columns (colptr: host, rowidx and val: device).
+int fill_plan_values(cholespy_gpu_solver *s, const BlockPlan &P, const int64_t *colptr, const int *rowidx,
+                     const double *val) {
+    DeviceBlockPlan &d = s->plan;
+    DeviceTemp tcol;
+    HIP_TRY(tcol.put(colptr, (size_t)P.n + 1));
+    const InverseArgs args{tcol.as<int64_t>(), rowidx, val, d.start, d.rptr, d.rlist, d.moff};
+    HIP_TRY(fill_block_plan_on_device(P, args, s->fbytes, d.mfwd, d.mbwd));
     return CHOLESPY_OK;
 }
 
-// Copies the values of M_B (both layouts) into the device plan, whose
-// structure they must match.
-int upload_plan_values(cholespy_gpu_solver *s, const BlockPlan &P) {
-    DeviceBlockPlan &d = s->plan;
-    const size_t me = (size_t)d.m_entries;
-    if (P.mfwd.size() != me || P.mbwd.size() != me)
-        return fail(CHOLESPY_ERR_STATE, "block plan values do not match the uploaded plan");
-    if (s->fbytes == 4) {
-        std::vector<float> f(me), b(me);
-        for (size_t i = 0; i < me; ++i) {
-            f[i] = (float)P.mfwd[i];
-            b[i] = (float)P.mbwd[i];
-        }
-        HIP_TRY(hipMemcpy(d.mfwd, f.data(), me * sizeof(float), hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(d.mbwd, b.data(), me * sizeof(float), hipMemcpyHostToDevice));
-    } else {
-        HIP_TRY(hipMemcpy(d.mfwd, P.mfwd.data(), me * sizeof(double), hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(d.mbwd, P.mbwd.data(), me * sizeof(double), hipMemcpyHostToDevice));
+// The values val of L (column form, host) on the device: both compressed
+// forms in the handle's precision and the block plan's dense values.
+int upload_values(cholespy_gpu_solver *s, const double *val) {
+    DeviceTemp tval;
+    HIP_TRY(tval.put(val, (size_t)s->nnz));
+    HIP_TRY(launch_cast_factor(s->fbytes, s->nnz, tval.as<double>(), s->csr_src, s->lvals, s->uvals));
+    const std::vector<int64_t> colptr(s->host_colptr.begin(), s->host_colptr.end());
+    return fill_plan_values(s, s->host_plan, colptr.data(), s->ucols, tval.as<double>());
+}
+
+// Plans the uploaded pattern with base options `base` and uploads the
+// structure (the values follow).
+int plan_system(cholespy_gpu_solver *s, const BlockPlanOptions &base) {
+    BlockPlan P;
+    try {
+        P = build_block_plan_structure(s->n, s->host_colptr.data(), s->host_rowidx.data(), plan_options(base));
+    } catch (const std::exception &ex) {
+        return fail(CHOLESPY_ERR_INVALID_ARGUMENT, ex.what());
     }
+    const int rc = upload_plan(s, P);
+    if (rc != CHOLESPY_OK) return rc;
+    s->host_plan = std::move(P);
+    s->plan_base = base;
     return CHOLESPY_OK;
 }
 
@@ -537,6 +539,7 @@ int cholespy_solver_destroy(cholespy_gpu_solver *s) {
     dev_free(s->urowptr);
     dev_free(s->ucols);
     dev_free(s->uvals);
+    dev_free(s->csr_src);
     dev_free(s->order[0]);
     dev_free(s->order[1]);
     dev_free(s->y);
@@ -621,26 +624,15 @@ int cholespy_solver_upload_factor(cholespy_gpu_solver *s, const int *perm, const
     HIP_TRY(hipMemcpy(s->urowptr, colptr, ((size_t)n + 1) * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(s->ucols, rowidx, (size_t)nnz * sizeof(int), hipMemcpyHostToDevice));
     s->nnz = nnz;
-    s->csr_src.swap(csr_src);
+    dev_free(s->csr_src);
+    HIP_TRY(upload(&s->csr_src, csr_src.data(), csr_src.size()));
     s->host_colptr.assign(colptr, colptr + n + 1);
     s->host_rowidx.assign(rowidx, rowidx + nnz);
-    int rc = upload_factor_values(s, val);
-    if (rc != CHOLESPY_OK) return rc;
     s->analysed[0] = s->analysed[1] = false;
-
-    BlockPlanOptions opt = plan_options(s->plan_base);
-    BlockPlan P;
-    try {
-        P = build_block_plan(n, colptr, rowidx, val, opt);
-    } catch (const std::exception &ex) {
-        return fail(CHOLESPY_ERR_INVALID_ARGUMENT, ex.what());
-    }
-    rc = upload_plan(s, P);
+    int rc = plan_system(s, s->plan_base);
     if (rc != CHOLESPY_OK) return rc;
-    // The structure stays on the host for refactorisations; the values are on the device.
-    std::vector<double>().swap(P.mfwd);
-    std::vector<double>().swap(P.mbwd);
-    s->host_plan = std::move(P);
+    rc = upload_values(s, val);
+    if (rc != CHOLESPY_OK) return rc;
     s->uploaded = true;
     s->buffers_path = -1;
     return CHOLESPY_OK;
@@ -681,16 +673,10 @@ int cholespy_solver_refactor(cholespy_gpu_solver *s, const double *val, int64_t 
         if (!(d > 0.0) || !std::isfinite(d))
             return fail(CHOLESPY_ERR_INVALID_ARGUMENT, "factor diagonal must be positive and finite");
     }
-    BlockPlan &P = s->host_plan;
-    fill_block_plan_values(P, s->host_colptr.data(), s->host_rowidx.data(), val, plan_options(s->plan_base).threads);
     // Solves still in flight read the old values: wait for them before
     // overwriting anything.
     HIP_TRY(hipDeviceSynchronize());
-    int rc = upload_factor_values(s, val);
-    if (rc == CHOLESPY_OK) rc = upload_plan_values(s, P);
-    std::vector<double>().swap(P.mfwd);
-    std::vector<double>().swap(P.mbwd);
-    return rc;
+    return upload_values(s, val);
 }
 
 int cholespy_solver_analyze(cholespy_gpu_solver *s, int lower, int *n_levels) {
@@ -1277,7 +1263,7 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
                 for (int i = (int)w; i < ns; i += (int)hw) {
                     const auto &h = s->pending[i];
                     try {
-                        plans[i] = build_block_plan(s->sys_n[i], h.colptr.data(), h.rowidx.data(), h.val.data(), opt);
+                        plans[i] = build_block_plan_structure(s->sys_n[i], h.colptr.data(), h.rowidx.data(), opt);
                     } catch (const std::exception &ex) {
                         errors[i] = ex.what();
                     }
@@ -1317,8 +1303,6 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
             blk_sys.push_back(i);
         }
         for (int v : P.rlist) G.rlist.push_back(v + R0);
-        G.mfwd.insert(G.mfwd.end(), P.mfwd.begin(), P.mfwd.end());
-        G.mbwd.insert(G.mbwd.end(), P.mbwd.begin(), P.mbwd.end());
         for (int r = 0; r < s->sys_n[i]; ++r) G.contrib_ptr.push_back(P.contrib_ptr[r] + C0);
         for (int v : P.contrib_slot) G.contrib_slot.push_back(v + S0);
         for (int v : P.gslot) G.gslot.push_back(v >= 0 ? v + S0 : -1);
@@ -1386,6 +1370,23 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
     HIP_TRY(hipMemcpy(s->perm, gperm.data(), (size_t)s->n * sizeof(int), hipMemcpyHostToDevice));
     int rc = upload_plan(s, G, &blk_sys);
     if (rc != CHOLESPY_OK) return rc;
+    {
+        // The factors one after another, as the block-diagonal factor of the merged plan.
+        std::vector<int64_t> colptr{0};
+        std::vector<int> rowidx;
+        std::vector<double> val;
+        for (int i = 0; i < ns; ++i) {
+            const auto &h = s->pending[i];
+            for (int j = 0; j < s->sys_n[i]; ++j) colptr.push_back((int64_t)rowidx.size() + h.colptr[j + 1]);
+            for (int v : h.rowidx) rowidx.push_back(v + s->sys_row0[i]);
+            val.insert(val.end(), h.val.begin(), h.val.end());
+        }
+        DeviceTemp trow, tval;
+        HIP_TRY(trow.put(rowidx.data(), rowidx.size()));
+        HIP_TRY(tval.put(val.data(), val.size()));
+        rc = fill_plan_values(s, G, colptr.data(), trow.as<int>(), tval.as<double>());
+        if (rc != CHOLESPY_OK) return rc;
+    }
     dev_free(s->blk_sys);
     HIP_TRY(upload(&s->blk_sys, blk_sys.data(), blk_sys.size()));
     dev_free(s->sys_k);
@@ -1687,20 +1688,9 @@ bool same_plan(const BlockPlanOptions &a, const BlockPlanOptions &b) {
 int replan(cholespy_gpu_solver *s, const double *val, const BlockPlanOptions &base) {
     if (same_plan(base, s->plan_base) && s->uploaded) return CHOLESPY_OK;
     HIP_TRY(hipDeviceSynchronize());
-    BlockPlan P;
-    try {
-        P = build_block_plan(s->n, s->host_colptr.data(), s->host_rowidx.data(), val, plan_options(base));
-    } catch (const std::exception &ex) {
-        return fail(CHOLESPY_ERR_INVALID_ARGUMENT, ex.what());
-    }
-    int rc = upload_plan(s, P);
-    if (rc != CHOLESPY_OK) return rc;
-    std::vector<double>().swap(P.mfwd);
-    std::vector<double>().swap(P.mbwd);
-    s->host_plan = std::move(P);
-    s->plan_base = base;
-    s->buffers_path = -1;
-    return CHOLESPY_OK;
+    int rc = plan_system(s, base);
+    if (rc == CHOLESPY_OK) rc = upload_values(s, val);
+    return rc;
 }
 
 int apply_config(cholespy_gpu_solver *s, const double *val, int k, const TuneConfig &c) {
