@@ -1,6 +1,7 @@
 // Dense values of the block plan (block_plan.hpp), formed on the GPU in FP64
 // from the factor L and rounded once to the solver's precision:
-//   M_B = [ L_BB^{-1} ; -L_RB L_BB^{-1} ]   per block, in both packed layouts.
+//   M_B = [ L_BB^{-1} ; -L_RB L_BB^{-1} ]   per block, in both packed layouts;
+//   S^{-1} = L_TT^{-T} L_TT^{-1}            for a dense top block, full square.
 //
 // Blocks of up to 64 rows (nearly all of them) take one workgroup each, all
 // in LDS: scatter L_BB, invert it column per thread, then multiply L_RB by
@@ -82,9 +83,9 @@ __global__ __launch_bounds__(kThreads) void small_blocks(InverseArgs a, const in
         for (int i = tid; i < kSmall * kLd; i += kThreads) L[i] = 0.0;
         __syncthreads();
         for (int c = wave; c < m; c += kThreads / 64) {
-            const int j = a0 + c;
+            const int j = a.src[a0 + c];
             for (int64_t p = a.colptr[j] + lane; p < a.colptr[j + 1]; p += 64) {
-                const int i = a.rowidx[p];
+                const int i = a.rank[a.rowidx[p]];
                 if ((i < a0 + m) != diag) continue;
                 const int q = diag ? i - a0 : find_row(a.rlist + r0, R, i) - q0;
                 if (q >= 0 && q < kSmall) L[q * kLd + c] = a.val[p];
@@ -139,9 +140,9 @@ __global__ __launch_bounds__(64) void scatter_columns(InverseArgs a, const Inver
     const InverseColumn col = cols[blockIdx.x];
     const int a0 = a.start[col.block], m = a.start[col.block + 1] - a0, r0 = a.rptr[col.block];
     const int R = a.rptr[col.block + 1] - r0;
-    const int j = a0 + col.c;
+    const int j = a.src[a0 + col.c];
     for (int64_t p = a.colptr[j] + threadIdx.x; p < a.colptr[j + 1]; p += 64) {
-        const int i = a.rowidx[p];
+        const int i = a.rank[a.rowidx[p]];
         const int q = i < a0 + m ? i - a0 : m + find_row(a.rlist + r0, R, i);
         col.dst[q] = a.val[p];
     }
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(kThreads) void diagonal_inverses(const InverseJob *
     }
 }
 
-// C := alpha A B on 64 x 64 tiles (column-major), one workgroup per tile:
+// C := alpha op(A) B on 64 x 64 tiles (column-major), one workgroup per tile:
 // 4 wavefronts of 2 x 2 MFMA 16x16x4 tiles, K in steps of 16 through LDS,
 // the next step's entries loaded while the current one is multiplied.
 __global__ __launch_bounds__(kThreads) void gemm_tiles(const InverseJob *jobs, const InverseTile *tiles) {
@@ -177,28 +178,37 @@ __global__ __launch_bounds__(kThreads) void gemm_tiles(const InverseJob *jobs, c
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int kb = 0, ke = job.K;
     if (job.flags & kBLower) kb = j0;
+    if (job.flags & kGram) kb = max(i0, j0);
     if (job.flags & kALower) ke = min(ke, i0 + kTile);
+    const bool ta = (job.flags & kGram) != 0;
     double ra[4], rb[4];
     auto load = [&](int k0) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int ak = k0 + wave + 4 * q;
-            ra[q] = i0 + lane < job.M && ak < ke ? job.A[i0 + lane + (int64_t)ak * job.lda] : 0.0;
+            const int ai = ta ? tid / 16 + 16 * q : lane, ak = k0 + (ta ? tid % 16 : wave + 4 * q);
+            const bool aok = i0 + ai < job.M && ak < ke;
+            ra[q] = aok ? job.A[ta ? ak + (int64_t)(i0 + ai) * job.lda : i0 + ai + (int64_t)ak * job.lda] : 0.0;
             const int bj = tid / 16 + 16 * q, bk = k0 + tid % 16;
             rb[q] = j0 + bj < job.N && bk < ke ? job.B[bk + (int64_t)(j0 + bj) * job.ldb] : 0.0;
         }
     };
-    f64x4 acc[2][2] = {};
+    // Sums of kKStep products, then a sum of those: long dot products (the
+    // Gram product's above all) round twice as badly in one running sum, and
+    // the FP64 solve's error doubled with them (64^2 grid, k = 3: 6.8e-16
+    // against 5.1e-16, and 4.5e-16 for the block passes).
+    f64x4 total[2][2] = {};
     const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
     if (kb < ke) load(kb);
     for (int k0 = kb; k0 < ke; k0 += kKStep) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            As[wave + 4 * q][lane] = ra[q];
+            if (ta) As[tid % 16][tid / 16 + 16 * q] = ra[q];
+            else As[wave + 4 * q][lane] = ra[q];
             Bs[tid % 16][tid / 16 + 16 * q] = rb[q];
         }
         __syncthreads();
         if (k0 + kKStep < ke) load(k0 + kKStep);
+        f64x4 acc[2][2] = {};
 #pragma unroll
         for (int kk = 0; kk < kKStep; kk += 4) {
             const int k = kk + (lane >> 4);
@@ -209,6 +219,10 @@ __global__ __launch_bounds__(kThreads) void gemm_tiles(const InverseJob *jobs, c
             acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
             acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
         }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) total[x][y] += acc[x][y];
         __syncthreads();
     }
     // Accumulator element v of lane l: row l / 16 + 4 v, column l % 16.
@@ -219,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tiles(const InverseJob *jobs, c
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int i = i0 + wi + 16 * x + (lane >> 4) + 4 * v, j = j0 + wj + 16 * y + (lane & 15);
-                if (i < job.M && j < job.N) job.C[i + (int64_t)j * job.ldc] = job.alpha * acc[x][y][v];
+                if (i < job.M && j < job.N) job.C[i + (int64_t)j * job.ldc] = job.alpha * total[x][y][v];
             }
 }
 
@@ -245,6 +259,27 @@ __global__ __launch_bounds__(kThreads) void pack_tiles(const InversePack *packs,
     for (int q = ly; q < 32; q += kThreads / 32) {
         const int r = tile.i0 + q, c = tile.j0 + lx;
         if (r < rows && c < m && r >= c) mbwd[pk.off + bwd_at(m, r, c)] = (F)t[lx][q];
+    }
+}
+
+// The inverse of a top block in the panel layout of dense_top.hip, from the
+// lower half of the column-major m x m Gram product. order not null: in the
+// caller's row order (caller row i is plan row order[i]).
+template <typename F>
+__global__ __launch_bounds__(kThreads) void pack_top(const double *S, int m, const int *order, F *dst) {
+    constexpr int V = 16 / (int)sizeof(F), G = 4 * V;
+    const int mp = (m + 15) / 16 * 16;
+    const int64_t total = (int64_t)mp * mp;
+    for (int64_t e = blockIdx.x * (int64_t)kThreads + threadIdx.x; e < total; e += (int64_t)gridDim.x * kThreads) {
+        const int panel = (int)(e / (16 * (int64_t)mp)), w = (int)(e % (16 * (int64_t)mp));
+        const int lane = w % (64 * V) / V;
+        const int c = panel * 16 + lane % 16, r = w / (64 * V) * G + w % V * 4 + lane / 16;
+        F v = F(0);
+        if (c < m && r < m) {
+            const int i = order ? order[c] : c, j = order ? order[r] : r;
+            v = (F)S[max(i, j) + (int64_t)min(i, j) * m];
+        }
+        dst[e] = v;
     }
 }
 
@@ -286,7 +321,7 @@ struct Arena {
 
 // The blocks `large` of P through dense work arrays.
 template <typename F>
-hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::vector<int> &large, F *mfwd, F *mbwd) {
+hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::vector<int> &large, const int *order, F *mfwd, F *mbwd, F *mtop) {
     Arena arena;
     // Work arrays: D = [L_BB ; L_RB] (rows x m), X and T (m x m), Q (R x m).
     size_t dn = 0, xn = 0, qn = 0;
@@ -312,21 +347,23 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
     struct Place {
         double *D, *X, *T, *Q;
         int m, R;
+        bool top;
     };
     std::vector<Place> at;
     {
         double *d = D, *x = X, *t = T, *q = Q;
         for (int b : large) {
             const int m = P.start[b + 1] - P.start[b], R = P.rptr[b + 1] - P.rptr[b], rows = m + R;
-            at.push_back({d, x, t, q, m, R});
+            at.push_back({d, x, t, q, m, R, P.is_top(b)});
             for (int c = 0; c < m; ++c) cols.push_back({b, c, d + (size_t)c * rows});
             for (int i = 0; i < m; i += kSmall) {
                 const int w = std::min(kSmall, m - i);
                 diag.push_back({d + i + (size_t)i * rows, nullptr, x + i + (size_t)i * m, rows, 0, m, w, w, w, 0, 1.0});
             }
             packs.push_back({x, q, P.moff[b], m, R});
-            for (int i = 0; i < rows; i += 32)
-                for (int j = 0; j < m && j <= i; j += 32) ptiles.push_back({(int)packs.size() - 1, i, j});
+            if (!P.is_top(b))
+                for (int i = 0; i < rows; i += 32)
+                    for (int j = 0; j < m && j <= i; j += 32) ptiles.push_back({(int)packs.size() - 1, i, j});
             max_m = std::max(max_m, m);
             d += (size_t)rows * m;
             x += (size_t)m * m;
@@ -337,7 +374,8 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
     auto add = [&](const InverseJob &j) {
         jobs.push_back(j);
         for (int i = 0; i < j.M; i += kTile)
-            for (int c = 0; c < j.N; c += kTile) tiles.push_back({(int)jobs.size() - 1, i, c});
+            for (int c = 0; c < j.N; c += kTile)
+                if (!(j.flags & kGram) || i >= c) tiles.push_back({(int)jobs.size() - 1, i, c});
     };
     for (int s = kSmall; s < max_m; s *= 2) {
         for (int half = 0; half < 2; ++half) {
@@ -354,9 +392,11 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
             stage.push_back(tiles.size());
         }
     }
-    for (const Place &p : at)
+    for (const Place &p : at) {
         if (p.R > 0)
             add({p.D + p.m, p.X, p.Q, p.m + p.R, p.m, p.R, p.R, p.m, p.m, kBLower, -1.0});
+        if (p.top) add({p.X, p.X, p.T, p.m, p.m, p.m, p.m, p.m, p.m, kGram, 1.0});
+    }
     stage.push_back(tiles.size());
     InverseColumn *dcols = nullptr;
     InverseJob *ddiag = nullptr, *djobs = nullptr;
@@ -382,15 +422,23 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
         pack_tiles<F><<<dim3((unsigned)ptiles.size()), kThreads>>>(dpacks, dptiles, mfwd, mbwd);
         INV_TRY(hipGetLastError());
     }
+    for (size_t i = 0; i < at.size(); ++i)
+        if (at[i].top) {
+            const unsigned grid = (unsigned)std::min<int64_t>((top_entries(at[i].m) + kThreads - 1) / kThreads, 1 << 16);
+            pack_top<F><<<grid, kThreads>>>(at[i].T, at[i].m, P.is_whole(large[i]) ? order + P.start[large[i]] : nullptr,
+                                           mtop + P.top_off[large[i]]);
+            INV_TRY(hipGetLastError());
+        }
     return hipDeviceSynchronize();   // the work arrays are freed on return
 }
 
 
 template <typename F>
-hipError_t fill(const BlockPlan &P, const InverseArgs &args, F *mfwd, F *mbwd) {
+hipError_t fill(const BlockPlan &P, const InverseArgs &args, const int *order, F *mfwd, F *mbwd, F *mtop) {
     std::vector<int> small, large;
     for (int b = 0; b < P.nblocks; ++b) {
-        (P.start[b + 1] - P.start[b] <= kSmall ? small : large).push_back(b);
+        const bool top = P.is_top(b);
+        (!top && P.start[b + 1] - P.start[b] <= kSmall ? small : large).push_back(b);
     }
     Arena arena;
     if (!small.empty()) {
@@ -410,7 +458,7 @@ hipError_t fill(const BlockPlan &P, const InverseArgs &args, F *mfwd, F *mbwd) {
             if (hi > lo && words > kGroup) break;
             group.push_back(large[hi]);
         }
-        INV_TRY(fill_large<F>(P, args, group, mfwd, mbwd));
+        INV_TRY(fill_large<F>(P, args, group, order, mfwd, mbwd, mtop));
         lo = hi;
     }
     return hipDeviceSynchronize();
@@ -418,10 +466,14 @@ hipError_t fill(const BlockPlan &P, const InverseArgs &args, F *mfwd, F *mbwd) {
 
 }  // namespace
 
-hipError_t fill_block_plan_on_device(const BlockPlan &P, const InverseArgs &args, int float_bytes, void *mfwd, void *mbwd) {
+hipError_t fill_block_plan_on_device(const BlockPlan &P, const InverseArgs &args, const int *order, int float_bytes,
+                                     void *mfwd, void *mbwd, void *mtop) {
     if (P.n == 0) return hipSuccess;
-    return float_bytes == 4 ? fill<float>(P, args, static_cast<float *>(mfwd), static_cast<float *>(mbwd))
-                            : fill<double>(P, args, static_cast<double *>(mfwd), static_cast<double *>(mbwd));
+    if (float_bytes == 4)
+        return fill<float>(P, args, order, static_cast<float *>(mfwd), static_cast<float *>(mbwd),
+                           static_cast<float *>(mtop));
+    return fill<double>(P, args, order, static_cast<double *>(mfwd), static_cast<double *>(mbwd),
+                        static_cast<double *>(mtop));
 }
 
 hipError_t launch_cast_factor(int float_bytes, int64_t nnz, const double *val, const int *csr_src, void *lvals,

@@ -97,7 +97,7 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
         for (size_t q = lo; q < hi; ++q) {
             const int b = order[q];
             const int64_t m = start[b + 1] - start[b], R = P.rptr[b + 1] - P.rptr[b];
-            if (m >= sg) entries += m * (m + 1) / 2 + R * m;
+            if (m >= sg && !P.is_top(b)) entries += m * (m + 1) / 2 + R * m;
         }
         const int64_t want = entries / opt.level_tasks;
         level_split = (int)std::max<int64_t>(opt.min_split_entries, std::min<int64_t>(opt.split_entries, want));
@@ -137,12 +137,17 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
         set_level_split(order, lo, hi, sg_l);
         for (size_t q = lo; q < hi; ++q) {
             const int b = order[q], m = start[b + 1] - start[b];
+            if (P.is_top(b)) {
+                for (int r0 = 0; r0 < m; r0 += rows_l) push(L.fwd, b, r0, std::min(m, r0 + rows_l), 4);
+                continue;
+            }
             if (m < sg_l) continue;
             for (int r0 = 0; r0 < m; r0 += rows_l) push(L.fwd, b, r0, std::min(m, r0 + rows_l), 1);
         }
         for (size_t q = lo; q < hi; ++q) {
             const int b = order[q], m = start[b + 1] - start[b];
             const int rows = m + (P.rptr[b + 1] - P.rptr[b]);
+            if (P.is_top(b)) continue;
             if (m < sg_l) {
                 for (int r0 = 0; r0 < rows; r0 += rows_l)
                     push(L.fwd, b, r0, std::min(rows, r0 + rows_l), 0);
@@ -199,6 +204,7 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
         for (size_t q = lo; q < hi; ++q) {
             const int b = order[q], m = start[b + 1] - start[b];
             const int rows = m + (P.rptr[b + 1] - P.rptr[b]);
+            if (P.is_top(b)) continue;
             const bool big = m >= sg_l;
             const int wmax = big ? bcols_big_l : opt.bwd_cols;
             for (int c0 = 0; c0 < m; c0 += wmax) {
@@ -228,7 +234,7 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
     //    the same order.
     auto is_leaf = [&](int b) {
         const int m = start[b + 1] - start[b], R = P.rptr[b + 1] - P.rptr[b];
-        return opt.leaf_partition && P.level_fwd[b] == 0 && m <= kLeafMaxM && m + R <= kLeafMaxRows &&
+        return opt.leaf_partition && !P.is_top(b) && P.level_fwd[b] == 0 && m <= kLeafMaxM && m + R <= kLeafMaxRows &&
                m < opt.split_gather && opt.fwd_rows <= 64 && opt.bwd_cols <= 32;
     };
     auto partition = [&](std::vector<int> &tasks, bool leaf_first, int &count) {
@@ -250,35 +256,44 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
 
 }  // namespace
 
-BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx, const BlockPlanOptions &opt) {
-    BlockPlan P;
-    P.n = n;
-    P.nnz_l = colptr[n];
-    std::vector<int> parent(n, -1), size(n, 1);
+namespace {
+
+// parent(j) = first row below the diagonal; size[j] = nodes of j's subtree.
+void elimination_tree(int n, const int *colptr, const int *rowidx, std::vector<int> &parent, std::vector<int> &size) {
+    parent.assign((size_t)n, -1);
+    size.assign((size_t)n, 1);
     for (int j = 0; j < n; ++j)
         if (colptr[j + 1] - colptr[j] > 1) parent[j] = rowidx[colptr[j] + 1];
     for (int j = 0; j < n; ++j)
         if (parent[j] >= 0) size[parent[j]] += size[j];
+}
 
-    // 1. Partition into contiguous blocks: small whole subtrees, then chains
-    //    (j and j + 1 share a block when parent(j) = j + 1), capped at max_block.
-    int max_block = opt.max_block;
-    if (max_block <= 0) {
-        int longest = n > 0 ? 1 : 0;
-        for (int j = 0, run = 1; j + 1 < n; ++j) {
-            run = parent[j] == j + 1 ? run + 1 : 1;
-            longest = std::max(longest, run);
-        }
-        max_block = 1024;
-        while (max_block < 4096 && 2 * max_block <= longest) max_block *= 2;
+// The largest power of two <= the longest chain (parent(j) = j + 1), within [1024, 4096].
+int automatic_max_block(int n, const std::vector<int> &parent) {
+    int longest = n > 0 ? 1 : 0;
+    for (int j = 0, run = 1; j + 1 < n; ++j) {
+        run = parent[j] == j + 1 ? run + 1 : 1;
+        longest = std::max(longest, run);
     }
-    std::vector<int> &start = P.start;
+    int max_block = 1024;
+    while (max_block < 4096 && 2 * max_block <= longest) max_block *= 2;
+    return max_block;
+}
+
+// Block starts (then n): small whole subtrees, then chains (j and j + 1 share
+// a block when parent(j) = j + 1), capped at max_block; the last top_rows
+// rows are one block.
+std::vector<int> partition_rows(int n, const std::vector<int> &parent, const std::vector<int> &size,
+                                const BlockPlanOptions &opt) {
+    const int end = n - std::min(n, opt.top_rows);
+    const int max_block = opt.max_block > 0 ? opt.max_block : automatic_max_block(n, parent);
+    std::vector<int> start;
     int j = 0;
-    while (j < n) {
+    while (j < end) {
         // Is j the first node of a small subtree whose root r has size <= leaf_max
         // and whose parent is not small? Subtree of r spans [r - size[r] + 1, r].
         int r = j;
-        while (parent[r] >= 0 && size[parent[r]] <= opt.leaf_max &&
+        while (parent[r] >= 0 && parent[r] < end && size[parent[r]] <= opt.leaf_max &&
                parent[r] - size[parent[r]] + 1 == j)
             r = parent[r];
         if (size[r] <= opt.leaf_max && r - size[r] + 1 == j && size[r] > 1) {
@@ -288,12 +303,35 @@ BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx
         }
         start.push_back(j);
         int e = j;
-        while (e + 1 < n && parent[e] == e + 1 && e + 1 - j + 1 <= max_block) ++e;
+        while (e + 1 < end && parent[e] == e + 1 && e + 1 - j + 1 <= max_block) ++e;
         j = e + 1;
     }
-    const int nb = (int)start.size();
+    if (end < n) start.push_back(end);
     start.push_back(n);
+    return start;
+}
+
+}  // namespace
+
+BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx, const BlockPlanOptions &opt) {
+    BlockPlan P;
+    P.n = n;
+    P.nnz_l = colptr[n];
+    std::vector<int> parent, size;
+    elimination_tree(n, colptr, rowidx, parent, size);
+
+    // 1. Partition into contiguous blocks.
+    std::vector<int> &start = P.start;
+    start = partition_rows(n, parent, size, opt);
+    const int nb = (int)start.size() - 1;
     P.nblocks = nb;
+    if (opt.top_rows > 0 && n > 0) {
+        P.top_off.assign((size_t)nb, -1);
+        P.top_off[(size_t)nb - 1] = 0;
+        P.top_size = top_entries(opt.top_rows);
+        P.top_whole.assign((size_t)nb, 0);
+        P.top_whole[(size_t)nb - 1] = nb == 1;
+    }
     std::vector<int> block_of(n);
     for (int b = 0; b < nb; ++b)
         for (int i = start[b]; i < start[b + 1]; ++i) block_of[i] = b;
@@ -318,6 +356,10 @@ BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx
         P.rlist.insert(P.rlist.end(), rows_b.begin(), rows_b.end());
         P.rptr[b + 1] = (int)P.rlist.size();
         const int64_t m = e - a, R = (int64_t)rows_b.size();
+        if (P.is_top(b)) {
+            P.moff[b + 1] = P.moff[b];
+            continue;
+        }
         // The panel kernels index one block's M_B with 32-bit offsets, and
         // their column-major offset c * (m + R) reaches m * (m + R).
         if (m * (m + R) >= (int64_t(1) << 31))
@@ -390,6 +432,7 @@ void fill_block_plan_values(BlockPlan &P, const int *colptr, const int *rowidx, 
         std::vector<double> Lbb, Pb, Linv, Q;
     };
     auto compute = [&](int b, int inner, Work &w) {
+        if (P.is_top(b)) return;
         const int a = P.start[b], e = P.start[b + 1];
         const int m = e - a;
         const int R = P.rptr[b + 1] - P.rptr[b];
@@ -468,6 +511,71 @@ BlockPlan build_block_plan(int n, const int *colptr, const int *rowidx, const do
     BlockPlan P = build_block_plan_structure(n, colptr, rowidx, opt);
     fill_block_plan_values(P, colptr, rowidx, val, opt.threads);
     return P;
+}
+
+DenseTop choose_dense_top(int n, const int *colptr, const int *rowidx, const BlockPlanOptions &opt, int float_bytes) {
+    DenseTop top;
+    if (n == 0) return top;
+    std::vector<int> parent, size;
+    elimination_tree(n, colptr, rowidx, parent, size);
+    BlockPlanOptions plain = opt;
+    plain.top_rows = 0;
+    const std::vector<int> start = partition_rows(n, parent, size, plain);
+    const int nb = (int)start.size() - 1;
+    std::vector<int> block_of((size_t)n), level((size_t)nb, 0);
+    for (int b = 0; b < nb; ++b)
+        for (int i = start[b]; i < start[b + 1]; ++i) block_of[i] = b;
+    // A block's R rows lie on the path from its last column to the root, so
+    // its forward level is one more than its highest child's.
+    int levels = 0;
+    for (int b = 0; b < nb; ++b) {
+        const int p = parent[start[b + 1] - 1];
+        if (p >= 0) level[block_of[p]] = std::max(level[block_of[p]], level[b] + 1);
+        levels = std::max(levels, level[b] + 1);
+    }
+    // Per level: the rows of the blocks from it up, and the entries of its M_B.
+    std::vector<int64_t> rows((size_t)levels + 1, 0), entries((size_t)levels, 0);
+    for (int b = 0; b < nb; ++b) {
+        const int64_t m = start[b + 1] - start[b], below = colptr[start[b + 1]] - colptr[start[b + 1] - 1] - 1;
+        rows[level[b]] += m;
+        entries[level[b]] += m * (m + 1) / 2 + m * below;   // (|R| >= the last column's rows below)
+    }
+    for (int l = levels - 1; l >= 0; --l) rows[l] += rows[l + 1];
+    double passes = opt.pass_us;
+    for (int l = 0; l < levels; ++l) passes += 2.0 * (opt.level_us + (double)entries[l] * float_bytes / opt.level_gbs * 1e-3);
+    int cut = levels;
+    double best = passes;
+    for (int l = levels - 1; l >= 0 && rows[l] <= opt.top_max_rows; --l) {
+        passes -= 2.0 * (opt.level_us + (double)entries[l] * float_bytes / opt.level_gbs * 1e-3);
+        const double us = (l > 0 ? passes : 0.0) + opt.top_us + (double)top_entries(rows[l]) * float_bytes / opt.top_gbs * 1e-3;
+        if (us < best) {
+            best = us;
+            cut = l;
+        }
+    }
+    if (cut == levels) return top;
+    top.max_block = opt.max_block > 0 ? opt.max_block : automatic_max_block(n, parent);
+    top.rows = (int)rows[cut];
+    for (int pass = 0; pass < 2; ++pass)
+        for (int b = 0; b < nb; ++b)
+            if ((level[b] >= cut) == (pass == 1))
+                for (int i = start[b]; i < start[b + 1]; ++i) top.src.push_back(i);
+    return top;
+}
+
+void renumber_pattern(int n, const int *colptr, const int *rowidx, const std::vector<int> &src,
+                      std::vector<int> &new_colptr, std::vector<int> &new_rowidx) {
+    std::vector<int> rank((size_t)n);
+    for (int r = 0; r < n; ++r) rank[src[r]] = r;
+    new_colptr.assign((size_t)n + 1, 0);
+    new_rowidx.resize((size_t)colptr[n]);
+    for (int r = 0; r < n; ++r) {
+        const int j = src[r];
+        int q = new_colptr[r];
+        for (int p = colptr[j]; p < colptr[j + 1]; ++p) new_rowidx[q++] = rank[rowidx[p]];
+        std::sort(new_rowidx.begin() + new_colptr[r], new_rowidx.begin() + q);
+        new_colptr[r + 1] = q;
+    }
 }
 
 }  // namespace cholespy_amd

@@ -14,6 +14,7 @@
 // workgroups are between blocks, whose tree is far shallower than the
 // elimination tree.
 #pragma once
+#include <cstddef>
 #include <cstdint>
 #include <vector>
 
@@ -87,6 +88,23 @@ struct BlockPlanOptions {
     // Blocks of one level are independent, so either order is a valid
     // schedule.
     bool critical_order = true;
+    // Rows of the dense top block: the last top_rows rows of the factor (an
+    // ancestor-closed set: see choose_dense_top) form one block that is
+    // solved by the explicit inverse of its Schur complement between the two
+    // passes. 0 = none. The host fill does not form its values.
+    int top_rows = 0;
+    // What choose_dense_top weighs, in microseconds and GB/s: the two passes'
+    // launches and leaf tasks, a level of a pass (its hand-offs, and its M_B
+    // at the rate the block tasks reach), and the dense product.
+    // Fitted to where the measured best cut lies: icosphere(7), k = 3, FP32 has
+    // 157.9 us with 2.9k rows, 166.8 with 5.1k, 168.0 with 978; icosphere(6)
+    // k = 3 85 us a solve with 3.5k rows, 100 with 5.4k, and k = 128 251 and
+    // 283 us; a 48^3 grid, k = 32, FP32 450 us with 6.2k rows, 510 with 3.2k;
+    // a 33^3 grid, k = 5, FP64 174 us with 3.7k, 186 with 1.5k. More rows
+    // than top_max_rows would cost a refactorisation more (n^3) than they
+    // give a solve.
+    double pass_us = 25.0, level_us = 3.5, level_gbs = 3000.0, top_us = 5.0, top_gbs = 5500.0;
+    int64_t top_max_rows = 6400;
     // Host threads for the dense block inverses (0 = hardware count, at most
     // 16). Batches already build one plan per thread and pass 1.
     int threads = 0;
@@ -116,6 +134,7 @@ struct BlockPlan {
     //   (block, first, last, kind, lo, hi, sbase, split).
     // Forward kinds: 0 = gather r_B and multiply rows [first, last) of M_B;
     // 1 = gather rows [first, last) of r_B only (published for kinds 2, 3);
+    // 4 = the same for a dense top block, into y (read after the pass);
     // 2 = multiply rows [first, last) of M_B by the published r_B;
     // 3 = split s of nsplit (split = split_code(s, nsplit)): as 2 over
     //     columns [lo, hi) only, result published to the split rows
@@ -133,6 +152,18 @@ struct BlockPlan {
     // The same two passes as tasks for wide right-hand sides (same records,
     // BlockPlanOptions' wide_* shape, no leaf partition).
     std::vector<int> fwd_task_wide, bwd_task_wide;
+    // Dense top blocks (none, or one per system): top_off[b] = offset of the
+    // block's inverse (top_entries(m) elements) in an array of its own, -1 for
+    // other blocks (empty: no top block). They have no entries in mfwd /
+    // mbwd, no R rows and no backward tasks; their forward tasks are gathers
+    // (kind 4) that leave r_B in y for the dense product.
+    std::vector<int64_t> top_off;
+    int64_t top_size = 0;                  // elements of all top inverses
+    // Top blocks that are a whole system: their inverse is stored in the
+    // caller's row order, so their plan rows stand for caller rows in order.
+    std::vector<char> top_whole;
+    bool is_whole(int b) const { return !top_whole.empty() && top_whole[(std::size_t)b] != 0; }
+    bool is_top(int b) const { return !top_off.empty() && top_off[(std::size_t)b] >= 0; }
     int nsplit_rows = 0;                   // rows of the split-result array (either list)
     int max_m = 0, max_rows = 0;           // largest m and m + |R|
     int64_t nnz_l = 0;
@@ -150,5 +181,27 @@ BlockPlan build_block_plan(int n, const int *colptr, const int *rowidx, const do
 // refactorisation keeps the structure and refills the values.
 BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx, const BlockPlanOptions &opt);
 void fill_block_plan_values(BlockPlan &P, const int *colptr, const int *rowidx, const double *val, int threads);
+
+// Elements of the stored inverse of an m-row top block: panels of 16 columns,
+// rows padded to a multiple of 16 (layout in dense_top.hip).
+constexpr int64_t top_entries(int64_t m) { return ((m + 15) / 16 * 16) * ((m + 15) / 16 * 16); }
+
+// The rows that are worth solving as one dense block, and a numbering that
+// puts them last. src[r] = factor row at plan row r (the other rows keep
+// their order, then the top rows in order: a topological order of the
+// elimination tree, so L keeps its pattern under it); empty src: no top
+// block. Blocks at forward level >= cut (in the partition that `opt` gives)
+// are the top rows; the cut minimises the estimated time of the levels below
+// it and of the dense product.
+struct DenseTop {
+    int rows = 0;
+    int max_block = 0;   // chain cap of the whole factor's partition
+    std::vector<int> src;
+};
+DenseTop choose_dense_top(int n, const int *colptr, const int *rowidx, const BlockPlanOptions &opt, int float_bytes);
+
+// The pattern of L in the numbering src (columns and rows renumbered, rows ascending).
+void renumber_pattern(int n, const int *colptr, const int *rowidx, const std::vector<int> &src,
+                      std::vector<int> &new_colptr, std::vector<int> &new_rowidx);
 
 }  // namespace cholespy_amd

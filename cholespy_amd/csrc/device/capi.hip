@@ -108,8 +108,20 @@ struct DeviceBlockPlan {
     int *cptr = nullptr, *cslot = nullptr, *gslot = nullptr;
     int *ftask = nullptr, *btask = nullptr;
     int *ftask_wide = nullptr, *btask_wide = nullptr;
+    // Dense top blocks (block_plan.hpp): their inverses and the tile lists of
+    // the dense product. whole: a single system that is one top block.
+    void *mtop = nullptr;
+    DenseTopTile *top_tiles = nullptr, *top_tiles_wide = nullptr;
+    int n_top_tiles = 0, n_top_tiles_wide = 0;
+    bool whole = false;
+    int top_rows = 0;      // of a single system
+    int *perm = nullptr;   // caller row of each plan row
 
     void release() {
+        dev_free(mtop);
+        dev_free(top_tiles);
+        dev_free(top_tiles_wide);
+        dev_free(perm);
         dev_free(start);
         dev_free(rptr);
         dev_free(rlist);
@@ -131,7 +143,8 @@ struct DeviceBlockPlan {
 struct cholespy_gpu_solver;
 namespace {
 BlockPlanOptions plan_options(const BlockPlanOptions &base = BlockPlanOptions());
-int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<int> *blk_sys = nullptr);
+int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<int> &perm,
+                const std::vector<int> *blk_sys = nullptr);
 }  // namespace
 
 struct cholespy_gpu_solver {
@@ -226,9 +239,10 @@ struct cholespy_gpu_solver {
     // Pattern of the uploaded factor, kept for cholespy_solver_refactor:
     // column form of L, for each position of the row form the column-form
     // position it copies (device), and the block plan's structure.
-    std::vector<int> host_colptr, host_rowidx;
+    std::vector<int> host_perm, host_colptr, host_rowidx;
     int *csr_src = nullptr;
     BlockPlan host_plan;
+    std::vector<int> plan_src;   // factor row of each plan row
 };
 
 namespace {
@@ -285,9 +299,10 @@ std::vector<int> device_tasks(const BlockPlan &P, const std::vector<int> &tasks,
 }
 
 // Copies the structure of a (possibly merged) block plan to the device and
-// allocates its values, which fill_plan_values forms there; blk_sys maps
-// blocks to systems for a batch.
-int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<int> *blk_sys) {
+// allocates its values, which fill_plan_values forms there. perm: caller row
+// of each plan row; blk_sys maps blocks to systems for a batch.
+int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<int> &perm,
+                const std::vector<int> *blk_sys) {
     DeviceBlockPlan &d = s->plan;
     d.release();
     d.nblocks = P.nblocks;
@@ -304,7 +319,12 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
     d.levels_fwd = d.levels_bwd = 0;
     for (int v : P.level_fwd) d.levels_fwd = std::max(d.levels_fwd, v + 1);
     for (int v : P.level_bwd) d.levels_bwd = std::max(d.levels_bwd, v + 1);
-    d.m_entries = P.moff[P.nblocks];
+    d.m_entries = P.moff[P.nblocks];   // (a top block's square serves both passes: half of it each)
+    for (int b = 0; b < P.nblocks; ++b)
+        if (P.is_top(b)) {
+            const int64_t m = P.start[b + 1] - P.start[b];
+            d.m_entries += (m * m + 1) / 2;
+        }
     s->plan_copy[0] = P.start;
     s->plan_copy[1] = P.rptr;
     s->plan_copy[2] = P.level_fwd;
@@ -329,9 +349,27 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
         HIP_TRY(upload(&d.ftask_wide, fw.data(), fw.size()));
         HIP_TRY(upload(&d.btask_wide, bw.data(), bw.size()));
     }
-    const size_t me = (size_t)d.m_entries, fb = (size_t)s->fbytes;
+    HIP_TRY(upload(&d.perm, perm.data(), perm.size()));
+    const size_t me = (size_t)P.moff[P.nblocks], fb = (size_t)s->fbytes;
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mfwd), me * fb));
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mbwd), me * fb));
+    HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mtop), (size_t)P.top_size * fb));
+    std::vector<DenseTopTile> tiles, wide;
+    for (int b = 0; b < P.nblocks; ++b) {
+        if (!P.is_top(b)) continue;
+        const int m = P.start[b + 1] - P.start[b], panels = (m + 15) / 16, sys = blk_sys ? (*blk_sys)[b] : 0;
+        for (int p = 0; p < panels; ++p) {
+            const DenseTopTile t{P.start[b], m, p, sys, P.top_off[b]};
+            tiles.push_back(t);
+            if (p % 2 == 0) wide.push_back(t);
+        }
+    }
+    d.n_top_tiles = (int)tiles.size();
+    d.n_top_tiles_wide = (int)wide.size();
+    d.top_rows = !blk_sys && !P.top_off.empty() ? P.n - P.start[P.nblocks - 1] : 0;
+    d.whole = !blk_sys && P.nblocks == 1 && P.is_whole(0);
+    HIP_TRY(upload(&d.top_tiles, tiles.data(), tiles.size()));
+    HIP_TRY(upload(&d.top_tiles_wide, wide.data(), wide.size()));
     for (auto &row : s->grid_blocks)
         for (int &g : row) g = 0;
     s->buffers_path = -1;
@@ -354,14 +392,28 @@ struct DeviceTemp {
 };
 
 // Forms the plan's dense values on the device (block_inverse.hip) from L in
-// compressed columns (colptr: host, rowidx and val: device).
+// compressed columns (colptr: host, rowidx and val: device), whose row
+// src[r] is plan row r (for a whole top block: its factor row, the plan rows
+// standing for caller rows). perm: caller row of each factor row.
 int fill_plan_values(cholespy_gpu_solver *s, const BlockPlan &P, const int64_t *colptr, const int *rowidx,
-                     const double *val) {
+                     const double *val, const std::vector<int> &src, const std::vector<int> &perm) {
     DeviceBlockPlan &d = s->plan;
-    DeviceTemp tcol;
-    HIP_TRY(tcol.put(colptr, (size_t)P.n + 1));
-    const InverseArgs args{tcol.as<int64_t>(), rowidx, val, d.start, d.rptr, d.rlist, d.moff};
-    HIP_TRY(fill_block_plan_on_device(P, args, s->fbytes, d.mfwd, d.mbwd));
+    const size_t n = (size_t)P.n;
+    std::vector<int> rank(n), order;
+    for (size_t r = 0; r < n; ++r) rank[(size_t)src[r]] = (int)r;
+    DeviceTemp tcol, tsrc, trank, torder;
+    HIP_TRY(tcol.put(colptr, n + 1));
+    HIP_TRY(tsrc.put(src.data(), n));
+    HIP_TRY(trank.put(rank.data(), n));
+    for (int b = 0; b < P.nblocks; ++b) {
+        if (!P.is_whole(b)) continue;
+        order.resize(n);
+        for (int r = P.start[b]; r < P.start[b + 1]; ++r) order[(size_t)perm[(size_t)src[(size_t)r]]] = r - P.start[b];
+    }
+    if (!order.empty()) HIP_TRY(torder.put(order.data(), n));
+    const InverseArgs args{tcol.as<int64_t>(), rowidx, val,    tsrc.as<int>(), trank.as<int>(),
+                           d.start,            d.rptr, d.rlist, d.moff};
+    HIP_TRY(fill_block_plan_on_device(P, args, torder.as<int>(), s->fbytes, d.mfwd, d.mbwd, d.mtop));
     return CHOLESPY_OK;
 }
 
@@ -372,21 +424,60 @@ int upload_values(cholespy_gpu_solver *s, const double *val) {
     HIP_TRY(tval.put(val, (size_t)s->nnz));
     HIP_TRY(launch_cast_factor(s->fbytes, s->nnz, tval.as<double>(), s->csr_src, s->lvals, s->uvals));
     const std::vector<int64_t> colptr(s->host_colptr.begin(), s->host_colptr.end());
-    return fill_plan_values(s, s->host_plan, colptr.data(), s->ucols, tval.as<double>());
+    return fill_plan_values(s, s->host_plan, colptr.data(), s->ucols, tval.as<double>(), s->plan_src,
+                            s->host_perm);
+}
+
+// Whether plans may have a dense top (CHOLESPY_DENSE_TOP: its most rows, 0 =
+// none). Knobs that shape the large blocks' tasks ask for those tasks: with
+// one of them set the plan keeps its levels.
+int64_t dense_top_rows(const BlockPlanOptions &opt) {
+    if (const char *e = std::getenv("CHOLESPY_DENSE_TOP")) return std::max(0, std::atoi(e));
+    for (const char *knob : {"CHOLESPY_MAX_BLOCK", "CHOLESPY_SPLIT_ENTRIES", "CHOLESPY_MAX_SPLIT", "CHOLESPY_SPLIT_GATHER",
+                             "CHOLESPY_FWD_ROWS_BIG", "CHOLESPY_BWD_COLS_BIG", "CHOLESPY_LEVEL_TASKS",
+                             "CHOLESPY_MIN_SPLIT_ENTRIES", "CHOLESPY_WIDE_FWD_ROWS_BIG", "CHOLESPY_WIDE_LEVEL_TASKS",
+                             "CHOLESPY_WIDE_FINE_BWD_COLS_BIG", "CHOLESPY_WIDE_MIN_SPLIT_ENTRIES",
+                             "CHOLESPY_WIDE_SPLIT_GATHER"})
+        if (std::getenv(knob)) return 0;
+    return opt.top_max_rows;
+}
+
+// The plan's structure for a factor's pattern and its row numbering (src).
+BlockPlan plan_structure(int n, const int *colptr, const int *rowidx, BlockPlanOptions opt, int float_bytes,
+                         std::vector<int> &src) {
+    opt.top_max_rows = dense_top_rows(opt);
+    DenseTop top;
+    if (opt.top_max_rows > 0) top = choose_dense_top(n, colptr, rowidx, opt, float_bytes);
+    opt.top_rows = top.rows;
+    if (top.rows == 0) {
+        src.resize((size_t)n);
+        for (int i = 0; i < n; ++i) src[(size_t)i] = i;
+        return build_block_plan_structure(n, colptr, rowidx, opt);
+    }
+    opt.max_block = top.max_block;   // (the shorter chains below the top keep their cuts)
+    src.swap(top.src);
+    std::vector<int> cp, ri;
+    renumber_pattern(n, colptr, rowidx, src, cp, ri);
+    return build_block_plan_structure(n, cp.data(), ri.data(), opt);
 }
 
 // Plans the uploaded pattern with base options `base` and uploads the
 // structure (the values follow).
 int plan_system(cholespy_gpu_solver *s, const BlockPlanOptions &base) {
     BlockPlan P;
+    std::vector<int> src;
     try {
-        P = build_block_plan_structure(s->n, s->host_colptr.data(), s->host_rowidx.data(), plan_options(base));
+        P = plan_structure(s->n, s->host_colptr.data(), s->host_rowidx.data(), plan_options(base), s->fbytes, src);
     } catch (const std::exception &ex) {
         return fail(CHOLESPY_ERR_INVALID_ARGUMENT, ex.what());
     }
-    const int rc = upload_plan(s, P);
+    const bool whole = P.nblocks == 1 && P.is_whole(0);
+    std::vector<int> perm((size_t)s->n);
+    for (int r = 0; r < s->n; ++r) perm[(size_t)r] = whole ? r : s->host_perm[(size_t)src[(size_t)r]];
+    const int rc = upload_plan(s, P, perm);
     if (rc != CHOLESPY_OK) return rc;
     s->host_plan = std::move(P);
+    s->plan_src.swap(src);
     s->plan_base = base;
     return CHOLESPY_OK;
 }
@@ -626,6 +717,7 @@ int cholespy_solver_upload_factor(cholespy_gpu_solver *s, const int *perm, const
     s->nnz = nnz;
     dev_free(s->csr_src);
     HIP_TRY(upload(&s->csr_src, csr_src.data(), csr_src.size()));
+    s->host_perm.assign(perm, perm + n);
     s->host_colptr.assign(colptr, colptr + n + 1);
     s->host_rowidx.assign(rowidx, rowidx + nnz);
     s->analysed[0] = s->analysed[1] = false;
@@ -868,6 +960,17 @@ int effective_tile(const cholespy_gpu_solver *s, int fbytes, int k) {
     return rule;
 }
 
+bool overlaps(const void *p, size_t pn, const void *q, size_t qn) {
+    const char *a = static_cast<const char *>(p), *b = static_cast<const char *>(q);
+    return a < b + qn && b < a + pn;
+}
+
+// Whether a block solve of the handle needs its work buffers at all.
+bool solves_directly(const cholespy_gpu_solver *s, const void *b, const void *x, int k, size_t x_elem) {
+    const size_t elems = (size_t)s->n * (size_t)k;
+    return s->path == CHOLESPY_PATH_BLOCKS && s->plan.whole && !overlaps(b, elems * (size_t)s->fbytes, x, elems * x_elem);
+}
+
 // Work buffers of one block solve (the handle's own, or the library's
 // scratch array for cholespy_solver_solve_noalloc).
 struct WorkSet {
@@ -892,7 +995,7 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
     bf.cptr = d.cptr;
     bf.cslot = d.cslot;
     bf.gslot = d.gslot;
-    bf.perm = s->perm;
+    bf.perm = d.perm;
     bf.b = b;
     bf.x = x;
     const WorkSet own{s->y, s->z, s->part, s->spart, s->rbuf};
@@ -911,9 +1014,36 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         bf.sys_pbase = s->sys_pbase;
         bf.sys_sbase = s->sys_sbase;
     }
+    DenseTopArgs top;
+    top.tiles = s->is_batch ? d.top_tiles : nullptr;
+    top.row0 = s->n - d.top_rows;
+    top.n = d.top_rows;
+    top.M = d.mtop;
+    top.in = w.y;
+    top.z = d.whole ? nullptr : w.z;
+    top.x = x;
+    top.perm = d.whole ? nullptr : d.perm;
+    top.k = k;
+    top.xmode = xmode;
+    top.sys_k = bf.sys_k;
+    top.sys_vbase = bf.sys_vbase;
+    if (d.whole) {
+        // One product. Its input is b itself, unless the passes run apart or
+        // x overlaps b: then a copy in y.
+        const size_t bytes = (size_t)s->n * (size_t)k * (size_t)fbytes;
+        if (only_pass == 0 || (only_pass < 0 && overlaps(b, bytes, x, xmode == 0 ? bytes : 8 * (bytes / fbytes))))
+            HIP_TRY(launch_copy(w.y, b, bytes, st));
+        else if (only_pass < 0)
+            top.in = b;
+        if (only_pass != 0)
+            HIP_TRY(launch_dense_top(fbytes, top, d.n_top_tiles, d.top_tiles_wide, d.n_top_tiles_wide, k, st));
+        return CHOLESPY_OK;
+    }
     for (int pass = 0; pass < 2; ++pass) {
         if (only_pass >= 0 && pass != only_pass) continue;
         const bool forward = pass == 0;
+        if (!forward && d.n_top_tiles > 0)
+            HIP_TRY(launch_dense_top(fbytes, top, d.n_top_tiles, d.top_tiles_wide, d.n_top_tiles_wide, bf.max_k, st));
         const int tile = effective_tile(s, fbytes, bf.max_k);
         if (is_panel_tile(tile)) {
             bf.ntasks = forward ? d.n_fwd_tasks_wide : d.n_bwd_tasks_wide;
@@ -959,6 +1089,7 @@ int solve_impl(cholespy_gpu_solver *s, int fbytes, int k, const void *b, void *x
     int rc = report_give_up(s);
     if (rc != CHOLESPY_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (only_pass < 0 && solves_directly(s, b, x, k, (size_t)fbytes)) return solve_blocks(s, k, b, x, st);
     rc = prepare_buffers(s, k, st);
     if (rc != CHOLESPY_OK) return rc;
     // Pass order. A forward pass publishes partial sums, gathered right-hand
@@ -1253,7 +1384,13 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
     if (ns >= 8 && !std::getenv("CHOLESPY_SPLIT_ENTRIES")) opt.split_entries = 0;
     if (ns >= 8 && !std::getenv("CHOLESPY_SPLIT_GATHER")) opt.split_gather = 257;
     if (ns >= 8) opt.wide_list = false;
+    // Levels of many systems overlap, so a dense top pays only where it ends
+    // the long unsplit tasks of each system's last levels: 64 grid systems, n
+    // 1k-20k, k 1-128: 1153 us without one, 1021 / 973 / 956 / 976 / 1051 us
+    // with up to 600 / 800 / 1000 / 1200 / 1600 rows.
+    if (ns >= 8) opt.top_max_rows = 1000;
     std::vector<BlockPlan> plans((size_t)ns);
+    std::vector<std::vector<int>> srcs((size_t)ns);
     {
         const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
         std::vector<std::thread> pool;
@@ -1263,7 +1400,7 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
                 for (int i = (int)w; i < ns; i += (int)hw) {
                     const auto &h = s->pending[i];
                     try {
-                        plans[i] = build_block_plan_structure(s->sys_n[i], h.colptr.data(), h.rowidx.data(), opt);
+                        plans[i] = plan_structure(s->sys_n[i], h.colptr.data(), h.rowidx.data(), opt, s->fbytes, srcs[i]);
                     } catch (const std::exception &ex) {
                         errors[i] = ex.what();
                     }
@@ -1277,7 +1414,7 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
     // offsets; tasks of all systems interleaved by block level.
     BlockPlan G;
     G.n = s->n;
-    std::vector<int> blk_sys, gperm((size_t)s->n);
+    std::vector<int> blk_sys, gperm((size_t)s->n), gsrc((size_t)s->n), fperm((size_t)s->n);
     s->sys_slots.assign((size_t)ns, 0);
     s->sys_slot0.assign((size_t)ns, 0);
     s->sys_splits.assign((size_t)ns, 0);
@@ -1293,7 +1430,12 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
         s->sys_slots[i] = P.rptr[P.nblocks];
         s->sys_split0[i] = SP0;
         s->sys_splits[i] = P.nsplit_rows;
-        for (int r = 0; r < s->sys_n[i]; ++r) gperm[(size_t)R0 + r] = R0 + s->pending[i].perm[r];
+        const bool whole = P.nblocks == 1 && P.is_whole(0);
+        for (int r = 0; r < s->sys_n[i]; ++r) {
+            fperm[(size_t)R0 + r] = R0 + s->pending[i].perm[r];
+            gsrc[(size_t)R0 + r] = R0 + srcs[i][r];
+            gperm[(size_t)R0 + r] = R0 + (whole ? r : s->pending[i].perm[srcs[i][r]]);
+        }
         for (int b = 0; b < P.nblocks; ++b) {
             G.start.push_back(P.start[b] + R0);
             G.rptr.push_back(P.rptr[b] + S0);
@@ -1301,7 +1443,10 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
             G.level_fwd.push_back(P.level_fwd[b]);
             G.level_bwd.push_back(P.level_bwd[b]);
             blk_sys.push_back(i);
+            G.top_off.push_back(P.is_top(b) ? P.top_off[b] + G.top_size : -1);
+            G.top_whole.push_back(P.is_whole(b));
         }
+        G.top_size += P.top_size;
         for (int v : P.rlist) G.rlist.push_back(v + R0);
         for (int r = 0; r < s->sys_n[i]; ++r) G.contrib_ptr.push_back(P.contrib_ptr[r] + C0);
         for (int v : P.contrib_slot) G.contrib_slot.push_back(v + S0);
@@ -1367,8 +1512,7 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
         emit(btasks_w, false, true, G.bwd_task_wide);
     }
     plans.clear();
-    HIP_TRY(hipMemcpy(s->perm, gperm.data(), (size_t)s->n * sizeof(int), hipMemcpyHostToDevice));
-    int rc = upload_plan(s, G, &blk_sys);
+    int rc = upload_plan(s, G, gperm, &blk_sys);
     if (rc != CHOLESPY_OK) return rc;
     {
         // The factors one after another, as the block-diagonal factor of the merged plan.
@@ -1384,7 +1528,7 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
         DeviceTemp trow, tval;
         HIP_TRY(trow.put(rowidx.data(), rowidx.size()));
         HIP_TRY(tval.put(val.data(), val.size()));
-        rc = fill_plan_values(s, G, colptr.data(), trow.as<int>(), tval.as<double>());
+        rc = fill_plan_values(s, G, colptr.data(), trow.as<int>(), tval.as<double>(), gsrc, fperm);
         if (rc != CHOLESPY_OK) return rc;
     }
     dev_free(s->blk_sys);
@@ -1540,6 +1684,7 @@ int cholespy_solver_solve_noalloc(cholespy_gpu_solver *s, int n_rhs, const void 
     const auto region = [](size_t bytes) { return (bytes + 255) & ~size_t(255); };
     const size_t vec = region((size_t)s->n * k * fb), part = region((size_t)s->plan.nslots * k * fb),
                  spart = region((size_t)s->plan.nsplit_rows * k * fb);
+    if (solves_directly(s, b, x, n_rhs, fb)) return solve_blocks(s, n_rhs, b, x, static_cast<hipStream_t>(stream));
     const size_t need = 3 * vec + part + spart;
     if (need > kScratchBytes)
         return fail(CHOLESPY_ERR_INVALID_ARGUMENT,

@@ -142,6 +142,28 @@ const void *block_pass_kernel(int float_bytes, bool forward, int tile);
 hipError_t launch_block_pass(int float_bytes, bool forward, const BlockPassBuffers &buf, int grid,
                              QueueState &queues, hipStream_t stream);
 
+// Dense top blocks (dense_top.hip): z_T = S^{-1} r_T. One record per panel of
+// 16 outputs (narrow: up to 4 right-hand sides) or per two panels (wide).
+struct DenseTopTile {
+    int row0, n;     // first row of the top block and its rows
+    int panel, sys;
+    int64_t off;     // the inverse's first element
+};
+struct DenseTopArgs {
+    const DenseTopTile *tiles;     // null: one system, whose top is the n rows from row0
+    int row0, n;
+    const void *M, *in;            // the inverses; r_T at rows row0.. of `in`
+    void *z, *x;                   // z may be null
+    const int *perm;               // solution row of each row; null: the row itself
+    int k, xmode;                  // xmode as in BlockPassBuffers
+    const int *sys_k;              // batches (null for a single system)
+    const long long *sys_vbase;
+};
+hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int narrow_tiles, const DenseTopTile *wide_list,
+                            int wide_tiles, int max_k, hipStream_t stream);
+// bytes (a multiple of 4) from src to dst, device to device, as a kernel.
+hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream);
+
 // Mixed-precision refinement helpers (refine.hip).
 hipError_t launch_cast_to_f32(const double *in, float *out, size_t count, hipStream_t stream);
 // With norm2 (k doubles, zeroed by the caller) not null, also adds the

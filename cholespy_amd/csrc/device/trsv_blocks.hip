@@ -331,7 +331,7 @@ __global__ __launch_bounds__(kTaskThreads) void block_forward(BlockPassArgs<F> a
         };
         F mpre[kPre];
         int npre = 0;
-        if (kind != 1 && rho < last) {
+        if (kind != 1 && kind != 4 && rho < last) {
             int cb, ce;
             cols_of(clo, min(chi, clo + a.chunk), cb, ce);
             npre = max(0, min(kPre, ce - cb));
@@ -344,8 +344,8 @@ __global__ __launch_bounds__(kTaskThreads) void block_forward(BlockPassArgs<F> a
         }
         for (int t0 = 0; t0 < k; t0 += KT) {
             const int kt = min(KT, k - t0);
-            if (kind == 1) {   // gather-only task: rows [first, last) of r_B to rbuf
-                gather_partials(a, bv, pv, rb, (F *)nullptr, a0, first, last, t0, kt, k, KT, KT, true);
+            if (kind == 1 || kind == 4) {   // gather-only task: rows [first, last) of r_B to rbuf (top: y)
+                gather_partials(a, bv, pv, kind == 4 ? yv : rb, (F *)nullptr, a0, first, last, t0, kt, k, KT, KT, true);
                 if (a.trace && tid == 0 && t0 == 0) a.trace[4 * (size_t)tk + 1] = wall_clock64();
                 continue;
             }
@@ -710,7 +710,10 @@ hipError_t launch_impl(bool forward, const BlockPassBuffers &bf, int grid, Queue
             f.leaf_trace = a.trace + 4 * leaf_off;
         }
         lds = std::max(lds, (size_t)kLeafWaves * kLeafMaxRows * kNarrowTile * sizeof(F));
-        const int g = std::max(1, std::min(grid, std::max(n_main, (n_leaf + kLeafWaves - 1) / kLeafWaves)));
+        // Workgroups for the leaf tasks and, on a grid that holds them, others
+        // for the block tasks, which then have their records, row indices and
+        // M entries loaded by the time their inputs are published.
+        const int g = std::max(1, std::min(grid, n_main + (n_leaf + kLeafWaves - 1) / kLeafWaves));
         // Every leaf queue needs a wavefront serving it (wavefront w serves
         // queue w mod nq, and the first workgroups are dispatched first).
         f.lqa.nq = std::max(1, std::min(f.lqa.nq, g * kLeafWaves));
