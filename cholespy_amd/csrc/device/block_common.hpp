@@ -44,11 +44,12 @@ struct BlockPassArgs {
     // Optional task timeline (nullptr = off): per task, 4 words =
     // {start, after the gather phase, end, workgroup id} in wall-clock ticks (100 MHz).
     unsigned long long *trace;
-    // Leaf phase of the launch (narrow kernels; n_leaf = 0: none): n_leaf
-    // leaf task records at leaf_task, taken per wavefront from the queues
-    // lqa, before the block tasks (forward) or after them (backward).
+    // Leaf phase of the launch (n_leaf = 0: none): n_leaf leaf task records at
+    // leaf_task, taken per wavefront from the queues lqa, before the block
+    // tasks (forward) or after them (backward); panel kernels: leaf_chunks
+    // units of right-hand sides each.
     const int *leaf_task;
-    int n_leaf;
+    int n_leaf, leaf_chunks;
     QueueArgs lqa;
     unsigned long long *leaf_trace;
 };
@@ -74,6 +75,9 @@ int panel_lds_bytes();
 const void *block_panel_kernel(int float_bytes, bool forward, int nt);
 hipError_t launch_panel_f32(bool forward, const BlockPassArgs<float> &a, int nt, int grid, hipStream_t stream);
 hipError_t launch_panel_f64(bool forward, const BlockPassArgs<double> &a, int nt, int grid, hipStream_t stream);
+// Their leaf phase (a.leaf_task, a.n_leaf, a.leaf_chunks) in a launch of its own.
+hipError_t launch_panel_leaf_f32(bool forward, const BlockPassArgs<float> &a, hipStream_t stream);
+hipError_t launch_panel_leaf_f64(bool forward, const BlockPassArgs<double> &a, hipStream_t stream);
 
 namespace {
 

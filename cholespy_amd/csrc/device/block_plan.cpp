@@ -55,7 +55,7 @@ TaskShape wide_shape(const BlockPlanOptions &o) {
     return TaskShape{o.wide_fwd_rows,          o.bwd_cols,      o.wide_split_gather, o.wide_fwd_rows_big,
                      o.bwd_cols_big,           o.split_entries, o.max_split,         o.wide_level_tasks,
                      o.wide_min_split_entries, o.fwd_rows,      o.split_gather,      o.wide_fine_bwd_cols_big,
-                     false,                    o.fwd_rows_big,  o.critical_order};
+                     true,                     o.fwd_rows_big,  o.critical_order};
 }
 
 // Tasks of both passes in level order (stable in block index) for one task shape.
@@ -82,6 +82,13 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
         b.push_back(hi);
         return b;
     };
+    // Leaf blocks: run by the leaf kernels, so never gathered in tasks of their
+    // own and never split.
+    auto is_leaf = [&](int b) {
+        const int m = start[b + 1] - start[b], R = P.rptr[b + 1] - P.rptr[b];
+        return opt.leaf_partition && !P.is_top(b) && P.level_fwd[b] == 0 && m <= kLeafMaxM && m + R <= kLeafMaxRows &&
+               m < opt.busy_split_gather && opt.busy_fwd_rows <= 64 && opt.bwd_cols <= 32;
+    };
     // Entries per split task at a level: split_entries, or finer (down to
     // min_split_entries) when the level's large blocks would otherwise give
     // fewer than level_tasks tasks.
@@ -97,7 +104,7 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
         for (size_t q = lo; q < hi; ++q) {
             const int b = order[q];
             const int64_t m = start[b + 1] - start[b], R = P.rptr[b + 1] - P.rptr[b];
-            if (m >= sg && !P.is_top(b)) entries += m * (m + 1) / 2 + R * m;
+            if (m >= sg && !P.is_top(b) && !is_leaf(b)) entries += m * (m + 1) / 2 + R * m;
         }
         const int64_t want = entries / opt.level_tasks;
         level_split = (int)std::max<int64_t>(opt.min_split_entries, std::min<int64_t>(opt.split_entries, want));
@@ -141,14 +148,14 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
                 for (int r0 = 0; r0 < m; r0 += rows_l) push(L.fwd, b, r0, std::min(m, r0 + rows_l), 4);
                 continue;
             }
-            if (m < sg_l) continue;
+            if (m < sg_l || is_leaf(b)) continue;
             for (int r0 = 0; r0 < m; r0 += rows_l) push(L.fwd, b, r0, std::min(m, r0 + rows_l), 1);
         }
         for (size_t q = lo; q < hi; ++q) {
             const int b = order[q], m = start[b + 1] - start[b];
             const int rows = m + (P.rptr[b + 1] - P.rptr[b]);
             if (P.is_top(b)) continue;
-            if (m < sg_l) {
+            if (m < sg_l || is_leaf(b)) {
                 for (int r0 = 0; r0 < rows; r0 += rows_l)
                     push(L.fwd, b, r0, std::min(rows, r0 + rows_l), 0);
                 continue;
@@ -205,7 +212,7 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
             const int b = order[q], m = start[b + 1] - start[b];
             const int rows = m + (P.rptr[b + 1] - P.rptr[b]);
             if (P.is_top(b)) continue;
-            const bool big = m >= sg_l;
+            const bool big = m >= sg_l && !is_leaf(b);
             const int wmax = big ? bcols_big_l : opt.bwd_cols;
             for (int c0 = 0; c0 < m; c0 += wmax) {
                 const int c1 = std::min(m, c0 + wmax), w = c1 - c0;
@@ -232,11 +239,6 @@ TaskList make_tasks(const BlockPlan &P, const TaskShape &opt) {
 
     // 6. Leaf blocks' tasks first (forward) and last (backward), otherwise in
     //    the same order.
-    auto is_leaf = [&](int b) {
-        const int m = start[b + 1] - start[b], R = P.rptr[b + 1] - P.rptr[b];
-        return opt.leaf_partition && !P.is_top(b) && P.level_fwd[b] == 0 && m <= kLeafMaxM && m + R <= kLeafMaxRows &&
-               m < opt.split_gather && opt.fwd_rows <= 64 && opt.bwd_cols <= 32;
-    };
     auto partition = [&](std::vector<int> &tasks, bool leaf_first, int &count) {
         std::vector<int> leaf, rest;
         const size_t nt = tasks.size() / kTaskInts;
@@ -413,6 +415,8 @@ BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx
     P.n_leaf_bwd = narrow.n_leaf_bwd;
     P.fwd_task_wide.swap(wide.fwd);
     P.bwd_task_wide.swap(wide.bwd);
+    P.n_leaf_fwd_wide = wide.n_leaf_fwd;
+    P.n_leaf_bwd_wide = wide.n_leaf_bwd;
     P.nsplit_rows = std::max(narrow.nsplit_rows, wide.nsplit_rows);
     return P;
 }

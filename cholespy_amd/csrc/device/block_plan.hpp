@@ -150,8 +150,9 @@ struct BlockPlan {
     // over all tasks).
     int n_leaf_fwd = 0, n_leaf_bwd = 0;
     // The same two passes as tasks for wide right-hand sides (same records,
-    // BlockPlanOptions' wide_* shape, no leaf partition).
+    // BlockPlanOptions' wide_* shape), leaf tasks first and last as well.
     std::vector<int> fwd_task_wide, bwd_task_wide;
+    int n_leaf_fwd_wide = 0, n_leaf_bwd_wide = 0;
     // Dense top blocks (none, or one per system): top_off[b] = offset of the
     // block's inverse (top_entries(m) elements) in an array of its own, -1 for
     // other blocks (empty: no top block). They have no entries in mfwd /

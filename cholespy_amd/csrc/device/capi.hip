@@ -99,6 +99,7 @@ struct DeviceBlockPlan {
     int nblocks = 0, nslots = 0, nsplit_rows = 0, max_m = 0, max_rows = 0;
     int n_fwd_tasks = 0, n_bwd_tasks = 0;
     int n_leaf_fwd = 0, n_leaf_bwd = 0;   // leaf tasks: forward prefix, backward suffix
+    int n_leaf_fwd_wide = 0, n_leaf_bwd_wide = 0;
     int n_fwd_tasks_wide = 0, n_bwd_tasks_wide = 0;   // task lists of the panel (wide k) kernels
     int levels_fwd = 0, levels_bwd = 0;
     int64_t m_entries = 0;
@@ -314,6 +315,8 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
     d.n_bwd_tasks = (int)(P.bwd_task.size() / kTaskInts);
     d.n_leaf_fwd = P.n_leaf_fwd;
     d.n_leaf_bwd = P.n_leaf_bwd;
+    d.n_leaf_fwd_wide = P.n_leaf_fwd_wide;
+    d.n_leaf_bwd_wide = P.n_leaf_bwd_wide;
     d.n_fwd_tasks_wide = (int)(P.fwd_task_wide.size() / kTaskInts);
     d.n_bwd_tasks_wide = (int)(P.bwd_task_wide.size() / kTaskInts);
     d.levels_fwd = d.levels_bwd = 0;
@@ -1047,7 +1050,11 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         const int tile = effective_tile(s, fbytes, bf.max_k);
         if (is_panel_tile(tile)) {
             bf.ntasks = forward ? d.n_fwd_tasks_wide : d.n_bwd_tasks_wide;
-            bf.n_leaf = 0;
+            // Leaf units carry two tiles of 16 right-hand sides: for one tile
+            // the workgroups' own tasks stay (33^3 grid, k = 5, FP64: 175 us,
+            // 192 with units).
+            const bool units = s->leaf_kernels && bf.max_k > 16;
+            bf.n_leaf = units ? (forward ? d.n_leaf_fwd_wide : d.n_leaf_bwd_wide) : 0;
             bf.task = forward ? d.ftask_wide : d.btask_wide;
         } else {
             bf.ntasks = forward ? d.n_fwd_tasks : d.n_bwd_tasks;
@@ -1462,10 +1469,15 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
                               i, (int)t});
         G.n_leaf_fwd += P.n_leaf_fwd;
         G.n_leaf_bwd += P.n_leaf_bwd;
-        for (size_t t = 0; t < P.fwd_task_wide.size() / kTaskInts; ++t)
-            ftasks_w.push_back({P.level_fwd[P.fwd_task_wide[kTaskInts * t]], i, (int)t});
-        for (size_t t = 0; t < P.bwd_task_wide.size() / kTaskInts; ++t)
-            btasks_w.push_back({P.level_bwd[P.bwd_task_wide[kTaskInts * t]], i, (int)t});
+        const size_t nfw = P.fwd_task_wide.size() / kTaskInts, nbw = P.bwd_task_wide.size() / kTaskInts;
+        for (size_t t = 0; t < nfw; ++t)
+            ftasks_w.push_back({(int)t < P.n_leaf_fwd_wide ? -1 : P.level_fwd[P.fwd_task_wide[kTaskInts * t]], i, (int)t});
+        for (size_t t = 0; t < nbw; ++t)
+            btasks_w.push_back({t >= nbw - (size_t)P.n_leaf_bwd_wide ? std::numeric_limits<int>::max()
+                                                                     : P.level_bwd[P.bwd_task_wide[kTaskInts * t]],
+                                i, (int)t});
+        G.n_leaf_fwd_wide += P.n_leaf_fwd_wide;
+        G.n_leaf_bwd_wide += P.n_leaf_bwd_wide;
 
         G.max_m = std::max(G.max_m, P.max_m);
         G.max_rows = std::max(G.max_rows, P.max_rows);

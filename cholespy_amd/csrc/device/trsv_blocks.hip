@@ -647,6 +647,14 @@ hipError_t launch_narrow(bool forward, const BlockPassArgs<F> &a, int tile, size
                            stream);
 }
 
+// Leaf units of a panel pass from which they run in a launch of their own, at
+// the leaf kernel's occupancy (5 to 7 wavefronts per SIMD against the panel
+// kernels' 3 or 4), instead of overlapping the block levels in one launch. 64
+// grid systems, k 1-128, FP32 (44k units): 802 us fused, 670 apart;
+// icosphere(6), k = 128 (4.5k): 249 and 261; 48^3 grid, k = 32 (7.9k): 416 and
+// 438; 511 x 389 grid, k = 17, FP64 (5.6k): 264 and 282.
+constexpr long long kOwnLeafLaunch = 16384;
+
 template <typename F>
 hipError_t launch_impl(bool forward, const BlockPassBuffers &bf, int grid, QueueState &queues,
                        hipStream_t stream) {
@@ -684,40 +692,61 @@ hipError_t launch_impl(bool forward, const BlockPassBuffers &bf, int grid, Queue
     queues.fill(a.qa);
     a.leaf_task = nullptr;
     a.n_leaf = 0;
+    a.leaf_chunks = 1;
     a.leaf_trace = nullptr;
     if (bf.leaf_queues) bf.leaf_queues->fill(a.lqa);
     else a.lqa = QueueArgs{nullptr, 1, a.qa.spin_limit, a.qa.abort};
-    if (is_panel_tile(tile)) {
-        if constexpr (sizeof(F) == 4) return launch_panel_f32(forward, a, tile / 16, grid, stream);
-        else return launch_panel_f64(forward, a, tile / 16, grid, stream);
-    }
-    size_t lds = block_pass_lds(sizeof(F), forward ? bf.max_m : bf.max_rows, tile);
     // Leaf tasks (forward: the first n_leaf, backward: the last n_leaf): in
-    // the block launch's leaf phase (fused), or in their own launch before /
-    // after the block pass over the others.
+    // the block launch's leaf phase (fused, always so in the panel kernels), or
+    // in their own launch before / after the block pass over the others.
     const int n_leaf = std::min(bf.n_leaf, bf.ntasks);
     const int n_main = bf.ntasks - n_leaf;
-    if (bf.fused_leaves && n_leaf > 0) {
-        BlockPassArgs<F> f = a;
+    BlockPassArgs<F> f = a;
+    int fused_grid = grid;
+    if (n_leaf > 0 && (bf.fused_leaves || is_panel_tile(tile))) {
         const size_t leaf_off = forward ? 0 : (size_t)n_main;
         const size_t main_off = forward ? (size_t)n_leaf : 0;
         f.task = a.task + main_off * kDevTaskInts;
         f.ntasks = n_main;
         f.leaf_task = a.task + leaf_off * kDevTaskInts;
         f.n_leaf = n_leaf;
+        f.leaf_chunks = is_panel_tile(tile) ? (bf.max_k + 31) / 32 : 1;
         if (a.trace) {
             f.trace = a.trace + 4 * main_off;
             f.leaf_trace = a.trace + 4 * leaf_off;
         }
-        lds = std::max(lds, (size_t)kLeafWaves * kLeafMaxRows * kNarrowTile * sizeof(F));
         // Workgroups for the leaf tasks and, on a grid that holds them, others
         // for the block tasks, which then have their records, row indices and
         // M entries loaded by the time their inputs are published.
-        const int g = std::max(1, std::min(grid, n_main + (n_leaf + kLeafWaves - 1) / kLeafWaves));
+        const long long leaf_groups = ((long long)n_leaf * f.leaf_chunks + kLeafWaves - 1) / kLeafWaves;
+        fused_grid = (int)std::max<long long>(1, std::min<long long>(grid, n_main + leaf_groups));
         // Every leaf queue needs a wavefront serving it (wavefront w serves
         // queue w mod nq, and the first workgroups are dispatched first).
-        f.lqa.nq = std::max(1, std::min(f.lqa.nq, g * kLeafWaves));
-        return launch_narrow<F>(forward, f, tile, lds, g, stream);
+        f.lqa.nq = std::max(1, std::min(f.lqa.nq, fused_grid * kLeafWaves));
+    }
+    if (is_panel_tile(tile)) {
+        const bool own = (long long)n_leaf * f.leaf_chunks >= kOwnLeafLaunch;
+        auto leaves = [&]() {
+            if (!own || f.n_leaf == 0) return hipSuccess;
+            if constexpr (sizeof(F) == 4) return launch_panel_leaf_f32(forward, f, stream);
+            else return launch_panel_leaf_f64(forward, f, stream);
+        };
+        auto blocks = [&]() {
+            BlockPassArgs<F> m = f;
+            if (own) m.n_leaf = 0;
+            if (m.n_leaf == 0 && m.ntasks == 0) return hipSuccess;
+            const int g = own ? std::max(1, std::min(grid, n_main)) : fused_grid;
+            if constexpr (sizeof(F) == 4) return launch_panel_f32(forward, m, tile / 16, g, stream);
+            else return launch_panel_f64(forward, m, tile / 16, g, stream);
+        };
+        const hipError_t e = forward ? leaves() : blocks();
+        if (e != hipSuccess) return e;
+        return forward ? blocks() : leaves();
+    }
+    size_t lds = block_pass_lds(sizeof(F), forward ? bf.max_m : bf.max_rows, tile);
+    if (f.n_leaf > 0) {
+        lds = std::max(lds, (size_t)kLeafWaves * kLeafMaxRows * kNarrowTile * sizeof(F));
+        return launch_narrow<F>(forward, f, tile, lds, fused_grid, stream);
     }
     auto leaf = [&](int offset) -> hipError_t {
         BlockPassArgs<F> l = a;

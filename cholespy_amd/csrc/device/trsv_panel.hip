@@ -76,13 +76,13 @@ template <typename F, int NT> constexpr int batch_steps() { return sizeof(F) == 
 // more waves put more tasks in flight where many small tasks run at once
 // (the leaf levels, batches). FP32, 8 tiles: 224 -> 166 registers forward
 // (3 waves), 116 backward (4). FP32, up to 4 tiles: 4 waves forward, 5
-// backward. FP64 forward with 4 tiles: 3 waves (left alone the compiler
-// takes AGPRs and 2); other FP64 forward kernels would spill at more waves
-// and keep the default; FP64 backward with up to 4 tiles fits 4 waves.
+// backward. FP64 forward with up to 4 tiles: 3 waves (left alone the compiler
+// takes AGPRs and 2); with 8 tiles it would spill at more waves and keeps the
+// default; FP64 backward with up to 4 tiles fits 4 waves.
 template <typename F, int NT, bool Forward> constexpr int kMinWavesFor() {
     if (sizeof(F) == 4) return NT >= 8 ? 3 : 4;
     if (!Forward) return NT <= 4 ? 4 : 1;
-    return NT == 4 ? 3 : 1;
+    return NT <= 4 ? 3 : 1;
 }
 // Backward tasks stage the R-row indices they read in LDS (up to this many).
 constexpr int kStageRlist = 4096;
@@ -376,6 +376,203 @@ __device__ __forceinline__ void reduce_splits(F *red, const WaveWork &w, int wav
         }
 }
 
+// p[i], or zero without a branch: a load under a condition splits the unrolled
+// batches into blocks, and the loads of a batch then spill registers (up to
+// 161 in the leaf tasks below). p itself has to be readable.
+template <typename F>
+__device__ __forceinline__ typename Bits<F>::U load_or_zero(const F *p, int i, bool ok) {
+    const typename Bits<F>::U v = peek_bits(p + (ok ? i : 0));
+    return ok ? v : 0;
+}
+
+// Leaf phase at wide k: one wavefront runs a leaf block's task (block_plan.hpp;
+// up to 64 rows of M_B forward, 32 columns backward) for kLeafTiles tiles of
+// 16 right-hand sides. As in the narrow kernels every wavefront takes these
+// units first (forward) or after its workgroup's block tasks (backward), from
+// queues of their own.
+// Why a wavefront: a leaf block has a few rows to 64 and its task is a chain of
+// four memory latencies, 7 to 12 us as a workgroup of which three or four fit a
+// CU; 12 to 16 wavefronts do. 511 x 389 grid, k = 17, FP64 (5,629 leaf tasks)
+// 320 -> 264 us, 48^3 grid, k = 32, FP32 450 -> 416 us, 64 grid systems,
+// k 1-128, FP32 1013 -> 670 us (in a launch of their own: trsv_blocks.hip).
+constexpr int kLeafTiles = 2;
+
+// Forward unit: the right-hand sides from column t0.
+template <typename F>
+__device__ __forceinline__ void leaf_forward_unit(const BlockPassArgs<F> &a, const Task &task, const VecMap &vm, int t0) {
+    using Acc = typename Mfma<F>::Acc;
+    using U = typename Bits<F>::U;
+    constexpr int kFly = 4, kGroups = 4, NT = kLeafTiles;
+    const int lane = threadIdx.x % kWave, q = lane / 16, l = lane % 16;
+    const int first = task.first, last = task.last, a0 = task.a0, m = task.m, k = vm.k;
+    const int rows = m + task.R;
+    const F *M = a.M + task.moff;
+    const F *bv = a.b + vm.vbase;
+    // Lanes past the block's rows hold a valid row too: a batch's vector base
+    // points outside its arrays for any other system's rows.
+    const int pr = a.perm[a0 + min(lane, m - 1)];
+    const int nsteps = (min(last, m) + 3) / 4, groups = (last - first + 15) / 16;
+    F *yv = a.y + vm.vbase, *pv = a.part + vm.pbase;
+    Acc acc[kGroups][NT];
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[g][n] = Acc{};
+#pragma unroll 1
+    for (int s0 = 0; s0 < nsteps; s0 += kFly) {
+        U av[kFly][kGroups], bb[kFly][NT];
+#pragma unroll
+        for (int u = 0; u < kFly; ++u) {
+            const int col = 4 * (s0 + u) + q;
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) {
+                const int row = first + 16 * g + l;
+                av[u][g] = load_or_zero(M, fwd_off32(rows, col, row), row < last && col < m && col <= row);
+            }
+            const F *brow = bv + (long long)__shfl(pr, min(col, kLeafMaxM - 1), kWave) * k;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) bb[u][n] = load_or_zero(brow, t0 + 16 * n + l, col < m && t0 + 16 * n + l < k);
+        }
+#pragma unroll
+        for (int u = 0; u < kFly; ++u)
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g)
+                if (g < groups)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+                        acc[g][n] = Mfma<F>::step(from_bits<F>(av[u][g]), from_bits<F>(bb[u][n]), acc[g][n]);
+    }
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int rho = first + 16 * g + Mfma<F>::row(q, v);
+            if (g >= groups || rho >= last) continue;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const int t = t0 + 16 * n + l;
+                if (t >= k) continue;
+                // (Nobody waits on a leaf row's z: it needs no sentinel.)
+                if (rho < m) yv[(long long)(a0 + rho) * k + t] = acc[g][n][v];
+                else publish(&pv[(long long)(task.r0 + rho - m) * k + t], acc[g][n][v]);
+            }
+        }
+}
+
+// Backward unit (rowidx: kLeafMaxRows ints of this wavefront's LDS).
+template <typename F>
+__device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, const Task &task, const VecMap &vm, int t0,
+                                                   int *rowidx) {
+    using Acc = typename Mfma<F>::Acc;
+    using U = typename Bits<F>::U;
+    constexpr int kFly = 4, kGroups = 2, NT = kLeafTiles;
+    const int lane = threadIdx.x % kWave, q = lane / 16, l = lane % 16;
+    const int first = task.first, last = task.last, a0 = task.a0, m = task.m, r0 = task.r0, R = task.R, k = vm.k;
+    const int rows = m + R;
+    const F *M = a.M + task.moff;
+    const F *yv = a.y + vm.vbase, *zv = a.z + vm.vbase;
+    for (int i = lane; i < R; i += kWave) rowidx[i] = a.rlist[r0 + i];
+    // (This wavefront's LDS, written and read by it alone.)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int nsteps = (rows - first + 3) / 4, groups = (last - first + 15) / 16;
+    // In FP32 even and odd steps are summed apart (up to 40 steps of 4 rows:
+    // the rounding of one long running sum grows with its length).
+    Acc acc[kGroups][NT], odd[kGroups][NT];
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[g][n] = odd[g][n] = Acc{};
+#pragma unroll 1
+    for (int s0 = 0; s0 < nsteps; s0 += kFly) {
+        U av[kFly][kGroups], bb[kFly][NT];
+        const F *src[kFly];
+#pragma unroll
+        for (int u = 0; u < kFly; ++u) {
+            const int rho = first + 4 * (s0 + u) + q;
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) {
+                const int c = first + 16 * g + l;
+                av[u][g] = load_or_zero(M, bwd_off32(m, rho, c), c < last && rho < rows && rho >= c);
+            }
+            // (Rows past the end read row a0 of y and drop it.)
+            const int zr = lds_int(rowidx, min(max(rho - m, 0), kLeafMaxRows - 1));
+            src[u] = rho < m || rho >= rows ? yv + (long long)(a0 + (rho < m ? rho : 0)) * k : zv + (long long)zr * k;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) bb[u][n] = load_or_zero(src[u], t0 + 16 * n + l, rho < rows && t0 + 16 * n + l < k);
+        }
+#pragma unroll
+        for (int u = 0; u < kFly; ++u) {
+            // (y rows never hold the sentinel, nor do entries read as zero.)
+            F b[NT];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) b[n] = ready_value(src[u] + t0 + 16 * n + l, bb[u][n], a.status, a.qa);
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g)
+                if (g < groups)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        Acc &sum = sizeof(F) == 4 && u % 2 ? odd[g][n] : acc[g][n];
+                        sum = Mfma<F>::step(from_bits<F>(av[u][g]), b[n], sum);
+                    }
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+            if (sizeof(F) == 4) acc[g][n] += odd[g][n];
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int c = first + 16 * g + Mfma<F>::row(q, v);
+            if (g >= groups || c >= last) continue;
+            const long long o = vm.vbase + (long long)a.perm[a0 + c] * k + t0 + l;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                if (t0 + 16 * n + l >= k) continue;
+                if (a.xmode == 0) {
+                    static_cast<F *>(a.x)[o + 16 * n] = acc[g][n][v];
+                } else {
+                    double *x64 = static_cast<double *>(a.x);
+                    x64[o + 16 * n] = (a.xmode == 2 ? x64[o + 16 * n] : 0.0) + (double)acc[g][n][v];
+                }
+            }
+        }
+    // Restore the sentinel in this unit's columns of the block's partial slots
+    // for the next solve (once per block: its first column task).
+    if (first == 0) {
+        const F sent = from_bits<F>(Bits<F>::sentinel);
+        const int w = min(16 * NT, k - t0);
+        F *pv = a.part + vm.pbase + (long long)r0 * k + t0;
+        for (int i = lane; i < R * 16 * NT; i += kWave)
+            if (i % (16 * NT) < w) pv[(long long)(i / (16 * NT)) * k + i % (16 * NT)] = sent;
+    }
+}
+
+// Takes units until this wavefront's queue is exhausted, the next one
+// requested while a unit runs (trsv_blocks.hip leaf_phase).
+template <typename F, bool FORWARD>
+__device__ __forceinline__ void leaf_phase_wide(const BlockPassArgs<F> &a, int *lds) {
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int q = (blockIdx.x * (kTaskThreads / kWave) + wave) % a.lqa.nq, units = a.n_leaf * a.leaf_chunks;
+    int t = lane == 0 ? take_ticket(a.lqa, q, units) : 0;
+    t = __builtin_amdgcn_readfirstlane(t);
+    while (t >= 0) {
+        const int next = lane == 0 ? take_ticket(a.lqa, q, units) : 0;
+        const Task task = load_task_at(a.leaf_task, t / a.leaf_chunks);
+        const VecMap vm = vec_map(a, task);
+        const int t0 = t % a.leaf_chunks * kLeafTiles * 16;
+        if (t0 < vm.k) {
+            if (FORWARD) leaf_forward_unit<F>(a, task, vm, t0);
+            else leaf_backward_unit<F>(a, task, vm, t0, lds + wave * kLeafMaxRows);
+        }
+        t = __builtin_amdgcn_readfirstlane(next);
+    }
+}
+
 template <typename F, int NT>
 __global__ __launch_bounds__(kTaskThreads) __attribute__((amdgpu_waves_per_eu(kMinWavesFor<F, NT, true>())))
 void block_forward_panel(BlockPassArgs<F> a) {
@@ -389,6 +586,10 @@ void block_forward_panel(BlockPassArgs<F> a) {
     __shared__ GatherStage stage;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int qid = blockIdx.x % a.qa.nq;
+    if (a.n_leaf > 0) {   // leaf tasks first: they wait on nothing
+        leaf_phase_wide<F, true>(a, nullptr);
+        __syncthreads();
+    }
     int tk = wg_first_ticket(a.qa, qid, a.ntasks, &s_next);
     while (tk >= 0) {
         if (a.trace && tid == 0) a.trace[4 * (size_t)tk] = wall_clock64();
@@ -560,7 +761,7 @@ void block_forward_panel(BlockPassArgs<F> a) {
         tk = s_next;
         __syncthreads();
     }
-    if (tid == 0) finish_queues(a.qa);
+    if (tid == 0) finish_queues(a.qa, a.lqa.ctr, a.n_leaf > 0 ? a.lqa.nq : 0);
 }
 
 template <typename F, int NT>
@@ -733,7 +934,27 @@ void block_backward_panel(BlockPassArgs<F> a) {
         tk = s_next;
         __syncthreads();
     }
-    if (tid == 0) finish_queues(a.qa);
+    if (a.n_leaf > 0) {   // leaf tasks last: they wait on the block tasks' z
+        leaf_phase_wide<F, false>(a, reinterpret_cast<int *>(smem));
+        __syncthreads();
+    }
+    if (tid == 0) finish_queues(a.qa, a.lqa.ctr, a.n_leaf > 0 ? a.lqa.nq : 0);
+}
+
+// The same units in a launch of their own, wavefront w running unit w.
+template <typename F, bool FORWARD>
+__global__ __launch_bounds__(kTaskThreads) __attribute__((amdgpu_waves_per_eu(sizeof(F) == 4 ? 5 : FORWARD ? 3 : 4)))
+void leaf_units(BlockPassArgs<F> a) {
+    __shared__ int rowidx[FORWARD ? 1 : kTaskThreads / kWave * kLeafMaxRows];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const long long u = (long long)blockIdx.x * (kTaskThreads / kWave) + wave;
+    if (u >= (long long)a.n_leaf * a.leaf_chunks) return;
+    const Task task = load_task_at(a.leaf_task, (int)(u / a.leaf_chunks));
+    const VecMap vm = vec_map(a, task);
+    const int t0 = (int)(u % a.leaf_chunks) * kLeafTiles * 16;
+    if (t0 >= vm.k) return;
+    if (FORWARD) leaf_forward_unit<F>(a, task, vm, t0);
+    else leaf_backward_unit<F>(a, task, vm, t0, rowidx + wave * kLeafMaxRows);
 }
 
 }  // namespace
@@ -760,9 +981,26 @@ template <typename F>
 static hipError_t launch_panel_impl(bool forward, const BlockPassArgs<F> &args, int nt, int grid, hipStream_t stream) {
     BlockPassArgs<F> a = args;
     a.lds_bytes = panel_lds_bytes();
+    static_assert(kTaskThreads / kWave * kLeafMaxRows * sizeof(int) <= 16 * 1024, "leaf row indices fit the least LDS");
     void *p[] = {&a};
     return hipLaunchKernel(block_panel_kernel(sizeof(F), forward, nt), dim3(grid), dim3(kTaskThreads), p,
                            (size_t)a.lds_bytes, stream);
+}
+
+template <typename F>
+static hipError_t launch_leaf_impl(bool forward, const BlockPassArgs<F> &args, hipStream_t stream) {
+    BlockPassArgs<F> a = args;
+    void *p[] = {&a};
+    const void *kern = forward ? reinterpret_cast<const void *>(&leaf_units<F, true>)
+                               : reinterpret_cast<const void *>(&leaf_units<F, false>);
+    const long long per = kTaskThreads / kWave, units = (long long)a.n_leaf * a.leaf_chunks;
+    return hipLaunchKernel(kern, dim3((unsigned)((units + per - 1) / per)), dim3(kTaskThreads), p, 0, stream);
+}
+hipError_t launch_panel_leaf_f32(bool forward, const BlockPassArgs<float> &a, hipStream_t stream) {
+    return launch_leaf_impl<float>(forward, a, stream);
+}
+hipError_t launch_panel_leaf_f64(bool forward, const BlockPassArgs<double> &a, hipStream_t stream) {
+    return launch_leaf_impl<double>(forward, a, stream);
 }
 
 hipError_t launch_panel_f32(bool forward, const BlockPassArgs<float> &a, int nt, int grid, hipStream_t stream) {
