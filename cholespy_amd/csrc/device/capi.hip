@@ -109,11 +109,11 @@ struct DeviceBlockPlan {
     int *cptr = nullptr, *cslot = nullptr, *gslot = nullptr;
     int *ftask = nullptr, *btask = nullptr;
     int *ftask_wide = nullptr, *btask_wide = nullptr;
-    // Dense top blocks (block_plan.hpp): their inverses and the tile lists of
+    // Dense top blocks (block_plan.hpp): their inverses and the tile list of
     // the dense product. whole: a single system that is one top block.
     void *mtop = nullptr;
-    DenseTopTile *top_tiles = nullptr, *top_tiles_wide = nullptr;
-    int n_top_tiles = 0, n_top_tiles_wide = 0;
+    DenseTopTile *top_tiles = nullptr;
+    int n_top_tiles = 0;
     bool whole = false;
     int top_rows = 0;      // of a single system
     int *perm = nullptr;   // caller row of each plan row
@@ -121,7 +121,6 @@ struct DeviceBlockPlan {
     void release() {
         dev_free(mtop);
         dev_free(top_tiles);
-        dev_free(top_tiles_wide);
         dev_free(perm);
         dev_free(start);
         dev_free(rptr);
@@ -357,22 +356,16 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mfwd), me * fb));
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mbwd), me * fb));
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mtop), (size_t)P.top_size * fb));
-    std::vector<DenseTopTile> tiles, wide;
+    std::vector<DenseTopTile> tiles;
     for (int b = 0; b < P.nblocks; ++b) {
         if (!P.is_top(b)) continue;
         const int m = P.start[b + 1] - P.start[b], panels = (m + 15) / 16, sys = blk_sys ? (*blk_sys)[b] : 0;
-        for (int p = 0; p < panels; ++p) {
-            const DenseTopTile t{P.start[b], m, p, sys, P.top_off[b]};
-            tiles.push_back(t);
-            if (p % 2 == 0) wide.push_back(t);
-        }
+        for (int p = 0; p < panels; ++p) tiles.push_back(DenseTopTile{P.start[b], m, p, sys, P.top_off[b]});
     }
     d.n_top_tiles = (int)tiles.size();
-    d.n_top_tiles_wide = (int)wide.size();
     d.top_rows = !blk_sys && !P.top_off.empty() ? P.n - P.start[P.nblocks - 1] : 0;
     d.whole = !blk_sys && P.nblocks == 1 && P.is_whole(0);
     HIP_TRY(upload(&d.top_tiles, tiles.data(), tiles.size()));
-    HIP_TRY(upload(&d.top_tiles_wide, wide.data(), wide.size()));
     for (auto &row : s->grid_blocks)
         for (int &g : row) g = 0;
     s->buffers_path = -1;
@@ -1039,14 +1032,14 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         else if (only_pass < 0)
             top.in = b;
         if (only_pass != 0)
-            HIP_TRY(launch_dense_top(fbytes, top, d.n_top_tiles, d.top_tiles_wide, d.n_top_tiles_wide, k, st));
+            HIP_TRY(launch_dense_top(fbytes, top, d.n_top_tiles, k, st));
         return CHOLESPY_OK;
     }
     for (int pass = 0; pass < 2; ++pass) {
         if (only_pass >= 0 && pass != only_pass) continue;
         const bool forward = pass == 0;
         if (!forward && d.n_top_tiles > 0)
-            HIP_TRY(launch_dense_top(fbytes, top, d.n_top_tiles, d.top_tiles_wide, d.n_top_tiles_wide, bf.max_k, st));
+            HIP_TRY(launch_dense_top(fbytes, top, d.n_top_tiles, bf.max_k, st));
         const int tile = effective_tile(s, fbytes, bf.max_k);
         if (is_panel_tile(tile)) {
             bf.ntasks = forward ? d.n_fwd_tasks_wide : d.n_bwd_tasks_wide;

@@ -10,7 +10,7 @@
 // (k = 3): icosphere(3), n = 642, FP32 52.9 -> 6.5 us; a 61 x 47 grid, FP64
 // 60.4 -> 13.4 us (its 66 MB inverse at 5 TB/s); icosphere(5), FP32, a top of
 // 2,640 rows 91.9 -> 45.6 us; icosphere(6), k = 128, FP32, a top of 3,488 rows
-// 371 -> 259 us. choose_dense_top (block_plan.cpp) weighs the two.
+// 371 -> 242 us. choose_dense_top (block_plan.cpp) weighs the two.
 //
 // Rounding: an inverse rounded to FP32 keeps the block passes' accuracy only
 // if its long dot products do not round in FP32 as well (one running FP32 sum
@@ -67,14 +67,14 @@ struct Top {
 };
 // Consecutive workgroups go to different XCDs (round robin over 8): give each
 // XCD a run of consecutive panels, so that what neighbours share stays in one L2.
-__device__ __forceinline__ Top top_of(const DenseTopArgs &a, int panels_per_group) {
+__device__ __forceinline__ Top top_of(const DenseTopArgs &a) {
     const int count = gridDim.x, per = count / 8, extra = count % 8, x = blockIdx.x % 8;
     const int g = x * per + min(x, extra) + blockIdx.x / 8;
     Top r;
     if (!a.tiles) {   // one system: no record to load
         r.row0 = a.row0;
         r.n = a.n;
-        r.panel = g * panels_per_group;
+        r.panel = g;
         r.k = a.k;
         r.vbase = 0;
         r.off = 0;
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kNarrowThreads) __attribute__((amdgpu_waves_per_eu(
     constexpr int kIn = kChunk * KT / kNarrowThreads;   // inputs a thread stages per chunk
     __shared__ __align__(16) F in[2][kChunk * KT];
     __shared__ double red[kNarrowWaves * 16 * KT];
-    const Top top = top_of(a, 1);
+    const Top top = top_of(a);
     const int k = top.k;
     if (k <= 0) return;
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
@@ -208,95 +208,123 @@ __global__ __launch_bounds__(kNarrowThreads) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
-// More right-hand sides: a workgroup takes two panels and NT tiles of 16
+// More right-hand sides: a workgroup takes a panel and NT tiles of 16
 // right-hand sides, its 8 wavefronts split the inputs and add their partial
-// tiles through LDS. A streams from the panels, B from the input rows (each
-// loaded once for both panels). Two wavefronts per SIMD cover the loads of
-// one group of inputs with the MFMAs of the other.
+// tiles through LDS. A streams from the panel, B from the input rows (out of
+// the L2: an XCD's workgroups read the same rows), D groups of inputs in
+// flight per wavefront. Bound by the latency of those streams, not by the
+// matrix cores. Two panels a workgroup with one group in flight and B loaded a
+// value at a time, against this: icosphere(6), k = 128, FP32 (top 3,488) 65 ->
+// 50 us, 511 x 389 grid, k = 17, FP64 (top 2,048) 39 -> 18 us, 48^3 grid,
+// k = 32, FP32 (top 6,256) 62 -> 56 us, a batch of 64 systems, k = 1 to 128,
+// FP32 159 -> 111 us; 33^3 grid, k = 5, FP64 (top 4,512) 63 -> 51 us. 16
+// wavefronts a workgroup measured the same.
 constexpr int kWideThreads = 512;
 constexpr int kWideWaves = kWideThreads / kWave;
-template <typename F, int NT>
-__global__ __launch_bounds__(kWideThreads) void dense_wide(DenseTopArgs a) {
+constexpr int kOneTileFly = 5;   // D of one tile
+template <typename F, int NT, int D>
+__device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top, int t0, double (*red)[kWave * 4]) {
     using P = Pack<F>;
     using Vec = typename P::Vec;
     using Acc = typename P::Acc;
-    constexpr int V = P::V, G = 4 * V, kPanels = 2, kTiles = kPanels * NT, kHalf = kWideWaves / 2;
-    __shared__ double red[kHalf][kTiles][kWave * 4];
-    const Top top = top_of(a, kPanels);
-    const int k = top.k, t0 = blockIdx.y * NT * 16;
-    if (t0 >= k) return;
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, q = lane / 16, l = lane % 16;
-    const bool two = (top.panel + 1) * 16 < top.npad;
-    const Vec *M0 = reinterpret_cast<const Vec *>(static_cast<const F *>(a.M) + top.off) + lane;
-    const Vec *M1 = two ? M0 + (size_t)top.npad * 16 / V : M0;
-    const F *src = static_cast<const F *>(a.in) + top.vbase + (long long)top.row0 * k + t0 + l;
-    double sum[kPanels][NT][4] = {};
+    constexpr int V = P::V, G = 4 * V, kHalf = kWideWaves / 2;
+    const int k = top.k;
+    const int lane = threadIdx.x % kWave, q = lane / 16, l = lane % 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const Buffer M(static_cast<const F *>(a.M) + top.off, (unsigned)top.npad * 16 * (unsigned)sizeof(F));
+    const Buffer src(static_cast<const F *>(a.in) + top.vbase + (long long)top.row0 * k,
+                     (unsigned)top.n * (unsigned)k * (unsigned)sizeof(F));
     const int ng = top.npad / G;
-    Vec m0 = {}, m1 = {};
-    F b[V][NT];
-    auto load = [&](int g) {
-        if (g < ng) {
-            m0 = M0[(size_t)g * kWave];
-            m1 = M1[(size_t)g * kWave];
-        }
+    Vec m[D];
+    // B of tile n, lane column l: right-hand side col0 + n, so that a lane's
+    // tiles are one load of NT consecutive values. Lanes past the row's end
+    // compute (and store) its last NT columns again. (NT > 1: k > 16.)
+    const int col0 = NT == 1 ? t0 + l : min(t0 + NT * l, k - NT);
+    const unsigned b0 = NT > 1 || col0 < k ? (unsigned)(q * k + col0) * (unsigned)sizeof(F) : 1u << 31;
+    F b[D][V][NT];
+    constexpr int kPer = NT * (int)sizeof(F) <= 16 ? NT : 16 / (int)sizeof(F);   // values per load
+    typedef F BVec __attribute__((ext_vector_type(kPer)));
+    auto load = [&](int d, int g) {
+        // (Groups past the end are past the end of both buffers: zero.)
+        m[d] = M.at<Vec>((unsigned)(g * kWave + lane) * (unsigned)sizeof(Vec));
 #pragma unroll
         for (int j = 0; j < V; ++j) {
-            const int r = g * G + 4 * j + q;
+            const unsigned at = b0 + (unsigned)((g * G + 4 * j) * k) * (unsigned)sizeof(F);
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
-                b[j][n] = r < top.n && t0 + 16 * n + l < k ? src[(long long)r * k + 16 * n] : F(0);
+            for (int n = 0; n < NT; n += kPer) {
+                if constexpr (kPer == 1) {
+                    b[d][j][n] = src.at<F>(at);
+                } else {
+                    const BVec v = src.at<BVec>(at + n * (unsigned)sizeof(F));
+#pragma unroll
+                    for (int e = 0; e < kPer; ++e) b[d][j][n + e] = v[e];
+                }
+            }
         }
     };
-    load(wave);
-    for (int g = wave; g < ng; g += kWideWaves) {
-        const Vec a0 = m0, a1 = m1;
-        F bb[V][NT];
 #pragma unroll
-        for (int j = 0; j < V; ++j)
+    for (int d = 0; d < D; ++d) {
+        load(d, wave + d * kWideWaves);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    double sum[NT][4] = {};
+    for (int g0 = wave; g0 < ng; g0 += D * kWideWaves) {
 #pragma unroll
-            for (int n = 0; n < NT; ++n) bb[j][n] = b[j][n];
-        load(g + kWideWaves);
-        // Two steps (8 products an entry) at a time, summed in FP64.
+        for (int d = 0; d < D; ++d) {
+            // Two steps (8 products an entry) at a time, summed in FP64.
 #pragma unroll
-        for (int j = 0; j < V; j += 2)
+            for (int j = 0; j < V; j += 2)
 #pragma unroll
-            for (int n = 0; n < NT; ++n)
+                for (int n = 0; n < NT; ++n) {
+                    const Acc acc = P::step(m[d][j + 1], b[d][j + 1][n], P::step(m[d][j], b[d][j][n], Acc{}));
 #pragma unroll
-                for (int p = 0; p < kPanels; ++p) {
-                    const Vec ap = p == 0 ? a0 : a1;
-                    const Acc acc = P::step(ap[j + 1], bb[j + 1][n], P::step(ap[j], bb[j][n], Acc{}));
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) sum[p][n][v] += (double)acc[v];
+                    for (int v = 0; v < 4; ++v) sum[n][v] += (double)acc[v];
                 }
+            // (The scheduler would gather the D loads at the loop's end, and
+            // its head would wait for all of them.)
+            __builtin_amdgcn_sched_barrier(0);
+            load(d, g0 + (D + d) * kWideWaves);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     // The upper half of the wavefronts hands its sums to the lower half, which
     // then shares out the tiles.
     for (int half = 1; half >= 0; --half) {
         if (wave / kHalf == half)
 #pragma unroll
-            for (int i = 0; i < kTiles; ++i)
+            for (int n = 0; n < NT; ++n)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) red[wave % kHalf][i][v * kWave + lane] = sum[i / NT][i % NT][v];
+                for (int v = 0; v < 4; ++v) red[wave % kHalf * NT + n][v * kWave + lane] = sum[n][v];
         __syncthreads();
         if (half == 1) {
             if (wave < kHalf)
 #pragma unroll
-                for (int i = 0; i < kTiles; ++i)
+                for (int n = 0; n < NT; ++n)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) sum[i / NT][i % NT][v] += red[wave][i][v * kWave + lane];
+                    for (int v = 0; v < 4; ++v) sum[n][v] += red[wave * NT + n][v * kWave + lane];
             __syncthreads();
         }
     }
-    for (int i = wave; i < kTiles; i += kWideWaves) {
-        const int p = i / NT, col = t0 + 16 * (i % NT) + l;
-        if (p == 1 && !two) continue;
+    for (int i = wave; i < 4 * NT; i += kWideWaves) {
+        const int n = i / 4, v = i % 4, col = col0 + n, e = v * kWave + lane, c = top.panel * 16 + P::row(q, v);
+        double s = 0.0;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int e = v * kWave + lane, c = (top.panel + p) * 16 + P::row(q, v);
-            const F s = (F)(red[0][i][e] + red[1][i][e] + red[2][i][e] + red[3][i][e]);
-            if (c < top.n && col < k) put(a, top, c, col, a.perm ? a.perm[top.row0 + c] : top.row0 + c, s);
-        }
+        for (int w = 0; w < kHalf; ++w) s += red[w * NT + n][e];
+        if (c < top.n && col < k) put(a, top, c, col, a.perm ? a.perm[top.row0 + c] : top.row0 + c, (F)s);
     }
+}
+
+template <typename F, int NT, int D>
+__global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(4))) void dense_wide(DenseTopArgs a) {
+    __shared__ double red[kWideWaves / 2 * NT][kWave * 4];
+    const Top top = top_of(a);
+    const int t0 = blockIdx.y * NT * 16;
+    if (t0 >= top.k) return;
+    // A rest of one tile: a batch's systems differ in their right-hand sides.
+    if (NT > 1 && top.k - t0 <= 16)
+        wide_tiles<F, 1, kOneTileFly>(a, top, t0, red);
+    else
+        wide_tiles<F, NT, D>(a, top, t0, red);
 }
 
 __global__ void copy_words(uint32_t *dst, const uint32_t *src, size_t count) {
@@ -314,25 +342,24 @@ hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t str
     return hipGetLastError();
 }
 
-hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int narrow_tiles, const DenseTopTile *wide_list,
-                            int wide_tiles, int max_k, hipStream_t stream) {
+hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int tiles, int max_k,
+                            hipStream_t stream) {
     DenseTopArgs a = args;
     void *p[] = {&a};
-    if (max_k <= kNarrowTile) {
-        const void *kern = float_bytes == 4 ? reinterpret_cast<const void *>(&dense_narrow<float, kNarrowTile>)
-                                            : reinterpret_cast<const void *>(&dense_narrow<double, kNarrowTile>);
-        return hipLaunchKernel(kern, dim3(narrow_tiles), dim3(kNarrowThreads), p, 0, stream);
-    }
-    if (a.tiles) a.tiles = wide_list;
-    const int nt = max_k <= 16 ? 1 : (max_k <= 32 ? 2 : 4);
     const void *kern;
-#define CHOLESPY_DENSE(F)                                                                \
-    (nt == 1 ? reinterpret_cast<const void *>(&dense_wide<F, 1>)                         \
-             : nt == 2 ? reinterpret_cast<const void *>(&dense_wide<F, 2>)               \
-                       : reinterpret_cast<const void *>(&dense_wide<F, 4>))
+    if (max_k <= kNarrowTile) {
+        kern = float_bytes == 4 ? reinterpret_cast<const void *>(&dense_narrow<float, kNarrowTile>)
+                                : reinterpret_cast<const void *>(&dense_narrow<double, kNarrowTile>);
+        return hipLaunchKernel(kern, dim3(tiles), dim3(kNarrowThreads), p, 0, stream);
+    }
+    const int nt = max_k <= 16 ? 1 : (max_k <= 32 ? 2 : 4);
+#define CHOLESPY_DENSE(F)                                                    \
+    (nt == 1   ? reinterpret_cast<const void *>(&dense_wide<F, 1, kOneTileFly>) \
+     : nt == 2 ? reinterpret_cast<const void *>(&dense_wide<F, 2, 3>)        \
+               : reinterpret_cast<const void *>(&dense_wide<F, 4, 2>))
     kern = float_bytes == 4 ? CHOLESPY_DENSE(float) : CHOLESPY_DENSE(double);
 #undef CHOLESPY_DENSE
-    return hipLaunchKernel(kern, dim3(wide_tiles, (max_k + 16 * nt - 1) / (16 * nt)), dim3(kWideThreads), p, 0, stream);
+    return hipLaunchKernel(kern, dim3(tiles, (max_k + 16 * nt - 1) / (16 * nt)), dim3(kWideThreads), p, 0, stream);
 }
 
 }  // namespace cholespy_amd

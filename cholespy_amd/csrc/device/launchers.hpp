@@ -143,7 +143,7 @@ hipError_t launch_block_pass(int float_bytes, bool forward, const BlockPassBuffe
                              QueueState &queues, hipStream_t stream);
 
 // Dense top blocks (dense_top.hip): z_T = S^{-1} r_T. One record per panel of
-// 16 outputs (narrow: up to 4 right-hand sides) or per two panels (wide).
+// 16 outputs.
 struct DenseTopTile {
     int row0, n;     // first row of the top block and its rows
     int panel, sys;
@@ -159,8 +159,8 @@ struct DenseTopArgs {
     const int *sys_k;              // batches (null for a single system)
     const long long *sys_vbase;
 };
-hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int narrow_tiles, const DenseTopTile *wide_list,
-                            int wide_tiles, int max_k, hipStream_t stream);
+hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int tiles, int max_k,
+                            hipStream_t stream);
 // bytes (a multiple of 4) from src to dst, device to device, as a kernel.
 hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream);
 

@@ -85,3 +85,22 @@ def test_batch_mixes_whole_systems_and_tops():
                 ref = oracle.solve(batch._factor(i), bs[i], np.float64)
                 assert np.abs(got[at:at + n * k].reshape(n, k) - ref).max() / np.abs(ref).max() < 1e-12, (i, k)
             at += n * k
+
+
+@pytest.mark.parametrize("ks", [[5, 17, 18, 19, 31, 6, 32, 16], [4, 33, 34, 47, 66, 7, 125, 64]])
+def test_batch_right_hand_sides_of_unequal_tiles(ks):
+    """The widest system of a batch sets the tiles of all (2 or 4 of 16
+    right-hand sides): rows that end before, inside and at the end of a tile."""
+    n = 20 * 21
+    v, idx = workloads.grid2d_laplacian(20, 21, 1.0)
+    batch = BatchedSolverD([(n, idx[0], idx[1], v, MatrixType.COO)] * len(ks))
+    bs = [np.random.default_rng(k).standard_normal((n, k)) for k in ks]
+    b = torch.tensor(np.concatenate([x.ravel() for x in bs]), device=DEV)
+    x = torch.zeros_like(b)
+    batch.solve(ks, b, x)
+    torch.cuda.synchronize()
+    batch._check()
+    got = np.split(x.cpu().numpy(), np.cumsum([n * k for k in ks])[:-1])
+    for i, k in enumerate(ks):
+        ref = oracle.solve(batch._factor(i), bs[i], np.float64)
+        assert np.abs(got[i].reshape(n, k) - ref).max() / np.abs(ref).max() < 1e-12, (i, k)
