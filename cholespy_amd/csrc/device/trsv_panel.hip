@@ -67,9 +67,14 @@ template <int NT> constexpr int kStepsFor() { return NT <= 2 ? 8 : 4; }
 // pays ~kBatchSteps times fewer dependent load rounds than one step at a
 // time.
 constexpr int kBatchTiles = 2;
-// FP32: 8 steps (12 for the 8-tile kernels, whose occupancy floors leave
-// room); FP64: 4 (more cost the forward kernels a wave per SIMD).
-template <typename F, int NT> constexpr int batch_steps() { return sizeof(F) == 4 ? (NT >= 8 ? 12 : 8) : (NT <= 2 ? 8 : 4); }
+// FP32: 8 steps (forward 12 for the 8-tile kernels, whose occupancy floors
+// leave room); FP64: 4 (more cost the forward kernels a wave per SIMD). The
+// backward kernels hold M_B of two batches and take what fits without spills
+// (FP64: 3; 4 measured 2 % slower on the 511 x 389 grid at k = 17).
+template <typename F, int NT, bool Forward> constexpr int batch_steps() {
+    if (Forward) return sizeof(F) == 4 ? (NT >= 8 ? 12 : 8) : (NT <= 2 ? 8 : 4);
+    return sizeof(F) == 4 ? (NT == 4 ? 6 : 8) : (NT <= 4 ? 3 : 4);
+}
 // Waves per SIMD the compiler must allow (amdgpu_waves_per_eu), chosen per
 // kernel as the most that compile with no register spills on gfx950. By
 // default the compiler keeps more accumulators in AGPRs and gets 2-3 waves;
@@ -385,6 +390,26 @@ __device__ __forceinline__ typename Bits<F>::U load_or_zero(const F *p, int i, b
     return ok ? v : 0;
 }
 
+// Waits for the B operands u of a batch that still hold the sentinel; at(q, j)
+// is the address of entry q, j. One test a batch: a test per entry made every
+// MFMA step a block of its own, with a full wait in front of it. (Entries are
+// then waited on one by one: loading the whole batch again until it is complete
+// slowed down whoever had to publish it.)
+template <typename F, int S, int T, typename At>
+__device__ __forceinline__ void settle(typename Bits<F>::U (&u)[S][T], int *status, const QueueArgs &qa, At at) {
+    bool waits = false;
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+#pragma unroll
+        for (int j = 0; j < T; ++j) waits |= u[q][j] == Bits<F>::sentinel;
+    if (!waits) return;
+#pragma unroll
+    for (int q = 0; q < S; ++q)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+            if (u[q][j] == Bits<F>::sentinel) u[q][j] = as_bits(wait_value(at(q, j), status, qa));
+}
+
 // Leaf phase at wide k: one wavefront runs a leaf block's task (block_plan.hpp;
 // up to 64 rows of M_B forward, 32 columns backward) for kLeafTiles tiles of
 // 16 right-hand sides. As in the narrow kernels every wavefront takes these
@@ -579,7 +604,7 @@ void block_forward_panel(BlockPassArgs<F> a) {
     using Acc = typename Mfma<F>::Acc;
     constexpr int kMaxTiles = NT;
     constexpr int kSteps = kStepsFor<NT>();
-    constexpr int kBatchSteps = batch_steps<F, NT>();
+    constexpr int kBatchSteps = batch_steps<F, NT, true>();
     extern __shared__ __align__(16) unsigned char smem[];
     F *rv = reinterpret_cast<F *>(smem);
     __shared__ int s_next;
@@ -770,11 +795,11 @@ void block_backward_panel(BlockPassArgs<F> a) {
     using Acc = typename Mfma<F>::Acc;
     constexpr int kMaxTiles = NT;
     constexpr int kSteps = kStepsFor<NT>();
-    constexpr int kBatchSteps = batch_steps<F, NT>();
+    constexpr int kBatchSteps = batch_steps<F, NT, false>();
     extern __shared__ __align__(16) unsigned char smem[];
     F *vs = reinterpret_cast<F *>(smem);
     __shared__ int s_next;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qid = blockIdx.x % a.qa.nq;
     int tk = wg_first_ticket(a.qa, qid, a.ntasks, &s_next);
     while (tk >= 0) {
@@ -806,6 +831,7 @@ void block_backward_panel(BlockPassArgs<F> a) {
             const WaveWork w = wave_work(wave, last - first, nT);
             const int cg0 = first + 16 * max(w.group, 0);
             const int c = cg0 + (lane & 15);   // A row (= column of M_B) of this lane
+            const int cc0 = min(c, last - 1);  // a column that exists: what columns past the end compute is not stored
             const int kk = lane >> 4;          // A column / B row within a step
             // The R rows the task reads, [rb0, rb1), have their indices staged
             // in LDS (one load each, all in parallel) when they fit.
@@ -827,68 +853,96 @@ void block_backward_panel(BlockPassArgs<F> a) {
             // idle ones included.
             using U = typename Bits<F>::U;
             const int hs = kind == 1 ? max(cg0, task.lo) : cg0;   // rows [hs, he)
-            const int nsteps = (he - hs + 3) / 4;
+            const int nsteps = w.ntiles > 0 ? (he - hs + 3) / 4 : 0;
             const int toff = (lane & 15) + 16 * w.tile0;
             const int nbt = NT <= kBatchTiles ? 1 : max(w.ntiles, w.nsplit > 1 ? 1 : 0);
             for (int tb = 0; tb < nbt; tb += kBatchTiles) {
                 Acc acc[kBatchTiles];
 #pragma unroll
                 for (int jj = 0; jj < kBatchTiles; ++jj) acc[jj] = Acc{};
-                // The batches, in two copies: R-row indices from LDS (staged) or
-                // from global memory. One copy choosing per row would join an
-                // LDS and a global load into one register, and the wait for it
-                // would drain every M load in flight.
-                auto batches = [&](auto staged_c) {
-                constexpr bool kStaged = decltype(staged_c)::value;
-                for (int s0 = w.split; w.ntiles > 0 && s0 < nsteps; s0 += w.nsplit * kBatchSteps) {
-                    F av[kBatchSteps];
-                    const F *bp[kBatchSteps];
-                    bool pubr[kBatchSteps];
+                // T tiles a batch. Every load is unconditional, of an address
+                // clamped into the task's range, and what lies outside is made
+                // zero afterwards, in the batches that need it: loads under
+                // conditions were a block and a wait each. M_B is loaded one
+                // batch ahead; y and z are not (a row of z read too early is
+                // waited for twice). Measured against a load and a test per
+                // entry (backward pass): 48^3 grid, k = 32, FP32 192 -> 163 us;
+                // icosphere(6), k = 128, FP32 97 -> 88 us; 64 grid systems,
+                // k = 1 to 128, FP32 82 -> 62 us; 33^3 grid, k = 5, FP64
+                // 49 -> 46 us; 511 x 389 grid, k = 17, FP64 the same. (The
+                // same change made the forward pass 2 to 15 % slower, whose
+                // B waits on the block's own gather tasks: it keeps them.)
+                // In two copies: R-row indices from LDS (staged) or from global
+                // memory. One copy choosing per row would join an LDS and a
+                // global load into one register, and the wait for it would
+                // drain every M load in flight.
+                auto batches = [&](auto staged_c, auto tiles) {
+                    constexpr bool kStaged = decltype(staged_c)::value;
+                    constexpr int T = decltype(tiles)::value;
+                    U av[2][kBatchSteps], bu[kBatchSteps][T];
+                    int tc[T];
 #pragma unroll
-                    for (int q = 0; q < kBatchSteps; ++q) {
-                        const int s = s0 + q * w.nsplit;
-                        const int rho = hs + 4 * s + kk;
-                        av[q] = (s < nsteps && c < last && rho < he && rho >= c) ? M[bwd_off32(m, rho, c)] : F(0);
-                        pubr[q] = rho >= m;
-                        bp[q] = nullptr;
-                        if (s < nsteps && rho < he)
-                            bp[q] = (rho < m ? yv + (long long)(a0 + rho) * k
-                                             : zv + (long long)(kStaged ? lds_int(srl, rho - rb0) : a.rlist[r0 + rho - m]) * k) +
-                                    toff;
-                    }
-                    U bu[kBatchSteps][kBatchTiles];
+                    for (int jj = 0; jj < T; ++jj) tc[jj] = min(toff + 16 * (tb + jj) * w.tstride, k - 1);
+                    // Row rho < he of v.
+                    auto vrow = [&](int rho) {
+                        const int i = max(rho, rb0) - rb0;   // (below rb0: not used)
+                        const int zr = kStaged ? lds_int(srl, i) : a.rlist[r0 + rb0 - m + i];
+                        return (rho < m ? yv : zv) + (long long)(rho < m ? a0 + rho : zr) * k;
+                    };
+                    auto rho_of = [&](int s0, int q) { return min(hs + 4 * (s0 + q * w.nsplit) + kk, he - 1); };
+                    auto load_m = [&](int d, int s0) {
 #pragma unroll
-                    for (int q = 0; q < kBatchSteps; ++q)
+                        for (int q = 0; q < kBatchSteps; ++q)
+                            av[d][q] = as_bits(M[(unsigned)bwd_off32(m, rho_of(s0, q), cc0)]);
+                    };
+                    auto load_b = [&](int s0) {
 #pragma unroll
-                        for (int jj = 0; jj < kBatchTiles; ++jj) {
-                            const int j = tb + jj;
-                            const int t = toff + 16 * j * w.tstride;
-                            const bool ok = j < w.ntiles && bp[q] && t < k;
-                            // y rows never hold the sentinel: one load form for both.
-                            bu[q][jj] = !ok ? U(0) : peek_bits(bp[q] + 16 * j * w.tstride);
+                        for (int q = 0; q < kBatchSteps; ++q) {
+                            const F *v = vrow(rho_of(s0, q));
+                            // (y rows never hold the sentinel: one load form for both.)
+#pragma unroll
+                            for (int jj = 0; jj < T; ++jj) bu[q][jj] = peek_bits(v + tc[jj]);
                         }
+                    };
+                    auto use = [&](int d, int s0) {
+                        // (The step made opaque: the addresses are computed again, not kept.)
+                        int s1 = s0;
+                        asm volatile("" : "+v"(s1));
+                        settle<F>(bu, a.status, a.qa, [&](int q, int jj) { return vrow(rho_of(s1, q)) + tc[jj]; });
+                        // (A's zeros above the diagonal, and both past the end.)
+                        if (hs + 4 * s0 < cg0 + 15 || hs + 4 * (s0 + (kBatchSteps - 1) * w.nsplit) + 3 >= he)
 #pragma unroll
-                    for (int q = 0; q < kBatchSteps; ++q) {
-                        const int s = s0 + q * w.nsplit;
-                        if (s < nsteps) {
+                            for (int q = 0; q < kBatchSteps; ++q) {
+                                const int rho = hs + 4 * (s0 + q * w.nsplit) + kk;
+                                if (rho < c || rho >= he) av[d][q] = 0;
 #pragma unroll
-                            for (int jj = 0; jj < kBatchTiles; ++jj) {
-                                const int j = tb + jj;
-                                if (j < w.ntiles) {
-                                    const F b = pubr[q] && bp[q]
-                                                    ? ready_value(bp[q] + 16 * j * w.tstride, bu[q][jj], a.status, a.qa)
-                                                    : from_bits<F>(bu[q][jj]);
-                                    acc[jj] = Mfma<F>::step(av[q], b, acc[jj]);
-                                }
+                                for (int jj = 0; jj < T; ++jj)
+                                    if (rho >= he) bu[q][jj] = 0;
                             }
-                        }
+#pragma unroll
+                        for (int q = 0; q < kBatchSteps; ++q)
+#pragma unroll
+                            for (int jj = 0; jj < T; ++jj)
+                                acc[jj] = Mfma<F>::step(from_bits<F>(av[d][q]), from_bits<F>(bu[q][jj]), acc[jj]);
+                    };
+                    const int ahead = w.nsplit * kBatchSteps;
+                    if (w.split < nsteps) load_m(0, w.split);
+                    for (int s0 = w.split; s0 < nsteps; s0 += 2 * ahead) {
+                        load_b(s0);
+                        if (s0 + ahead < nsteps) load_m(1, s0 + ahead);
+                        use(0, s0);
+                        if (s0 + ahead >= nsteps) break;
+                        load_b(s0 + ahead);
+                        if (s0 + 2 * ahead < nsteps) load_m(0, s0 + 2 * ahead);
+                        use(1, s0 + ahead);
                     }
-                }
                 };
-                if (staged)
-                    batches(std::true_type{});
+                if (!staged)   // (a second tile past the last computes its last column, unused)
+                    batches(std::false_type{}, std::integral_constant<int, 2>{});
+                else if (w.ntiles - tb >= 2)
+                    batches(std::true_type{}, std::integral_constant<int, 2>{});
                 else
-                    batches(std::false_type{});
+                    batches(std::true_type{}, std::integral_constant<int, 1>{});
                 if (w.nsplit > 1) {
                     __syncthreads();   // the staged R-row indices are no longer read
                     reduce_splits(vs, w, wave, lane, acc);
