@@ -381,15 +381,6 @@ __device__ __forceinline__ void reduce_splits(F *red, const WaveWork &w, int wav
         }
 }
 
-// p[i], or zero without a branch: a load under a condition splits the unrolled
-// batches into blocks, and the loads of a batch then spill registers (up to
-// 161 in the leaf tasks below). p itself has to be readable.
-template <typename F>
-__device__ __forceinline__ typename Bits<F>::U load_or_zero(const F *p, int i, bool ok) {
-    const typename Bits<F>::U v = peek_bits(p + (ok ? i : 0));
-    return ok ? v : 0;
-}
-
 // Waits for the B operands u of a batch that still hold the sentinel; at(q, j)
 // is the address of entry q, j. One test a batch: a test per entry made every
 // MFMA step a block of its own, with a full wait in front of it. (Entries are
@@ -421,13 +412,20 @@ __device__ __forceinline__ void settle(typename Bits<F>::U (&u)[S][T], int *stat
 // 320 -> 264 us, 48^3 grid, k = 32, FP32 450 -> 416 us, 64 grid systems,
 // k 1-128, FP32 1013 -> 670 us (in a launch of their own: trsv_blocks.hip).
 constexpr int kLeafTiles = 2;
+// Steps of 4 rows loaded together; two such rounds are in flight, their loads
+// without conditions (clamped, made zero when used). Rounds of 4 steps one at
+// a time, loads zeroed by a condition each: 64 grid systems, k = 1 to 128, FP32
+// 618 us against 595; 511 x 389 grid, k = 17, FP64 239 against 234; 48^3
+// grid, k = 32, FP32 383 against 380. (Two rounds of 3 or 4 take a wave's
+// registers: 601 to 605.)
+constexpr int kLeafFly = 2;
 
 // Forward unit: the right-hand sides from column t0.
 template <typename F>
 __device__ __forceinline__ void leaf_forward_unit(const BlockPassArgs<F> &a, const Task &task, const VecMap &vm, int t0) {
     using Acc = typename Mfma<F>::Acc;
     using U = typename Bits<F>::U;
-    constexpr int kFly = 4, kGroups = 4, NT = kLeafTiles;
+    constexpr int kFly = kLeafFly, kGroups = 4, NT = kLeafTiles;
     const int lane = threadIdx.x % kWave, q = lane / 16, l = lane % 16;
     const int first = task.first, last = task.last, a0 = task.a0, m = task.m, k = vm.k;
     const int rows = m + task.R;
@@ -443,29 +441,47 @@ __device__ __forceinline__ void leaf_forward_unit(const BlockPassArgs<F> &a, con
     for (int g = 0; g < kGroups; ++g)
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[g][n] = Acc{};
-#pragma unroll 1
-    for (int s0 = 0; s0 < nsteps; s0 += kFly) {
-        U av[kFly][kGroups], bb[kFly][NT];
+    int rowc[kGroups], tc[NT];   // rows and right-hand sides that exist: what those past the end compute is not stored
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) rowc[g] = min(first + 16 * g + l, last - 1);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) tc[n] = min(t0 + 16 * n + l, k - 1);
+    U av[2][kFly][kGroups], bb[2][kFly][NT];
+    auto load = [&](int d, int s0) {
+#pragma unroll
+        for (int u = 0; u < kFly; ++u) {
+            const int col = min(4 * (s0 + u) + q, m - 1);
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) av[d][u][g] = as_bits(M[(unsigned)fwd_off32(rows, col, rowc[g])]);
+            const F *brow = bv + (long long)__shfl(pr, col, kWave) * k;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) bb[d][u][n] = as_bits(brow[tc[n]]);
+        }
+    };
+    auto use = [&](int d, int s0) {
 #pragma unroll
         for (int u = 0; u < kFly; ++u) {
             const int col = 4 * (s0 + u) + q;
+            F b[NT];
 #pragma unroll
-            for (int g = 0; g < kGroups; ++g) {
-                const int row = first + 16 * g + l;
-                av[u][g] = load_or_zero(M, fwd_off32(rows, col, row), row < last && col < m && col <= row);
-            }
-            const F *brow = bv + (long long)__shfl(pr, min(col, kLeafMaxM - 1), kWave) * k;
-#pragma unroll
-            for (int n = 0; n < NT; ++n) bb[u][n] = load_or_zero(brow, t0 + 16 * n + l, col < m && t0 + 16 * n + l < k);
-        }
-#pragma unroll
-        for (int u = 0; u < kFly; ++u)
+            for (int n = 0; n < NT; ++n) b[n] = col < m ? from_bits<F>(bb[d][u][n]) : F(0);
 #pragma unroll
             for (int g = 0; g < kGroups; ++g)
-                if (g < groups)
+                if (g < groups) {
+                    const F x = col < m && col <= rowc[g] ? from_bits<F>(av[d][u][g]) : F(0);
 #pragma unroll
-                    for (int n = 0; n < NT; ++n)
-                        acc[g][n] = Mfma<F>::step(from_bits<F>(av[u][g]), from_bits<F>(bb[u][n]), acc[g][n]);
+                    for (int n = 0; n < NT; ++n) acc[g][n] = Mfma<F>::step(x, b[n], acc[g][n]);
+                }
+        }
+    };
+    load(0, 0);
+#pragma unroll 1
+    for (int s0 = 0; s0 < nsteps; s0 += 2 * kFly) {
+        if (s0 + kFly < nsteps) load(1, s0 + kFly);
+        use(0, s0);
+        if (s0 + kFly >= nsteps) break;
+        if (s0 + 2 * kFly < nsteps) load(0, s0 + 2 * kFly);
+        use(1, s0 + kFly);
     }
 #pragma unroll
     for (int g = 0; g < kGroups; ++g)
@@ -490,7 +506,7 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
                                                    int *rowidx) {
     using Acc = typename Mfma<F>::Acc;
     using U = typename Bits<F>::U;
-    constexpr int kFly = 4, kGroups = 2, NT = kLeafTiles;
+    constexpr int kFly = kLeafFly, kGroups = 2, NT = kLeafTiles;
     const int lane = threadIdx.x % kWave, q = lane / 16, l = lane % 16;
     const int first = task.first, last = task.last, a0 = task.a0, m = task.m, r0 = task.r0, R = task.R, k = vm.k;
     const int rows = m + R;
@@ -509,39 +525,59 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
     for (int g = 0; g < kGroups; ++g)
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[g][n] = odd[g][n] = Acc{};
-#pragma unroll 1
-    for (int s0 = 0; s0 < nsteps; s0 += kFly) {
-        U av[kFly][kGroups], bb[kFly][NT];
-        const F *src[kFly];
+    int cc[kGroups], tc[NT];   // columns and right-hand sides that exist, as above
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) cc[g] = min(first + 16 * g + l, last - 1);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) tc[n] = min(t0 + 16 * n + l, k - 1);
+    U av[2][kFly][kGroups], bb[2][kFly][NT];
+    auto vrow = [&](int rho) {
+        const int zr = lds_int(rowidx, max(rho - m, 0));   // (y rows: not used)
+        return rho < m ? yv + (long long)(a0 + rho) * k : zv + (long long)zr * k;
+    };
+    auto load = [&](int d, int s0) {
+#pragma unroll
+        for (int u = 0; u < kFly; ++u) {
+            const int rho = min(first + 4 * (s0 + u) + q, rows - 1);
+#pragma unroll
+            for (int g = 0; g < kGroups; ++g) av[d][u][g] = as_bits(M[(unsigned)bwd_off32(m, rho, cc[g])]);
+            const F *src = vrow(rho);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) bb[d][u][n] = peek_bits(src + tc[n]);
+        }
+    };
+    auto use = [&](int d, int s0) {
+        int s1 = s0;
+        asm volatile("" : "+v"(s1));   // addresses computed again, not kept
+        // (y rows never hold the sentinel.)
+        settle<F>(bb[d], a.status, a.qa,
+                  [&](int u, int n) { return vrow(min(first + 4 * (s1 + u) + q, rows - 1)) + tc[n]; });
 #pragma unroll
         for (int u = 0; u < kFly; ++u) {
             const int rho = first + 4 * (s0 + u) + q;
-#pragma unroll
-            for (int g = 0; g < kGroups; ++g) {
-                const int c = first + 16 * g + l;
-                av[u][g] = load_or_zero(M, bwd_off32(m, rho, c), c < last && rho < rows && rho >= c);
-            }
-            // (Rows past the end read row a0 of y and drop it.)
-            const int zr = lds_int(rowidx, min(max(rho - m, 0), kLeafMaxRows - 1));
-            src[u] = rho < m || rho >= rows ? yv + (long long)(a0 + (rho < m ? rho : 0)) * k : zv + (long long)zr * k;
-#pragma unroll
-            for (int n = 0; n < NT; ++n) bb[u][n] = load_or_zero(src[u], t0 + 16 * n + l, rho < rows && t0 + 16 * n + l < k);
-        }
-#pragma unroll
-        for (int u = 0; u < kFly; ++u) {
-            // (y rows never hold the sentinel, nor do entries read as zero.)
             F b[NT];
 #pragma unroll
-            for (int n = 0; n < NT; ++n) b[n] = ready_value(src[u] + t0 + 16 * n + l, bb[u][n], a.status, a.qa);
+            for (int n = 0; n < NT; ++n) b[n] = rho < rows ? from_bits<F>(bb[d][u][n]) : F(0);
 #pragma unroll
             for (int g = 0; g < kGroups; ++g)
-                if (g < groups)
+                if (g < groups) {
+                    const F x = rho < rows && rho >= first + 16 * g + l ? from_bits<F>(av[d][u][g]) : F(0);
 #pragma unroll
                     for (int n = 0; n < NT; ++n) {
                         Acc &sum = sizeof(F) == 4 && u % 2 ? odd[g][n] : acc[g][n];
-                        sum = Mfma<F>::step(from_bits<F>(av[u][g]), b[n], sum);
+                        sum = Mfma<F>::step(x, b[n], sum);
                     }
+                }
         }
+    };
+    load(0, 0);
+#pragma unroll 1
+    for (int s0 = 0; s0 < nsteps; s0 += 2 * kFly) {
+        if (s0 + kFly < nsteps) load(1, s0 + kFly);
+        use(0, s0);
+        if (s0 + kFly >= nsteps) break;
+        if (s0 + 2 * kFly < nsteps) load(0, s0 + 2 * kFly);
+        use(1, s0 + kFly);
     }
 #pragma unroll
     for (int g = 0; g < kGroups; ++g)
