@@ -76,9 +76,9 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // acc[t] += sum over j < n of mv[j] * r[j * KT + t] (n >= 1, r in LDS), in the
-// order of j. The rows are read four (FP64: two) at a time without a condition (a row past
-// the end is the last one, its values replaced by zeros): a condition per row
-// made each read wait for the one before. With the sums below one a thread
+// order of j. The rows are read four (FP64: two) at a time without a condition
+// (a row past the end is the last one, its values replaced by zeros): a
+// condition per row made each read wait for the one before. With the sums below one a thread
 // (one thread summed all right-hand sides of a row, up to 60 reads in a row):
 // icosphere(7), k = 3, FP32 148 -> 136 us, FP64 169 -> 159 us; icosphere(6)
 // FP32 82 -> 75 us; 501 x 300 grid, k = 4, FP32 131 -> 115 us.
@@ -115,7 +115,13 @@ __device__ __forceinline__ F sum_segments(const F *v, int i, int width, int segs
 }
 
 // Forward leaf task tk of the records `tasks` (r: kLeafMaxM x KT of this
-// wavefront's LDS).
+// wavefront's LDS). A leaf task is a chain of memory latencies (record, row
+// index, b or z, up to four rounds of M_B), so its loads carry no conditions
+// (addresses clamped into the block, what lies outside multiplied by zeros) and
+// M_B is loaded a round ahead. Measured, loads under conditions and one round
+// at a time against this, both directions: icosphere(5), k = 3, FP32 44 -> 38
+// us a solve, icosphere(6) 75 -> 68, icosphere(7) FP32 136 -> 128, FP64 159 ->
+// 155 us, 501 x 300 grid, k = 4, FP32 115 -> 107 us.
 template <typename F, int KT>
 __device__ __forceinline__ void leaf_forward_task(const BlockPassArgs<F> &a, const int *tasks,
                                                   unsigned long long *trace, int tk, F *r) {
@@ -130,40 +136,37 @@ __device__ __forceinline__ void leaf_forward_task(const BlockPassArgs<F> &a, con
     // Lane = row rho of M_B; row rho uses columns [0, cend).
     const int rho = first + lane;
     const int cend = rho < last ? min(rho + 1, m) : 0;
-    F mv[kLeafMU];
-    int64_t o = fwd_off(rows, 0, rho);
+    // Loads clamped into the row, two rounds of kLeafMU columns in flight.
+    const int rc = min(rho, last - 1), cl = min(rc + 1, m) - 1;
+    F mv[2][kLeafMU];
+    auto load = [&](int d, int c) {
 #pragma unroll
-    for (int j = 0; j < kLeafMU; ++j) {
-        mv[j] = j < cend ? M[o] : F(0);
-        o += rows - j - 1;
-    }
+        for (int j = 0; j < kLeafMU; ++j) {
+            const int cc = min(c + j, cl);
+            mv[d][j] = M[(unsigned)(cc * rows - cc * (cc - 1) / 2 + rc - cc)];
+        }
+    };
+    load(0, 0);
     // r_B = (P b)_B, rows [0, m).
-    if (lane < m) {
+    if (lane < m && k > 0) {
         const long long pr = vm.vbase + (long long)a.perm[a0 + lane] * k;
 #pragma unroll
-        for (int t = 0; t < KT; ++t) r[lane * KT + t] = t < k ? a.b[pr + t] : F(0);
+        for (int t = 0; t < KT; ++t) {
+            const F x = a.b[pr + min(t, k - 1)];
+            r[lane * KT + t] = t < k ? x : F(0);
+        }
     }
     wave_sync();
     if (trace && lane == 0) trace[4 * (size_t)tk + 1] = wall_clock64();
     F acc[KT];
 #pragma unroll
     for (int t = 0; t < KT; ++t) acc[t] = F(0);
-    for (int c = 0;;) {
-#pragma unroll
-        for (int j = 0; j < kLeafMU; ++j) {
-            if (c + j < cend) {
-                const F *rr = r + (c + j) * KT;
-#pragma unroll
-                for (int t = 0; t < KT; ++t) acc[t] = fma(mv[j], rr[t], acc[t]);
-            }
-        }
-        c += kLeafMU;
-        if (c >= cend) break;
-#pragma unroll
-        for (int j = 0; j < kLeafMU; ++j) {
-            mv[j] = c + j < cend ? M[o] : F(0);
-            o += rows - (c + j) - 1;
-        }
+    const int cmax = min(last, m);   // columns of the task's last row
+    for (int c = 0; c < cmax; c += 2 * kLeafMU) {
+        if (c + kLeafMU < cmax) load(1, c + kLeafMU);
+        if (c < cend) add_rows(acc, mv[0], r + c * KT, cend - c);
+        if (c + 2 * kLeafMU < cmax) load(0, c + 2 * kLeafMU);
+        if (c + kLeafMU < cend) add_rows(acc, mv[1], r + (c + kLeafMU) * KT, cend - c - kLeafMU);
     }
     if (rho < last) {
         F *yv = a.y + vm.vbase, *zv = a.z + vm.vbase, *pv = a.part + vm.pbase;
@@ -208,12 +211,17 @@ __device__ __forceinline__ void leaf_backward_task(const BlockPassArgs<F> &a, co
     // consecutive entries of the row-major packed M_B across the lanes).
     const int c = first + (lane & 31), h = lane >> 5;
     const bool active = c < last;
-    F mv[kLeafMUB];
+    // Loads clamped into the column, two rounds of kLeafMUB rows in flight.
+    const int cc = min(c, last - 1);
+    F mv[2][kLeafMUB];
+    auto load = [&](int d, int j0) {
 #pragma unroll
-    for (int j = 0; j < kLeafMUB; ++j) {
-        const int rr = first + h + 2 * j;
-        mv[j] = active && rr >= c && rr < rows ? M[bwd_off(m, rr, c)] : F(0);
-    }
+        for (int j = 0; j < kLeafMUB; ++j) {
+            const int rr = min(max(first + h + 2 * (j0 + j), cc), rows - 1);
+            mv[d][j] = M[(unsigned)(rr < m ? rr * (rr + 1) / 2 + cc : m * (m + 1) / 2 + (rr - m) * m + cc)];
+        }
+    };
+    load(0, 0);
     // v = [y_B ; z_R], rows [first, rows): y from the forward pass, z_R from
     // the backward block tasks.
     for (int i = first + lane; i < rows; i += kWave) {
@@ -236,22 +244,31 @@ __device__ __forceinline__ void leaf_backward_task(const BlockPassArgs<F> &a, co
     F acc[KT];
 #pragma unroll
     for (int t = 0; t < KT; ++t) acc[t] = F(0);
-    for (int j0 = 0;; j0 += kLeafMUB) {
+    auto add = [&](int d, int j0) {
+        constexpr int kG = 16 / (int)sizeof(F);   // rows read together (add_rows)
 #pragma unroll
-        for (int j = 0; j < kLeafMUB; ++j) {
-            const int rr = first + h + 2 * (j0 + j);
-            if (active && rr >= c && rr < rows) {
-                const F *vv = v + (rr - first) * KT;
+        for (int g = 0; g < kLeafMUB; g += kG) {
+            const int r0g = first + h + 2 * (j0 + g);
+            if (r0g >= rows || r0g + 2 * (kG - 1) < cc) continue;
+            F x[kG][KT];
 #pragma unroll
-                for (int t = 0; t < KT; ++t) acc[t] = fma(mv[j], vv[t], acc[t]);
+            for (int j = 0; j < kG; ++j)
+#pragma unroll
+                for (int t = 0; t < KT; ++t) x[j][t] = v[(min(r0g + 2 * j, rows - 1) - first) * KT + t];
+#pragma unroll
+            for (int j = 0; j < kG; ++j) {
+                const int rr = r0g + 2 * j;
+#pragma unroll
+                for (int t = 0; t < KT; ++t) acc[t] = fma(mv[d][g + j], rr >= cc && rr < rows ? x[j][t] : F(0), acc[t]);
             }
         }
-        if (first + h + 2 * (j0 + kLeafMUB) >= rows) break;
-#pragma unroll
-        for (int j = 0; j < kLeafMUB; ++j) {
-            const int rr = first + h + 2 * (j0 + kLeafMUB + j);
-            mv[j] = active && rr >= c && rr < rows ? M[bwd_off(m, rr, c)] : F(0);
-        }
+    };
+    const int nj = (rows - first + 1) / 2;
+    for (int j0 = 0; j0 < nj; j0 += 2 * kLeafMUB) {
+        if (j0 + kLeafMUB < nj) load(1, j0 + kLeafMUB);
+        add(0, j0);
+        if (j0 + 2 * kLeafMUB < nj) load(0, j0 + 2 * kLeafMUB);
+        if (j0 + kLeafMUB < nj) add(1, j0 + kLeafMUB);
     }
 #pragma unroll
     for (int t = 0; t < KT; ++t) acc[t] += __shfl_xor(acc[t], 32, kWave);
