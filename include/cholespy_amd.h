@@ -269,17 +269,20 @@ int cholespy_probe_handoff(double *results, int count);
 int cholespy_solver_tune_report(const cholespy_gpu_solver *solver, char *report, size_t report_len);
 
 /* Block-plan statistics: info[0..count) = {blocks, dense entries of all
- * M_B, forward block levels, backward block levels, forward tasks, backward
- * tasks, partial slots, largest m + |R|, forward tasks and backward tasks of
- * the wide right-hand-side list}. No counterpart in the reference. */
+ * M_B (of a dense top, whose square inverse serves both passes, half),
+ * forward block levels, backward block levels, forward tasks, backward tasks,
+ * partial slots, largest m + |R|, forward tasks and backward tasks of the
+ * wide right-hand-side list}. No counterpart in the reference. */
 int cholespy_solver_plan_info(const cholespy_gpu_solver *solver, int64_t *info, int count);
 
 /* Copies of the block plan (diagnostics; no counterpart in the reference):
  * which = 0 block row starts (blocks + 1), 1 partial-slot ranges
  * (blocks + 1), 2 forward block levels (blocks), 3 backward block levels
  * (blocks), 4 forward tasks and 5 backward tasks (CHOLESPY_TASK_INTS ints
- * each: block, first, last, kind, lo, hi, split-row base, splits), 6 and 7
- * the forward and backward tasks of the wide right-hand-side list. Copies
+ * each: block, first, last, kind, lo, hi, split-row base, splits; forward
+ * kinds 0 gather and product, 1 gather, 2 product, 3 split product, 4 gather
+ * of a dense top; backward 0 product, 1 split product), 6 and 7 the forward
+ * and backward tasks of the wide right-hand-side list. Copies
  * min(count, size) ints to out; *size (if not null) receives the full size. */
 #define CHOLESPY_TASK_INTS 8
 int cholespy_solver_plan_arrays(const cholespy_gpu_solver *solver, int which, int32_t *out, int64_t count,
