@@ -56,9 +56,10 @@ template <> struct Mfma<double> {
 
 // Kernels are instantiated for NT = 2, 4 or 8 tiles of 16 right-hand sides
 // (the launch picks the smallest that holds the largest k), so small k keeps
-// few accumulators and loads more steps ahead: kSteps(NT) MFMA steps have
-// their A (and B) loads issued together.
-template <int NT> constexpr int kStepsFor() { return NT <= 2 ? 8 : 4; }
+// few accumulators. Small blocks forward issue kSteps MFMA steps' A loads
+// together (4 at 2 tiles instead of 8: forward pass of icosphere(6), k = 8,
+// FP32 48.2 -> 47.3 us, of a 400 x 300 grid, k = 32, 87.3 -> 86.2).
+constexpr int kSteps = 4;
 // Tasks whose B comes straight from global memory (large blocks forward,
 // every backward task) run a wavefront's tiles in batches of kBatchTiles,
 // each batch with kBatchSteps MFMA steps' A and B loads issued together:
@@ -69,11 +70,13 @@ template <int NT> constexpr int kStepsFor() { return NT <= 2 ? 8 : 4; }
 constexpr int kBatchTiles = 2;
 // FP32: 8 steps (forward 12 for the 8-tile kernels, whose occupancy floors
 // leave room); FP64: 4 (more cost the forward kernels a wave per SIMD). The
-// backward kernels hold M_B of two batches and take what fits without spills
-// (FP64: 3; 4 measured 2 % slower on the 511 x 389 grid at k = 17).
+// backward kernels hold M_B of two batches: FP32 6 steps (8 at 2 tiles:
+// icosphere(6), k = 8, 80 us a solve against 78, a 400 x 300 grid, k = 32, 152
+// against 148; 3 or 4 lose on the 48^3 grid), FP64 3 (4 measured 2 % slower
+// on the 511 x 389 grid at k = 17).
 template <typename F, int NT, bool Forward> constexpr int batch_steps() {
     if (Forward) return sizeof(F) == 4 ? (NT >= 8 ? 12 : 8) : (NT <= 2 ? 8 : 4);
-    return sizeof(F) == 4 ? (NT == 4 ? 6 : 8) : (NT <= 4 ? 3 : 4);
+    return sizeof(F) == 4 ? 6 : (NT <= 4 ? 3 : 4);
 }
 // Waves per SIMD the compiler must allow (amdgpu_waves_per_eu), chosen per
 // kernel as the most that compile with no register spills on gfx950. By
@@ -639,7 +642,6 @@ __global__ __launch_bounds__(kTaskThreads) __attribute__((amdgpu_waves_per_eu(kM
 void block_forward_panel(BlockPassArgs<F> a) {
     using Acc = typename Mfma<F>::Acc;
     constexpr int kMaxTiles = NT;
-    constexpr int kSteps = kStepsFor<NT>();
     constexpr int kBatchSteps = batch_steps<F, NT, true>();
     extern __shared__ __align__(16) unsigned char smem[];
     F *rv = reinterpret_cast<F *>(smem);
@@ -830,7 +832,6 @@ __global__ __launch_bounds__(kTaskThreads) __attribute__((amdgpu_waves_per_eu(kM
 void block_backward_panel(BlockPassArgs<F> a) {
     using Acc = typename Mfma<F>::Acc;
     constexpr int kMaxTiles = NT;
-    constexpr int kSteps = kStepsFor<NT>();
     constexpr int kBatchSteps = batch_steps<F, NT, false>();
     extern __shared__ __align__(16) unsigned char smem[];
     F *vs = reinterpret_cast<F *>(smem);
