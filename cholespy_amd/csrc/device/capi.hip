@@ -1044,8 +1044,8 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         if (is_panel_tile(tile)) {
             bf.ntasks = forward ? d.n_fwd_tasks_wide : d.n_bwd_tasks_wide;
             // Leaf units carry two tiles of 16 right-hand sides: for one tile
-            // the workgroups' own tasks stay (33^3 grid, k = 5, FP64: 175 us,
-            // 192 with units).
+            // the workgroups' own tasks stay (33^3 grid, k = 5, FP64: 139 us,
+            // 148 with units; icosphere(6), k = 8, FP32 80 and 90).
             const bool units = s->leaf_kernels && bf.max_k > 16;
             bf.n_leaf = units ? (forward ? d.n_leaf_fwd_wide : d.n_leaf_bwd_wide) : 0;
             bf.task = forward ? d.ftask_wide : d.btask_wide;

@@ -6,17 +6,19 @@
 // their levels costs three hand-offs between workgroups in the forward pass
 // and two in the backward one (7 us a level and pass, whatever its size),
 // while the inverse of the rows above a cut streams at memory bandwidth. A
-// small system is one product. Measured, block passes alone and with this
-// (k = 3): icosphere(3), n = 642, FP32 52.9 -> 6.5 us; a 61 x 47 grid, FP64
-// 60.4 -> 13.4 us (its 66 MB inverse at 5 TB/s); icosphere(5), FP32, a top of
-// 2,640 rows 91.9 -> 45.6 us; icosphere(6), k = 128, FP32, a top of 3,488 rows
-// 371 -> 242 us. choose_dense_top (block_plan.cpp) weighs the two.
+// small system is one product. Measured, block passes alone and with this:
+// k = 3, icosphere(3), n = 642, FP32 41.9 -> 6.9 us; icosphere(5), FP32, a top
+// of 2,640 rows 66 -> 39 us; a vector, 61 x 47 grid, FP64 50.7 -> 13.4 us (its
+// 66 MB inverse at 5 TB/s); k = 128, icosphere(6), FP32, 3,488 rows 342 -> 225
+// us; k = 32, 48^3 grid, FP32, 6,256 rows 460 -> 382 us; k = 3, icosphere(7),
+// FP64, 2,896 rows 163 -> 160 us.
+// choose_dense_top (block_plan.cpp) weighs the two.
 //
 // Rounding: an inverse rounded to FP32 keeps the block passes' accuracy only
 // if its long dot products do not round in FP32 as well (one running FP32 sum
 // lost a factor of 3 to 4): products are summed a few at a time, and those
 // sums in FP64. FP32 solves are then 1.1 to 3 times closer to the exact
-// solution than the block passes' were, FP64 ones within 15 % of them.
+// solution than the block passes' were, FP64 ones within 20 % of them.
 //
 // Layout: S^{-1} (symmetric) in panels of 16 output rows, each contiguous:
 // the entry of output c and input rho is element
