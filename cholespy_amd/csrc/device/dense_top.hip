@@ -240,7 +240,9 @@ __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top
     Vec m[D];
     // B of tile n, lane column l: right-hand side col0 + n, so that a lane's
     // tiles are one load of NT consecutive values. Lanes past the row's end
-    // compute (and store) its last NT columns again. (NT > 1: k > 16.)
+    // compute its last NT columns again and store only those from their own
+    // first column on: a column stored twice, by lanes that reach it with
+    // different n, would take a refinement's += twice. (NT > 1: k > 16.)
     const int col0 = NT == 1 ? t0 + l : min(t0 + NT * l, k - NT);
     const unsigned b0 = NT > 1 || col0 < k ? (unsigned)(q * k + col0) * (unsigned)sizeof(F) : 1u << 31;
     F b[D][V][NT];
@@ -312,7 +314,7 @@ __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top
         double s = 0.0;
 #pragma unroll
         for (int w = 0; w < kHalf; ++w) s += red[w * NT + n][e];
-        if (c < top.n && col < k) put(a, top, c, col, a.perm ? a.perm[top.row0 + c] : top.row0 + c, (F)s);
+        if (c < top.n && col < k && col >= t0 + NT * l) put(a, top, c, col, a.perm ? a.perm[top.row0 + c] : top.row0 + c, (F)s);
     }
 }
 
