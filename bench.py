@@ -315,8 +315,8 @@ def main():
     else:
         pass_kernels = ["leaf_forward" + tname, "block_forward" + tname] if dom == 0 else \
                        ["block_backward" + tname, "leaf_backward" + tname]
-    if dom == 1 and (solver._plan_arrays()["fwd_task"][:, 3] == 4).any():   # a dense top: its product comes first
-        pass_kernels.insert(0, "dense_narrow" + tname)
+    if (solver._plan_arrays()["fwd_task"][:, 3] == 4).any():   # a dense top: X r ends the forward pass, X'y starts the backward
+        pass_kernels.insert(len(pass_kernels) if dom == 0 else 0, "dense_narrow" + tname[:-1] + (",0>" if dom == 0 else ",1>"))
     kernel = ("forward" if dom == 0 else "backward") + " pass: " + " + ".join(pass_kernels)
     workload_name = f"mesh smoothing I+10(D-W) on icosphere({args.level})"
     traffic = measured_traffic(pass_kernels, workload_name, k)

@@ -1,7 +1,7 @@
 // Dense values of the block plan (block_plan.hpp), formed on the GPU in FP64
 // from the factor L and rounded once to the solver's precision:
 //   M_B = [ L_BB^{-1} ; -L_RB L_BB^{-1} ]   per block, in both packed layouts;
-//   S^{-1} = L_TT^{-T} L_TT^{-1}            for a dense top block, full square.
+//   X = L_TT^{-1}                           for a dense top block, in the panels of dense_top.hip.
 //
 // Blocks of up to 64 rows (nearly all of them) take one workgroup each, all
 // in LDS: scatter L_BB, invert it column per thread, then multiply L_RB by
@@ -10,7 +10,8 @@
 //   X_21 = -X_22 (L_21 X_11),
 // two tile products per doubling for all blocks at once (gemm_tiles, FP64
 // MFMA, zero parts of triangular operands skipped), then -L_RB X, and a pack
-// kernel that writes both layouts through LDS.
+// kernel that writes both layouts through LDS. Top blocks take the same steps
+// on the tiles that X has (dense_top_plan.hpp), in place.
 //
 // Why on the GPU: the host fill is a few GFLOP of FP64 products and the
 // writing, conversion and upload of two copies of M; here only L is uploaded
@@ -148,25 +149,130 @@ __global__ __launch_bounds__(64) void scatter_columns(InverseArgs a, const Inver
     }
 }
 
-// 64 x 64 diagonal inverses: job.C (ldc) := inverse of the M x M lower triangle job.A (lda).
-__global__ __launch_bounds__(kThreads) void diagonal_inverses(const InverseJob *jobs) {
+// total += A B of one step of kKStep in LDS, for the wavefront's 32 x 32
+// quarter at (wi, wj). Sums of kKStep products, then a sum of those: long dot
+// products round twice as badly in one running sum.
+template <int LD>
+__device__ __forceinline__ void step_products(const double (&As)[kKStep][LD], const double (&Bs)[kKStep][LD], int lane, int wi,
+                                              int wj, f64x4 (&total)[2][2]) {
+    f64x4 acc[2][2] = {};
+#pragma unroll
+    for (int kk = 0; kk < kKStep; kk += 4) {
+        const int k = kk + (lane >> 4);
+        const double a0 = As[k][wi + (lane & 15)], a1 = As[k][wi + 16 + (lane & 15)];
+        const double b0 = Bs[k][wj + (lane & 15)], b1 = Bs[k][wj + 16 + (lane & 15)];
+        acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
+        acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
+        acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
+        acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) total[x][y] += acc[x][y];
+}
+
+// C (ldc) := inverse of the m x m lower triangle A (lda), m <= kSmall, by one
+// workgroup; C may be A.
+__device__ __forceinline__ void invert_tile(const double *A, int64_t lda, double *C, int64_t ldc, int m) {
     __shared__ double L[kSmall * kLd], X[kSmall * kLd];
-    const InverseJob job = jobs[blockIdx.x];
-    const int m = job.M;
     for (int i = threadIdx.x; i < m * kSmall; i += kThreads) {
         const int r = i % kSmall, c = i / kSmall;
-        if (r < m) L[r * kLd + c] = r >= c ? job.A[r + c * job.lda] : 0.0;
+        if (r < m) L[r * kLd + c] = r >= c ? A[r + c * lda] : 0.0;
     }
     __syncthreads();
     if (threadIdx.x < 64) invert_lower(L, X, m);
     __syncthreads();
     for (int i = threadIdx.x; i < m * kSmall; i += kThreads) {
         const int r = i % kSmall, c = i / kSmall;
-        if (r < m && r >= c) job.C[r + c * job.ldc] = X[r * kLd + c];
+        if (r < m && r >= c) C[r + c * ldc] = X[r * kLd + c];
     }
 }
 
-// C := alpha op(A) B on 64 x 64 tiles (column-major), one workgroup per tile:
+// 64 x 64 diagonal inverses: job.C (ldc) := inverse of the M x M lower triangle job.A (lda).
+__global__ __launch_bounds__(kThreads) void diagonal_inverses(const InverseJob *jobs) {
+    const InverseJob job = jobs[blockIdx.x];
+    invert_tile(job.A, job.lda, job.C, job.ldc, job.M);
+}
+
+// Top blocks (dense_top_plan.hpp): L into their tiles (zeroed by the caller),
+// one wavefront per column; the diagonal tiles inverted in place; a stage of
+// tile products; both layouts from the finished tiles.
+__global__ __launch_bounds__(64) void top_scatter(InverseArgs a, const TopLists::Column *columns, const int *map, double *D) {
+    const TopLists::Column col = columns[blockIdx.x];
+    const int nt = map[col.map], j = a.src[col.row0 + col.c];
+    const int *tile = map + col.map + 1;
+    for (int64_t p = a.colptr[j] + threadIdx.x; p < a.colptr[j + 1]; p += 64) {
+        const int i = a.rank[a.rowidx[p]] - col.row0;
+        const int t = tile[i / kTopTile * nt + col.c / kTopTile];
+        D[(int64_t)t * kTopTileEntries + i % kTopTile + col.c % kTopTile * kTopTile] = a.val[p];
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void top_diagonals(const TopLists::Diagonal *diagonals, double *D) {
+    const TopLists::Diagonal d = diagonals[blockIdx.x];
+    double *t = D + (int64_t)d.tile * kTopTileEntries;
+    invert_tile(t, kTopTile, t, kTopTile, d.rows);
+}
+
+// Out tile := alpha times the sum of the job's tile products A B, as gemm_tiles.
+__global__ __launch_bounds__(kThreads) void top_products(const TopLists::Job *jobs, const TopLists::Pair *pairs,
+                                                         const double *A, const double *B, double *C, double alpha) {
+    constexpr int kLdA = kTopTile + 2, kSteps = kTopTile / kKStep;
+    __shared__ double As[kKStep][kLdA], Bs[kKStep][kLdA];
+    const TopLists::Job job = jobs[blockIdx.x];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, total_steps = job.count * kSteps;
+    double ra[4], rb[4];
+    auto load = [&](int s) {
+        const TopLists::Pair pr = pairs[job.first + s / kSteps];
+        const double *ta = A + (int64_t)pr.a * kTopTileEntries + s % kSteps * kKStep * kTopTile;
+        const double *tb = B + (int64_t)pr.b * kTopTileEntries + s % kSteps * kKStep;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            ra[q] = ta[lane + (wave + 4 * q) * kTopTile];
+            rb[q] = tb[tid % 16 + (tid / 16 + 16 * q) * kTopTile];
+        }
+    };
+    f64x4 total[2][2] = {};
+    const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
+    if (total_steps > 0) load(0);
+    for (int s = 0; s < total_steps; ++s) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            As[wave + 4 * q][lane] = ra[q];
+            Bs[tid % 16][tid / 16 + 16 * q] = rb[q];
+        }
+        __syncthreads();
+        if (s + 1 < total_steps) load(s + 1);
+        step_products(As, Bs, lane, wi, wj, total);
+        __syncthreads();
+    }
+    double *out = C + (int64_t)job.out * kTopTileEntries;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                out[wi + 16 * x + (lane >> 4) + 4 * v + (wj + 16 * y + (lane & 15)) * kTopTile] = alpha * total[x][y][v];
+}
+
+// One unit a workgroup: units [0, gridDim.x / 2) of X, then as many of X'.
+template <typename F>
+__global__ __launch_bounds__(kTopUnitEntries) void top_pack(const int *pack, const double *D, F *dst) {
+    constexpr int V = 16 / (int)sizeof(F), G = 4 * V;
+    const int code = pack[blockIdx.x], tid = threadIdx.x;
+    const int lane = tid % (64 * V) / V, c = lane % 16, rho = tid / (64 * V) * G + tid % V * 4 + lane / 16;
+    double v = 0.0;
+    if (code >= 0) {
+        const int i0 = code / 4 % 4 * kTopUnit, j0 = code % 4 * kTopUnit;
+        const bool fwd = blockIdx.x < gridDim.x / 2;
+        v = D[(int64_t)(code / 16) * kTopTileEntries + i0 + (fwd ? c : rho) + (j0 + (fwd ? rho : c)) * kTopTile];
+    }
+    dst[(int64_t)blockIdx.x * kTopUnitEntries + tid] = (F)v;
+}
+
+// C := alpha A B on 64 x 64 tiles (column-major), one workgroup per tile:
 // 4 wavefronts of 2 x 2 MFMA 16x16x4 tiles, K in steps of 16 through LDS,
 // the next step's entries loaded while the current one is multiplied.
 __global__ __launch_bounds__(kThreads) void gemm_tiles(const InverseJob *jobs, const InverseTile *tiles) {
@@ -178,51 +284,29 @@ __global__ __launch_bounds__(kThreads) void gemm_tiles(const InverseJob *jobs, c
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int kb = 0, ke = job.K;
     if (job.flags & kBLower) kb = j0;
-    if (job.flags & kGram) kb = max(i0, j0);
     if (job.flags & kALower) ke = min(ke, i0 + kTile);
-    const bool ta = (job.flags & kGram) != 0;
     double ra[4], rb[4];
     auto load = [&](int k0) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int ai = ta ? tid / 16 + 16 * q : lane, ak = k0 + (ta ? tid % 16 : wave + 4 * q);
-            const bool aok = i0 + ai < job.M && ak < ke;
-            ra[q] = aok ? job.A[ta ? ak + (int64_t)(i0 + ai) * job.lda : i0 + ai + (int64_t)ak * job.lda] : 0.0;
+            const int ak = k0 + wave + 4 * q;
+            ra[q] = i0 + lane < job.M && ak < ke ? job.A[i0 + lane + (int64_t)ak * job.lda] : 0.0;
             const int bj = tid / 16 + 16 * q, bk = k0 + tid % 16;
             rb[q] = j0 + bj < job.N && bk < ke ? job.B[bk + (int64_t)(j0 + bj) * job.ldb] : 0.0;
         }
     };
-    // Sums of kKStep products, then a sum of those: long dot products (the
-    // Gram product's above all) round twice as badly in one running sum, and
-    // the FP64 solve's error doubled with them (64^2 grid, k = 3: 6.8e-16
-    // against 5.1e-16, and 4.5e-16 for the block passes).
     f64x4 total[2][2] = {};
     const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
     if (kb < ke) load(kb);
     for (int k0 = kb; k0 < ke; k0 += kKStep) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            if (ta) As[tid % 16][tid / 16 + 16 * q] = ra[q];
-            else As[wave + 4 * q][lane] = ra[q];
+            As[wave + 4 * q][lane] = ra[q];
             Bs[tid % 16][tid / 16 + 16 * q] = rb[q];
         }
         __syncthreads();
         if (k0 + kKStep < ke) load(k0 + kKStep);
-        f64x4 acc[2][2] = {};
-#pragma unroll
-        for (int kk = 0; kk < kKStep; kk += 4) {
-            const int k = kk + (lane >> 4);
-            const double a0 = As[k][wi + (lane & 15)], a1 = As[k][wi + 16 + (lane & 15)];
-            const double b0 = Bs[k][wj + (lane & 15)], b1 = Bs[k][wj + 16 + (lane & 15)];
-            acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-        }
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-            for (int y = 0; y < 2; ++y) total[x][y] += acc[x][y];
+        step_products(As, Bs, lane, wi, wj, total);
         __syncthreads();
     }
     // Accumulator element v of lane l: row l / 16 + 4 v, column l % 16.
@@ -259,27 +343,6 @@ __global__ __launch_bounds__(kThreads) void pack_tiles(const InversePack *packs,
     for (int q = ly; q < 32; q += kThreads / 32) {
         const int r = tile.i0 + q, c = tile.j0 + lx;
         if (r < rows && c < m && r >= c) mbwd[pk.off + bwd_at(m, r, c)] = (F)t[lx][q];
-    }
-}
-
-// The inverse of a top block in the panel layout of dense_top.hip, from the
-// lower half of the column-major m x m Gram product. order not null: in the
-// caller's row order (caller row i is plan row order[i]).
-template <typename F>
-__global__ __launch_bounds__(kThreads) void pack_top(const double *S, int m, const int *order, F *dst) {
-    constexpr int V = 16 / (int)sizeof(F), G = 4 * V;
-    const int mp = (m + 15) / 16 * 16;
-    const int64_t total = (int64_t)mp * mp;
-    for (int64_t e = blockIdx.x * (int64_t)kThreads + threadIdx.x; e < total; e += (int64_t)gridDim.x * kThreads) {
-        const int panel = (int)(e / (16 * (int64_t)mp)), w = (int)(e % (16 * (int64_t)mp));
-        const int lane = w % (64 * V) / V;
-        const int c = panel * 16 + lane % 16, r = w / (64 * V) * G + w % V * 4 + lane / 16;
-        F v = F(0);
-        if (c < m && r < m) {
-            const int i = order ? order[c] : c, j = order ? order[r] : r;
-            v = (F)S[max(i, j) + (int64_t)min(i, j) * m];
-        }
-        dst[e] = v;
     }
 }
 
@@ -321,7 +384,7 @@ struct Arena {
 
 // The blocks `large` of P through dense work arrays.
 template <typename F>
-hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::vector<int> &large, const int *order, F *mfwd, F *mbwd, F *mtop) {
+hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::vector<int> &large, F *mfwd, F *mbwd) {
     Arena arena;
     // Work arrays: D = [L_BB ; L_RB] (rows x m), X and T (m x m), Q (R x m).
     size_t dn = 0, xn = 0, qn = 0;
@@ -347,23 +410,21 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
     struct Place {
         double *D, *X, *T, *Q;
         int m, R;
-        bool top;
     };
     std::vector<Place> at;
     {
         double *d = D, *x = X, *t = T, *q = Q;
         for (int b : large) {
             const int m = P.start[b + 1] - P.start[b], R = P.rptr[b + 1] - P.rptr[b], rows = m + R;
-            at.push_back({d, x, t, q, m, R, P.is_top(b)});
+            at.push_back({d, x, t, q, m, R});
             for (int c = 0; c < m; ++c) cols.push_back({b, c, d + (size_t)c * rows});
             for (int i = 0; i < m; i += kSmall) {
                 const int w = std::min(kSmall, m - i);
                 diag.push_back({d + i + (size_t)i * rows, nullptr, x + i + (size_t)i * m, rows, 0, m, w, w, w, 0, 1.0});
             }
             packs.push_back({x, q, P.moff[b], m, R});
-            if (!P.is_top(b))
-                for (int i = 0; i < rows; i += 32)
-                    for (int j = 0; j < m && j <= i; j += 32) ptiles.push_back({(int)packs.size() - 1, i, j});
+            for (int i = 0; i < rows; i += 32)
+                for (int j = 0; j < m && j <= i; j += 32) ptiles.push_back({(int)packs.size() - 1, i, j});
             max_m = std::max(max_m, m);
             d += (size_t)rows * m;
             x += (size_t)m * m;
@@ -374,8 +435,7 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
     auto add = [&](const InverseJob &j) {
         jobs.push_back(j);
         for (int i = 0; i < j.M; i += kTile)
-            for (int c = 0; c < j.N; c += kTile)
-                if (!(j.flags & kGram) || i >= c) tiles.push_back({(int)jobs.size() - 1, i, c});
+            for (int c = 0; c < j.N; c += kTile) tiles.push_back({(int)jobs.size() - 1, i, c});
     };
     for (int s = kSmall; s < max_m; s *= 2) {
         for (int half = 0; half < 2; ++half) {
@@ -392,11 +452,8 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
             stage.push_back(tiles.size());
         }
     }
-    for (const Place &p : at) {
-        if (p.R > 0)
-            add({p.D + p.m, p.X, p.Q, p.m + p.R, p.m, p.R, p.R, p.m, p.m, kBLower, -1.0});
-        if (p.top) add({p.X, p.X, p.T, p.m, p.m, p.m, p.m, p.m, p.m, kGram, 1.0});
-    }
+    for (const Place &p : at)
+        if (p.R > 0) add({p.D + p.m, p.X, p.Q, p.m + p.R, p.m, p.R, p.R, p.m, p.m, kBLower, -1.0});
     stage.push_back(tiles.size());
     InverseColumn *dcols = nullptr;
     InverseJob *ddiag = nullptr, *djobs = nullptr;
@@ -418,33 +475,44 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
         gemm_tiles<<<dim3((unsigned)count), kThreads>>>(djobs, dtiles + stage[q]);
         INV_TRY(hipGetLastError());
     }
-    if (!ptiles.empty()) {
-        pack_tiles<F><<<dim3((unsigned)ptiles.size()), kThreads>>>(dpacks, dptiles, mfwd, mbwd);
-        INV_TRY(hipGetLastError());
-    }
-    for (size_t i = 0; i < at.size(); ++i)
-        if (at[i].top) {
-            const unsigned grid = (unsigned)std::min<int64_t>((top_entries(at[i].m) + kThreads - 1) / kThreads, 1 << 16);
-            pack_top<F><<<grid, kThreads>>>(at[i].T, at[i].m, P.is_whole(large[i]) ? order + P.start[large[i]] : nullptr,
-                                           mtop + P.top_off[large[i]]);
-            INV_TRY(hipGetLastError());
-        }
+    pack_tiles<F><<<dim3((unsigned)ptiles.size()), kThreads>>>(dpacks, dptiles, mfwd, mbwd);
+    INV_TRY(hipGetLastError());
     return hipDeviceSynchronize();   // the work arrays are freed on return
 }
 
+// The top blocks' X and X'.
+template <typename F>
+hipError_t fill_tops(const InverseArgs &args, const DeviceTopLists &t, F *mtop) {
+    Arena arena;
+    double *D = nullptr, *T = nullptr;
+    INV_TRY(arena.get(&D, (size_t)t.tiles * kTopTileEntries));
+    INV_TRY(arena.get(&T, (size_t)t.temps * kTopTileEntries));
+    INV_TRY(hipMemsetAsync(D, 0, (size_t)t.tiles * kTopTileEntries * sizeof(double), nullptr));
+    top_scatter<<<dim3((unsigned)t.n_columns), 64>>>(args, t.columns, t.map, D);
+    INV_TRY(hipGetLastError());
+    top_diagonals<<<dim3((unsigned)t.n_diagonals), kThreads>>>(t.diagonals, D);
+    INV_TRY(hipGetLastError());
+    for (size_t s = 0; s + 1 < t.stages.size(); ++s) {
+        const int count = t.stages[s + 1] - t.stages[s];
+        if (count == 0) continue;
+        const bool even = s % 2 == 0;
+        top_products<<<dim3((unsigned)count), kThreads>>>(t.jobs + t.stages[s], t.pairs, D, even ? D : T, even ? T : D,
+                                                          even ? 1.0 : -1.0);
+        INV_TRY(hipGetLastError());
+    }
+    top_pack<F><<<dim3((unsigned)(2 * (t.entries / kTopUnitEntries))), kTopUnitEntries>>>(t.pack, D, mtop);
+    INV_TRY(hipGetLastError());
+    return hipDeviceSynchronize();   // the work arrays are freed on return
+}
 
 template <typename F>
-hipError_t fill(const BlockPlan &P, const InverseArgs &args, const int *order, F *mfwd, F *mbwd, F *mtop) {
-    std::vector<int> small, large;
-    for (int b = 0; b < P.nblocks; ++b) {
-        const bool top = P.is_top(b);
-        (!top && P.start[b + 1] - P.start[b] <= kSmall ? small : large).push_back(b);
-    }
-    Arena arena;
-    if (!small.empty()) {
-        int *ids = nullptr;
-        INV_TRY(arena.put(&ids, small));
-        small_blocks<F><<<dim3((unsigned)small.size()), kThreads>>>(args, ids, mfwd, mbwd);
+hipError_t fill(const BlockPlan &P, const InverseArgs &args, const int *small, int n_small, const DeviceTopLists &tops,
+                F *mfwd, F *mbwd, F *mtop) {
+    std::vector<int> large;
+    for (int b = 0; b < P.nblocks; ++b)
+        if (!P.is_top(b) && P.start[b + 1] - P.start[b] > kSmall) large.push_back(b);
+    if (n_small > 0) {
+        small_blocks<F><<<dim3((unsigned)n_small), kThreads>>>(args, small, mfwd, mbwd);
         INV_TRY(hipGetLastError());
     }
     // In groups whose work arrays take up to 4 GiB.
@@ -458,21 +526,60 @@ hipError_t fill(const BlockPlan &P, const InverseArgs &args, const int *order, F
             if (hi > lo && words > kGroup) break;
             group.push_back(large[hi]);
         }
-        INV_TRY(fill_large<F>(P, args, group, order, mfwd, mbwd, mtop));
+        INV_TRY(fill_large<F>(P, args, group, mfwd, mbwd));
         lo = hi;
     }
+    if (tops.n_columns > 0) INV_TRY(fill_tops<F>(args, tops, mtop));
     return hipDeviceSynchronize();
+}
+
+template <typename T>
+hipError_t put(T **dst, const std::vector<T> &v) {
+    *dst = nullptr;
+    if (v.empty()) return hipSuccess;
+    const hipError_t e = hipMalloc(reinterpret_cast<void **>(dst), v.size() * sizeof(T));
+    return e != hipSuccess ? e : hipMemcpy(*dst, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice);
 }
 
 }  // namespace
 
-hipError_t fill_block_plan_on_device(const BlockPlan &P, const InverseArgs &args, const int *order, int float_bytes,
-                                     void *mfwd, void *mbwd, void *mtop) {
+void DeviceTopLists::release() {
+    for (void *p : {(void *)columns, (void *)map, (void *)pack, (void *)diagonals, (void *)jobs, (void *)pairs})
+        if (p) (void)hipFree(p);
+    *this = DeviceTopLists();
+}
+
+hipError_t DeviceTopLists::upload(const TopLists &l) {
+    release();
+    INV_TRY(put(&columns, l.columns));
+    INV_TRY(put(&map, l.map));
+    INV_TRY(put(&pack, l.pack));
+    INV_TRY(put(&diagonals, l.diagonals));
+    INV_TRY(put(&jobs, l.jobs));
+    INV_TRY(put(&pairs, l.pairs));
+    n_columns = (int)l.columns.size();
+    n_diagonals = (int)l.diagonals.size();
+    tiles = l.tiles;
+    temps = l.temps;
+    entries = l.entries;
+    stages = l.stages;
+    return hipSuccess;
+}
+
+std::vector<int> small_block_list(const BlockPlan &P) {
+    std::vector<int> small;
+    for (int b = 0; b < P.nblocks; ++b)
+        if (!P.is_top(b) && P.start[b + 1] - P.start[b] <= kSmall) small.push_back(b);
+    return small;
+}
+
+hipError_t fill_block_plan_on_device(const BlockPlan &P, const InverseArgs &args, const int *small, int n_small,
+                                     const DeviceTopLists &tops, int float_bytes, void *mfwd, void *mbwd, void *mtop) {
     if (P.n == 0) return hipSuccess;
     if (float_bytes == 4)
-        return fill<float>(P, args, order, static_cast<float *>(mfwd), static_cast<float *>(mbwd),
+        return fill<float>(P, args, small, n_small, tops, static_cast<float *>(mfwd), static_cast<float *>(mbwd),
                            static_cast<float *>(mtop));
-    return fill<double>(P, args, order, static_cast<double *>(mfwd), static_cast<double *>(mbwd),
+    return fill<double>(P, args, small, n_small, tops, static_cast<double *>(mfwd), static_cast<double *>(mbwd),
                         static_cast<double *>(mtop));
 }
 

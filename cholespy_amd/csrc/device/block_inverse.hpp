@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include "block_plan.hpp"
+#include "dense_top_plan.hpp"
 
 namespace cholespy_amd {
 
@@ -19,10 +20,9 @@ struct InverseArgs {
     const int64_t *moff;
 };
 
-// One product C := alpha op(A) B (column-major, M x N, reduction K).
+// One product C := alpha A B (column-major, M x N, reduction K).
 constexpr int kBLower = 1;   // B is lower triangular: columns from j0 start at k = j0
 constexpr int kALower = 2;   // A is lower triangular: rows up to i0 + 63 end at k = i0 + 63
-constexpr int kGram = 4;     // op(A) = A', A = B lower triangular; only the lower half of C
 struct InverseJob {
     const double *A, *B;
     double *C;
@@ -43,12 +43,28 @@ struct InversePack {
     int m, R;
 };
 
-// Fills mfwd and mbwd (offsets P.moff) and, for dense top blocks, mtop
-// (offsets P.top_off). order (device, null if no top block is a whole system):
-// for a whole system, caller row i of it (plan row start + i) is row
-// order[start + i] of its factor.
-hipError_t fill_block_plan_on_device(const BlockPlan &P, const InverseArgs &args, const int *order, int float_bytes,
-                                     void *mfwd, void *mbwd, void *mtop);
+// Device copies of the lists that form the top blocks' inverses
+// (dense_top_plan.hpp), the stages on the host.
+struct DeviceTopLists {
+    TopLists::Column *columns = nullptr;
+    int *map = nullptr, *pack = nullptr;
+    TopLists::Diagonal *diagonals = nullptr;
+    TopLists::Job *jobs = nullptr;
+    TopLists::Pair *pairs = nullptr;
+    int n_columns = 0, n_diagonals = 0, tiles = 0, temps = 0;
+    int64_t entries = 0;           // elements of one direction's array
+    std::vector<int> stages;
+    void release();
+    hipError_t upload(const TopLists &lists);
+};
+
+// Fills mfwd and mbwd (offsets P.moff) and the top blocks' mtop (X, then X',
+// tops.entries elements each). small: device list of the n_small blocks of up
+// to 64 rows that are not top blocks.
+hipError_t fill_block_plan_on_device(const BlockPlan &P, const InverseArgs &args, const int *small, int n_small,
+                                     const DeviceTopLists &tops, int float_bytes, void *mfwd, void *mbwd, void *mtop);
+// The blocks of P that `small` lists.
+std::vector<int> small_block_list(const BlockPlan &P);
 
 // The factor's values in the solver's precision: uvals[p] = val[p] (column
 // form), lvals[p] = val[csr_src[p]] (row form).

@@ -4,6 +4,7 @@
 
 #include <atomic>
 #include <functional>
+#include <limits>
 #include <thread>
 
 #include <algorithm>
@@ -328,11 +329,15 @@ BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx
     const int nb = (int)start.size() - 1;
     P.nblocks = nb;
     if (opt.top_rows > 0 && n > 0) {
-        P.top_off.assign((size_t)nb, -1);
-        P.top_off[(size_t)nb - 1] = 0;
-        P.top_size = top_entries(opt.top_rows);
-        P.top_whole.assign((size_t)nb, 0);
-        P.top_whole[(size_t)nb - 1] = nb == 1;
+        const int end = n - std::min(n, opt.top_rows);
+        P.top_flag.assign((size_t)nb, 0);
+        for (int b = 0; b < nb; ++b) {
+            if (start[b] < end) continue;
+            P.top_flag[(size_t)b] = 1;
+            BlockPlan::TopBlock top{b, {}};
+            for (int i = start[b]; i < start[b + 1]; ++i) top.parent.push_back(parent[i] < 0 ? -1 : parent[i] - start[b]);
+            P.tops.push_back(std::move(top));
+        }
     }
     std::vector<int> block_of(n);
     for (int b = 0; b < nb; ++b)
@@ -359,6 +364,7 @@ BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx
         P.rptr[b + 1] = (int)P.rlist.size();
         const int64_t m = e - a, R = (int64_t)rows_b.size();
         if (P.is_top(b)) {
+            if (R > 0) throw std::logic_error("block plan: a top block has rows below it");
             P.moff[b + 1] = P.moff[b];
             continue;
         }
@@ -537,21 +543,33 @@ DenseTop choose_dense_top(int n, const int *colptr, const int *rowidx, const Blo
         if (p >= 0) level[block_of[p]] = std::max(level[block_of[p]], level[b] + 1);
         levels = std::max(levels, level[b] + 1);
     }
-    // Per level: the rows of the blocks from it up, and the entries of its M_B.
-    std::vector<int64_t> rows((size_t)levels + 1, 0), entries((size_t)levels, 0);
+    // Per row: its ancestors with itself (the entries of its column of X:
+    // every ancestor of a top row is one too).
+    std::vector<int> depth((size_t)n);
+    for (int j = n - 1; j >= 0; --j) depth[j] = parent[j] < 0 ? 1 : depth[parent[j]] + 1;
+    // Per level: the rows of the blocks from it up and the entries of their X,
+    // and the entries of its own M_B.
+    std::vector<int64_t> rows((size_t)levels + 1, 0), inverse((size_t)levels + 1, 0), entries((size_t)levels, 0);
     for (int b = 0; b < nb; ++b) {
         const int64_t m = start[b + 1] - start[b], below = colptr[start[b + 1]] - colptr[start[b + 1] - 1] - 1;
         rows[level[b]] += m;
         entries[level[b]] += m * (m + 1) / 2 + m * below;   // (|R| >= the last column's rows below)
+        for (int i = start[b]; i < start[b + 1]; ++i) inverse[level[b]] += depth[i];
     }
-    for (int l = levels - 1; l >= 0; --l) rows[l] += rows[l + 1];
+    for (int l = levels - 1; l >= 0; --l) {
+        rows[l] += rows[l + 1];
+        inverse[l] += inverse[l + 1];
+    }
     double passes = opt.pass_us;
     for (int l = 0; l < levels; ++l) passes += 2.0 * (opt.level_us + (double)entries[l] * float_bytes / opt.level_gbs * 1e-3);
     int cut = levels;
-    double best = passes;
-    for (int l = levels - 1; l >= 0 && rows[l] <= opt.top_max_rows; --l) {
+    double best = opt.top_forced ? std::numeric_limits<double>::infinity() : passes;
+    const int64_t most = std::min<int64_t>(opt.top_max_rows, kTopMaxRows);
+    for (int l = levels - 1; l >= 0 && rows[l] <= most; --l) {
         passes -= 2.0 * (opt.level_us + (double)entries[l] * float_bytes / opt.level_gbs * 1e-3);
-        const double us = (l > 0 ? passes : 0.0) + opt.top_us + (double)top_entries(rows[l]) * float_bytes / opt.top_gbs * 1e-3;
+        // X is stored twice, in 16 x 16 units: about 48 more entries a row than it has.
+        const double stored = 2.0 * ((double)inverse[l] + 48.0 * (double)rows[l]);
+        const double us = (l > 0 ? passes : 0.0) + opt.top_us + stored * float_bytes / opt.top_gbs * 1e-3;
         if (us < best) {
             best = us;
             cut = l;
@@ -567,6 +585,7 @@ DenseTop choose_dense_top(int n, const int *colptr, const int *rowidx, const Blo
     return top;
 }
 
+// (A column's rows are ancestors of one another, which a topological order keeps in order.)
 void renumber_pattern(int n, const int *colptr, const int *rowidx, const std::vector<int> &src,
                       std::vector<int> &new_colptr, std::vector<int> &new_rowidx) {
     std::vector<int> rank((size_t)n);
@@ -577,7 +596,6 @@ void renumber_pattern(int n, const int *colptr, const int *rowidx, const std::ve
         const int j = src[r];
         int q = new_colptr[r];
         for (int p = colptr[j]; p < colptr[j + 1]; ++p) new_rowidx[q++] = rank[rowidx[p]];
-        std::sort(new_rowidx.begin() + new_colptr[r], new_rowidx.begin() + q);
         new_colptr[r + 1] = q;
     }
 }

@@ -88,23 +88,27 @@ struct BlockPlanOptions {
     // Blocks of one level are independent, so either order is a valid
     // schedule.
     bool critical_order = true;
-    // Rows of the dense top block: the last top_rows rows of the factor (an
-    // ancestor-closed set: see choose_dense_top) form one block that is
-    // solved by the explicit inverse of its Schur complement between the two
-    // passes. 0 = none. The host fill does not form its values.
+    // Rows of the dense top: the last top_rows rows of the factor (an
+    // ancestor-closed set: see choose_dense_top), one block, solved with the
+    // explicit inverse X of L's part between the two passes. 0 = none. The
+    // host fill does not form its values.
     int top_rows = 0;
     // What choose_dense_top weighs, in microseconds and GB/s: the two passes'
     // launches and leaf tasks, a level of a pass (its hand-offs, and its M_B
-    // at the rate the block tasks reach), and the dense product.
-    // Fitted to where the measured best cut lies: icosphere(7), k = 3, FP32 has
-    // 157.9 us with 2.9k rows, 166.8 with 5.1k, 168.0 with 978; icosphere(6)
-    // k = 3 85 us a solve with 3.5k rows, 100 with 5.4k, and k = 128 251 and
-    // 283 us; a 48^3 grid, k = 32, FP32 450 us with 6.2k rows, 510 with 3.2k;
-    // a 33^3 grid, k = 5, FP64 174 us with 3.7k, 186 with 1.5k. More rows
-    // than top_max_rows would cost a refactorisation more (n^3) than they
-    // give a solve.
-    double pass_us = 25.0, level_us = 3.5, level_gbs = 3000.0, top_us = 5.0, top_gbs = 5500.0;
+    // at the rate the block tasks reach), and the products with X and X' (two
+    // launches and X's entries at the rate they reach). Fitted to solves of
+    // k = 3 over all cuts of eight systems, in us without a top and with what
+    // the rule takes: icosphere(5) FP32 65.5 -> 43.3 (2,640 rows), (6) FP32
+    // 93.0 -> 70.2 (5,274), (6) FP64 98.7 -> 77.5, (7) FP32 143.5 -> 146.3
+    // (5,109; k = 17 257 -> 227), (7) FP64 none (163.4; 169.6 with 2,886 rows,
+    // k = 17 288 and 270), 511 x 389 grid FP64 161.7 -> 156.2 (3,479; 161.7
+    // with 6,114), 200 x 150 grid FP64 78.3 -> 57.6 (5,455), 33^3 grid FP64
+    // 154.5 -> 126.5 (4,507), 48^3 grid FP32 243.3 -> 228.7 (6,241). More right-
+    // hand sides gain more from the same cuts. More rows than top_max_rows
+    // were hardly measured, and cost a refactorisation more than they give.
+    double pass_us = 25.0, level_us = 3.0, level_gbs = 4000.0, top_us = 12.0, top_gbs = 4000.0;
     int64_t top_max_rows = 6400;
+    bool top_forced = false;   // a top wherever a cut fits top_max_rows, estimate or not
     // Host threads for the dense block inverses (0 = hardware count, at most
     // 16). Batches already build one plan per thread and pass 1.
     int threads = 0;
@@ -134,7 +138,7 @@ struct BlockPlan {
     //   (block, first, last, kind, lo, hi, sbase, split).
     // Forward kinds: 0 = gather r_B and multiply rows [first, last) of M_B;
     // 1 = gather rows [first, last) of r_B only (published for kinds 2, 3);
-    // 4 = the same for a dense top block, into y (read after the pass);
+    // 4 = the same for a dense top block, into z (read after the pass);
     // 2 = multiply rows [first, last) of M_B by the published r_B;
     // 3 = split s of nsplit (split = split_code(s, nsplit)): as 2 over
     //     columns [lo, hi) only, result published to the split rows
@@ -153,18 +157,18 @@ struct BlockPlan {
     // BlockPlanOptions' wide_* shape), leaf tasks first and last as well.
     std::vector<int> fwd_task_wide, bwd_task_wide;
     int n_leaf_fwd_wide = 0, n_leaf_bwd_wide = 0;
-    // Dense top blocks (none, or one per system): top_off[b] = offset of the
-    // block's inverse (top_entries(m) elements) in an array of its own, -1 for
-    // other blocks (empty: no top block). They have no entries in mfwd /
-    // mbwd, no R rows and no backward tasks; their forward tasks are gathers
-    // (kind 4) that leave r_B in y for the dense product.
-    std::vector<int64_t> top_off;
-    int64_t top_size = 0;                  // elements of all top inverses
-    // Top blocks that are a whole system: their inverse is stored in the
-    // caller's row order, so their plan rows stand for caller rows in order.
-    std::vector<char> top_whole;
-    bool is_whole(int b) const { return !top_whole.empty() && top_whole[(std::size_t)b] != 0; }
-    bool is_top(int b) const { return !top_off.empty() && top_off[(std::size_t)b] >= 0; }
+    // Dense top blocks (none, or one per system). They have no
+    // entries in mfwd / mbwd, no R rows and no backward tasks; their forward
+    // tasks are gathers (kind 4) that leave r_B in z, for the products of
+    // dense_top.hip. parent: the elimination tree among the block's rows
+    // (counted from its first, -1 at the root).
+    struct TopBlock {
+        int block;
+        std::vector<int> parent;
+    };
+    std::vector<TopBlock> tops;
+    std::vector<char> top_flag;            // per block (empty: no top block)
+    bool is_top(int b) const { return !top_flag.empty() && top_flag[(std::size_t)b] != 0; }
     int nsplit_rows = 0;                   // rows of the split-result array (either list)
     int max_m = 0, max_rows = 0;           // largest m and m + |R|
     int64_t nnz_l = 0;
@@ -183,17 +187,16 @@ BlockPlan build_block_plan(int n, const int *colptr, const int *rowidx, const do
 BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx, const BlockPlanOptions &opt);
 void fill_block_plan_values(BlockPlan &P, const int *colptr, const int *rowidx, const double *val, int threads);
 
-// Elements of the stored inverse of an m-row top block: panels of 16 columns,
-// rows padded to a multiple of 16 (layout in dense_top.hip).
-constexpr int64_t top_entries(int64_t m) { return ((m + 15) / 16 * 16) * ((m + 15) / 16 * 16); }
+// The most rows of a dense top (dense_top.hip keeps a wavefront's input units
+// in two registers of a row).
+constexpr int kTopMaxRows = 7168;
 
-// The rows that are worth solving as one dense block, and a numbering that
-// puts them last. src[r] = factor row at plan row r (the other rows keep
+// The rows that are worth solving by an explicit inverse, and a numbering
+// that puts them last. src[r] = factor row at plan row r (the other rows keep
 // their order, then the top rows in order: a topological order of the
-// elimination tree, so L keeps its pattern under it); empty src: no top
-// block. Blocks at forward level >= cut (in the partition that `opt` gives)
-// are the top rows; the cut minimises the estimated time of the levels below
-// it and of the dense product.
+// elimination tree, so L keeps its pattern under it); empty src: no top block. Blocks at forward level >= cut (in the partition that
+// `opt` gives) are the top rows; the cut minimises the estimated time of the
+// levels below it and of the products with the inverse.
 struct DenseTop {
     int rows = 0;
     int max_block = 0;   // chain cap of the whole factor's partition

@@ -24,6 +24,7 @@
 #include "block_inverse.hpp"
 #include "block_plan.hpp"
 #include "common.hpp"
+#include "dense_top_plan.hpp"
 #include "launchers.hpp"
 
 using namespace cholespy_amd;
@@ -109,19 +110,31 @@ struct DeviceBlockPlan {
     int *cptr = nullptr, *cslot = nullptr, *gslot = nullptr;
     int *ftask = nullptr, *btask = nullptr;
     int *ftask_wide = nullptr, *btask_wide = nullptr;
-    // Dense top blocks (block_plan.hpp): their inverses and the tile list of
-    // the dense product. whole: a single system that is one top block.
+    // Dense top blocks (dense_top_plan.hpp): X and X', the panels of the two
+    // products and the lists that form X. whole: every block is a top block.
     void *mtop = nullptr;
-    DenseTopTile *top_tiles = nullptr;
-    int n_top_tiles = 0;
+    DenseTopPanel *top_fwd = nullptr, *top_bwd = nullptr;
+    int *top_units = nullptr;
+    int n_top_panels = 0;
     bool whole = false;
-    int top_rows = 0;      // of a single system
+    DeviceTopLists tops;
     int *perm = nullptr;   // caller row of each plan row
+    // What a fill reads besides the plan (fill_plan_values).
+    int64_t *colptr = nullptr;
+    int *src = nullptr, *rank = nullptr, *small = nullptr;
+    int n_small = 0;
 
     void release() {
         dev_free(mtop);
-        dev_free(top_tiles);
+        dev_free(top_fwd);
+        dev_free(top_bwd);
+        dev_free(top_units);
+        tops.release();
         dev_free(perm);
+        dev_free(colptr);
+        dev_free(src);
+        dev_free(rank);
+        dev_free(small);
         dev_free(start);
         dev_free(rptr);
         dev_free(rlist);
@@ -144,6 +157,7 @@ struct cholespy_gpu_solver;
 namespace {
 BlockPlanOptions plan_options(const BlockPlanOptions &base = BlockPlanOptions());
 int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<int> &perm,
+                const std::vector<int64_t> &colptr, const std::vector<int> &src,
                 const std::vector<int> *blk_sys = nullptr);
 }  // namespace
 
@@ -242,7 +256,6 @@ struct cholespy_gpu_solver {
     std::vector<int> host_perm, host_colptr, host_rowidx;
     int *csr_src = nullptr;
     BlockPlan host_plan;
-    std::vector<int> plan_src;   // factor row of each plan row
 };
 
 namespace {
@@ -300,9 +313,10 @@ std::vector<int> device_tasks(const BlockPlan &P, const std::vector<int> &tasks,
 
 // Copies the structure of a (possibly merged) block plan to the device and
 // allocates its values, which fill_plan_values forms there. perm: caller row
-// of each plan row; blk_sys maps blocks to systems for a batch.
+// of each plan row; L in compressed columns (colptr), whose row src[r] is plan
+// row r; blk_sys maps blocks to systems for a batch.
 int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<int> &perm,
-                const std::vector<int> *blk_sys) {
+                const std::vector<int64_t> &colptr, const std::vector<int> &src, const std::vector<int> *blk_sys) {
     DeviceBlockPlan &d = s->plan;
     d.release();
     d.nblocks = P.nblocks;
@@ -321,12 +335,8 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
     d.levels_fwd = d.levels_bwd = 0;
     for (int v : P.level_fwd) d.levels_fwd = std::max(d.levels_fwd, v + 1);
     for (int v : P.level_bwd) d.levels_bwd = std::max(d.levels_bwd, v + 1);
-    d.m_entries = P.moff[P.nblocks];   // (a top block's square serves both passes: half of it each)
-    for (int b = 0; b < P.nblocks; ++b)
-        if (P.is_top(b)) {
-            const int64_t m = P.start[b + 1] - P.start[b];
-            d.m_entries += (m * m + 1) / 2;
-        }
+    const TopLists tops = top_lists(P, blk_sys);
+    d.m_entries = P.moff[P.nblocks] + tops.entries;
     s->plan_copy[0] = P.start;
     s->plan_copy[1] = P.rptr;
     s->plan_copy[2] = P.level_fwd;
@@ -355,17 +365,21 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
     const size_t me = (size_t)P.moff[P.nblocks], fb = (size_t)s->fbytes;
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mfwd), me * fb));
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mbwd), me * fb));
-    HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mtop), (size_t)P.top_size * fb));
-    std::vector<DenseTopTile> tiles;
-    for (int b = 0; b < P.nblocks; ++b) {
-        if (!P.is_top(b)) continue;
-        const int m = P.start[b + 1] - P.start[b], panels = (m + 15) / 16, sys = blk_sys ? (*blk_sys)[b] : 0;
-        for (int p = 0; p < panels; ++p) tiles.push_back(DenseTopTile{P.start[b], m, p, sys, P.top_off[b]});
-    }
-    d.n_top_tiles = (int)tiles.size();
-    d.top_rows = !blk_sys && !P.top_off.empty() ? P.n - P.start[P.nblocks - 1] : 0;
-    d.whole = !blk_sys && P.nblocks == 1 && P.is_whole(0);
-    HIP_TRY(upload(&d.top_tiles, tiles.data(), tiles.size()));
+    HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mtop), 2 * (size_t)tops.entries * fb));
+    d.n_top_panels = (int)tops.fwd.size();
+    d.whole = !blk_sys && P.nblocks > 0 && (int)P.tops.size() == P.nblocks;
+    HIP_TRY(upload(&d.top_fwd, tops.fwd.data(), tops.fwd.size()));
+    HIP_TRY(upload(&d.top_bwd, tops.bwd.data(), tops.bwd.size()));
+    HIP_TRY(upload(&d.top_units, tops.units.data(), tops.units.size()));
+    HIP_TRY(d.tops.upload(tops));
+    std::vector<int> rank(src.size());
+    for (size_t r = 0; r < src.size(); ++r) rank[(size_t)src[r]] = (int)r;
+    HIP_TRY(upload(&d.colptr, colptr.data(), colptr.size()));
+    HIP_TRY(upload(&d.src, src.data(), src.size()));
+    HIP_TRY(upload(&d.rank, rank.data(), rank.size()));
+    const std::vector<int> small = small_block_list(P);
+    d.n_small = (int)small.size();
+    HIP_TRY(upload(&d.small, small.data(), small.size()));
     for (auto &row : s->grid_blocks)
         for (int &g : row) g = 0;
     s->buffers_path = -1;
@@ -388,28 +402,11 @@ struct DeviceTemp {
 };
 
 // Forms the plan's dense values on the device (block_inverse.hip) from L in
-// compressed columns (colptr: host, rowidx and val: device), whose row
-// src[r] is plan row r (for a whole top block: its factor row, the plan rows
-// standing for caller rows). perm: caller row of each factor row.
-int fill_plan_values(cholespy_gpu_solver *s, const BlockPlan &P, const int64_t *colptr, const int *rowidx,
-                     const double *val, const std::vector<int> &src, const std::vector<int> &perm) {
+// compressed columns (rowidx and val: device).
+int fill_plan_values(cholespy_gpu_solver *s, const BlockPlan &P, const int *rowidx, const double *val) {
     DeviceBlockPlan &d = s->plan;
-    const size_t n = (size_t)P.n;
-    std::vector<int> rank(n), order;
-    for (size_t r = 0; r < n; ++r) rank[(size_t)src[r]] = (int)r;
-    DeviceTemp tcol, tsrc, trank, torder;
-    HIP_TRY(tcol.put(colptr, n + 1));
-    HIP_TRY(tsrc.put(src.data(), n));
-    HIP_TRY(trank.put(rank.data(), n));
-    for (int b = 0; b < P.nblocks; ++b) {
-        if (!P.is_whole(b)) continue;
-        order.resize(n);
-        for (int r = P.start[b]; r < P.start[b + 1]; ++r) order[(size_t)perm[(size_t)src[(size_t)r]]] = r - P.start[b];
-    }
-    if (!order.empty()) HIP_TRY(torder.put(order.data(), n));
-    const InverseArgs args{tcol.as<int64_t>(), rowidx, val,    tsrc.as<int>(), trank.as<int>(),
-                           d.start,            d.rptr, d.rlist, d.moff};
-    HIP_TRY(fill_block_plan_on_device(P, args, torder.as<int>(), s->fbytes, d.mfwd, d.mbwd, d.mtop));
+    const InverseArgs args{d.colptr, rowidx, val, d.src, d.rank, d.start, d.rptr, d.rlist, d.moff};
+    HIP_TRY(fill_block_plan_on_device(P, args, d.small, d.n_small, d.tops, s->fbytes, d.mfwd, d.mbwd, d.mtop));
     return CHOLESPY_OK;
 }
 
@@ -419,13 +416,11 @@ int upload_values(cholespy_gpu_solver *s, const double *val) {
     DeviceTemp tval;
     HIP_TRY(tval.put(val, (size_t)s->nnz));
     HIP_TRY(launch_cast_factor(s->fbytes, s->nnz, tval.as<double>(), s->csr_src, s->lvals, s->uvals));
-    const std::vector<int64_t> colptr(s->host_colptr.begin(), s->host_colptr.end());
-    return fill_plan_values(s, s->host_plan, colptr.data(), s->ucols, tval.as<double>(), s->plan_src,
-                            s->host_perm);
+    return fill_plan_values(s, s->host_plan, s->ucols, tval.as<double>());
 }
 
-// Whether plans may have a dense top (CHOLESPY_DENSE_TOP: its most rows, 0 =
-// none). Knobs that shape the large blocks' tasks ask for those tasks: with
+// Whether plans may have a dense top (CHOLESPY_DENSE_TOP: its most rows, and
+// then one wherever it fits; 0 = none). Knobs that shape the large blocks' tasks ask for those tasks: with
 // one of them set the plan keeps its levels.
 int64_t dense_top_rows(const BlockPlanOptions &opt) {
     if (const char *e = std::getenv("CHOLESPY_DENSE_TOP")) return std::max(0, std::atoi(e));
@@ -442,6 +437,7 @@ int64_t dense_top_rows(const BlockPlanOptions &opt) {
 BlockPlan plan_structure(int n, const int *colptr, const int *rowidx, BlockPlanOptions opt, int float_bytes,
                          std::vector<int> &src) {
     opt.top_max_rows = dense_top_rows(opt);
+    opt.top_forced = std::getenv("CHOLESPY_DENSE_TOP") != nullptr;
     DenseTop top;
     if (opt.top_max_rows > 0) top = choose_dense_top(n, colptr, rowidx, opt, float_bytes);
     opt.top_rows = top.rows;
@@ -467,13 +463,11 @@ int plan_system(cholespy_gpu_solver *s, const BlockPlanOptions &base) {
     } catch (const std::exception &ex) {
         return fail(CHOLESPY_ERR_INVALID_ARGUMENT, ex.what());
     }
-    const bool whole = P.nblocks == 1 && P.is_whole(0);
     std::vector<int> perm((size_t)s->n);
-    for (int r = 0; r < s->n; ++r) perm[(size_t)r] = whole ? r : s->host_perm[(size_t)src[(size_t)r]];
-    const int rc = upload_plan(s, P, perm);
+    for (int r = 0; r < s->n; ++r) perm[(size_t)r] = s->host_perm[(size_t)src[(size_t)r]];
+    const int rc = upload_plan(s, P, perm, std::vector<int64_t>(s->host_colptr.begin(), s->host_colptr.end()), src);
     if (rc != CHOLESPY_OK) return rc;
     s->host_plan = std::move(P);
-    s->plan_src.swap(src);
     s->plan_base = base;
     return CHOLESPY_OK;
 }
@@ -956,17 +950,6 @@ int effective_tile(const cholespy_gpu_solver *s, int fbytes, int k) {
     return rule;
 }
 
-bool overlaps(const void *p, size_t pn, const void *q, size_t qn) {
-    const char *a = static_cast<const char *>(p), *b = static_cast<const char *>(q);
-    return a < b + qn && b < a + pn;
-}
-
-// Whether a block solve of the handle needs its work buffers at all.
-bool solves_directly(const cholespy_gpu_solver *s, const void *b, const void *x, int k, size_t x_elem) {
-    const size_t elems = (size_t)s->n * (size_t)k;
-    return s->path == CHOLESPY_PATH_BLOCKS && s->plan.whole && !overlaps(b, elems * (size_t)s->fbytes, x, elems * x_elem);
-}
-
 // Work buffers of one block solve (the handle's own, or the library's
 // scratch array for cholespy_solver_solve_noalloc).
 struct WorkSet {
@@ -1010,36 +993,38 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         bf.sys_pbase = s->sys_pbase;
         bf.sys_sbase = s->sys_sbase;
     }
-    DenseTopArgs top;
-    top.tiles = s->is_batch ? d.top_tiles : nullptr;
-    top.row0 = s->n - d.top_rows;
-    top.n = d.top_rows;
-    top.M = d.mtop;
-    top.in = w.y;
-    top.z = d.whole ? nullptr : w.z;
-    top.x = x;
-    top.perm = d.whole ? nullptr : d.perm;
-    top.k = k;
-    top.xmode = xmode;
-    top.sys_k = bf.sys_k;
-    top.sys_vbase = bf.sys_vbase;
-    if (d.whole) {
-        // One product. Its input is b itself, unless the passes run apart or
-        // x overlaps b: then a copy in y.
-        const size_t bytes = (size_t)s->n * (size_t)k * (size_t)fbytes;
-        if (only_pass == 0 || (only_pass < 0 && overlaps(b, bytes, x, xmode == 0 ? bytes : 8 * (bytes / fbytes))))
-            HIP_TRY(launch_copy(w.y, b, bytes, st));
-        else if (only_pass < 0)
+    // The products with the top's inverse: y_T = X r_T at the end of the
+    // forward pass, r_T in z (gathered there by its tasks, or for a whole
+    // system b itself), and z_T = X' y_T at the start of the backward pass.
+    auto dense_top = [&](bool forward) -> hipError_t {
+        DenseTopArgs top{};
+        const size_t half = (size_t)d.tops.entries * (size_t)fbytes;
+        top.panels = forward ? d.top_fwd : d.top_bwd;
+        top.units = forward ? nullptr : d.top_units;
+        top.M = static_cast<const char *>(d.mtop) + (forward ? 0 : half);
+        top.in = forward ? w.z : w.y;
+        top.out = forward ? w.y : d.whole ? nullptr : w.z;
+        top.x = forward ? nullptr : x;
+        top.perm = d.perm;
+        top.k = k;
+        top.xmode = xmode;
+        top.sys_k = bf.sys_k;
+        top.sys_vbase = bf.sys_vbase;
+        if (forward && d.whole && k <= kNarrowTile) {
             top.in = b;
-        if (only_pass != 0)
-            HIP_TRY(launch_dense_top(fbytes, top, d.n_top_tiles, k, st));
-        return CHOLESPY_OK;
-    }
+            top.rows = d.perm;
+            top.b_rows = s->n;
+        } else if (forward && d.whole) {
+            const hipError_t e = launch_gather_rows(fbytes, w.z, b, d.perm, s->n, k, st);
+            if (e != hipSuccess) return e;
+        }
+        return launch_dense_top(fbytes, top, d.n_top_panels, bf.max_k, st);
+    };
     for (int pass = 0; pass < 2; ++pass) {
         if (only_pass >= 0 && pass != only_pass) continue;
         const bool forward = pass == 0;
-        if (!forward && d.n_top_tiles > 0)
-            HIP_TRY(launch_dense_top(fbytes, top, d.n_top_tiles, bf.max_k, st));
+        if (d.n_top_panels > 0 && (!forward || d.whole)) HIP_TRY(dense_top(forward));
+        if (d.whole) continue;
         const int tile = effective_tile(s, fbytes, bf.max_k);
         if (is_panel_tile(tile)) {
             bf.ntasks = forward ? d.n_fwd_tasks_wide : d.n_bwd_tasks_wide;
@@ -1067,6 +1052,7 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         bf.tile = tile;
         bf.leaf_queues = &s->queues[6 + (forward ? 1 : 0)];
         HIP_TRY(launch_block_pass(fbytes, forward, bf, grid, s->queues[4 + (forward ? 1 : 0)], st));
+        if (d.n_top_panels > 0 && forward) HIP_TRY(dense_top(true));
     }
     return CHOLESPY_OK;
 }
@@ -1089,7 +1075,6 @@ int solve_impl(cholespy_gpu_solver *s, int fbytes, int k, const void *b, void *x
     int rc = report_give_up(s);
     if (rc != CHOLESPY_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (only_pass < 0 && solves_directly(s, b, x, k, (size_t)fbytes)) return solve_blocks(s, k, b, x, st);
     rc = prepare_buffers(s, k, st);
     if (rc != CHOLESPY_OK) return rc;
     // Pass order. A forward pass publishes partial sums, gathered right-hand
@@ -1414,7 +1399,7 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
     // offsets; tasks of all systems interleaved by block level.
     BlockPlan G;
     G.n = s->n;
-    std::vector<int> blk_sys, gperm((size_t)s->n), gsrc((size_t)s->n), fperm((size_t)s->n);
+    std::vector<int> blk_sys, gperm((size_t)s->n), gsrc((size_t)s->n);
     s->sys_slots.assign((size_t)ns, 0);
     s->sys_slot0.assign((size_t)ns, 0);
     s->sys_splits.assign((size_t)ns, 0);
@@ -1430,11 +1415,9 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
         s->sys_slots[i] = P.rptr[P.nblocks];
         s->sys_split0[i] = SP0;
         s->sys_splits[i] = P.nsplit_rows;
-        const bool whole = P.nblocks == 1 && P.is_whole(0);
         for (int r = 0; r < s->sys_n[i]; ++r) {
-            fperm[(size_t)R0 + r] = R0 + s->pending[i].perm[r];
             gsrc[(size_t)R0 + r] = R0 + srcs[i][r];
-            gperm[(size_t)R0 + r] = R0 + (whole ? r : s->pending[i].perm[srcs[i][r]]);
+            gperm[(size_t)R0 + r] = R0 + s->pending[i].perm[srcs[i][r]];
         }
         for (int b = 0; b < P.nblocks; ++b) {
             G.start.push_back(P.start[b] + R0);
@@ -1443,10 +1426,9 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
             G.level_fwd.push_back(P.level_fwd[b]);
             G.level_bwd.push_back(P.level_bwd[b]);
             blk_sys.push_back(i);
-            G.top_off.push_back(P.is_top(b) ? P.top_off[b] + G.top_size : -1);
-            G.top_whole.push_back(P.is_whole(b));
+            G.top_flag.push_back(P.is_top(b));
         }
-        G.top_size += P.top_size;
+        for (const BlockPlan::TopBlock &top : P.tops) G.tops.push_back({top.block + B0, top.parent});
         for (int v : P.rlist) G.rlist.push_back(v + R0);
         for (int r = 0; r < s->sys_n[i]; ++r) G.contrib_ptr.push_back(P.contrib_ptr[r] + C0);
         for (int v : P.contrib_slot) G.contrib_slot.push_back(v + S0);
@@ -1517,23 +1499,24 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
         emit(btasks_w, false, true, G.bwd_task_wide);
     }
     plans.clear();
-    int rc = upload_plan(s, G, gperm, &blk_sys);
+    // The factors one after another, as the block-diagonal factor of the merged plan.
+    std::vector<int64_t> colptr{0};
+    std::vector<int> rowidx;
+    std::vector<double> val;
+    for (int i = 0; i < ns; ++i) {
+        const auto &h = s->pending[i];
+        const int64_t at = (int64_t)rowidx.size();
+        for (int j = 0; j < s->sys_n[i]; ++j) colptr.push_back(at + h.colptr[j + 1]);
+        for (int v : h.rowidx) rowidx.push_back(v + s->sys_row0[i]);
+        val.insert(val.end(), h.val.begin(), h.val.end());
+    }
+    int rc = upload_plan(s, G, gperm, colptr, gsrc, &blk_sys);
     if (rc != CHOLESPY_OK) return rc;
     {
-        // The factors one after another, as the block-diagonal factor of the merged plan.
-        std::vector<int64_t> colptr{0};
-        std::vector<int> rowidx;
-        std::vector<double> val;
-        for (int i = 0; i < ns; ++i) {
-            const auto &h = s->pending[i];
-            for (int j = 0; j < s->sys_n[i]; ++j) colptr.push_back((int64_t)rowidx.size() + h.colptr[j + 1]);
-            for (int v : h.rowidx) rowidx.push_back(v + s->sys_row0[i]);
-            val.insert(val.end(), h.val.begin(), h.val.end());
-        }
         DeviceTemp trow, tval;
         HIP_TRY(trow.put(rowidx.data(), rowidx.size()));
         HIP_TRY(tval.put(val.data(), val.size()));
-        rc = fill_plan_values(s, G, colptr.data(), trow.as<int>(), tval.as<double>(), gsrc, fperm);
+        rc = fill_plan_values(s, G, trow.as<int>(), tval.as<double>());
         if (rc != CHOLESPY_OK) return rc;
     }
     dev_free(s->blk_sys);
@@ -1689,7 +1672,6 @@ int cholespy_solver_solve_noalloc(cholespy_gpu_solver *s, int n_rhs, const void 
     const auto region = [](size_t bytes) { return (bytes + 255) & ~size_t(255); };
     const size_t vec = region((size_t)s->n * k * fb), part = region((size_t)s->plan.nslots * k * fb),
                  spart = region((size_t)s->plan.nsplit_rows * k * fb);
-    if (solves_directly(s, b, x, n_rhs, fb)) return solve_blocks(s, n_rhs, b, x, static_cast<hipStream_t>(stream));
     const size_t need = 3 * vec + part + spart;
     if (need > kScratchBytes)
         return fail(CHOLESPY_ERR_INVALID_ARGUMENT,

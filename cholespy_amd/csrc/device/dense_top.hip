@@ -1,32 +1,36 @@
-// The dense top of a solve: z_T = S^{-1} r_T with the explicit inverse of the
-// Schur complement of the top rows, between the forward and the backward
-// pass; or, for a small system, the whole solve x = A^{-1} b in one launch.
+// The dense top of a solve: z_T = X' (X r_T) with X = L_TT^{-1}, the explicit
+// inverse of L's top rows, as one product after the block tasks of the forward
+// pass (y_T = X r_T) and one before those of the backward pass (z_T = X' y_T);
+// or, where every row is a top row, the whole solve in these two launches.
 //
 // Why: near the root of the elimination tree few blocks are left and each of
 // their levels costs three hand-offs between workgroups in the forward pass
 // and two in the backward one (7 us a level and pass, whatever its size),
-// while the inverse of the rows above a cut streams at memory bandwidth. A
-// small system is one product. Measured, block passes alone and with this:
-// k = 3, icosphere(3), n = 642, FP32 41.9 -> 6.9 us; icosphere(5), FP32, a top
-// of 2,640 rows 66 -> 39 us; a vector, 61 x 47 grid, FP64 50.7 -> 13.4 us (its
-// 66 MB inverse at 5 TB/s); k = 128, icosphere(6), FP32, 3,488 rows 342 -> 225
-// us; k = 32, 48^3 grid, FP32, 6,256 rows 460 -> 382 us; k = 3, icosphere(7),
-// FP64, 2,896 rows 163 -> 160 us.
-// choose_dense_top (block_plan.cpp) weighs the two.
+// while a product with X streams at memory bandwidth. choose_dense_top
+// (block_plan.cpp) weighs the two.
 //
-// Rounding: an inverse rounded to FP32 keeps the block passes' accuracy only
-// if its long dot products do not round in FP32 as well (one running FP32 sum
-// lost a factor of 3 to 4): products are summed a few at a time, and those
-// sums in FP64. FP32 solves are then 1.1 to 3 times closer to the exact
-// solution than the block passes' were, FP64 ones within 20 % of them.
+// Why two triangular products and not one with S^{-1} = X' X: that one square
+// is not backward stable, its residual grows with the condition number; the
+// two triangular ones keep the residual of the block passes. ||b - A x|| /
+// ||b||, k = 3, block passes / S^{-1} / X'(X r): 61 x 47 grid, shift 1e-4,
+// FP64 2.9e-16 / 3.6e-15 / 3.4e-16, FP32 1.4e-7 / 7.8e-7 / 9.7e-8; 16^3 grid,
+// kappa 1e6, FP64 3.2e-16 / 1.5e-12 / 1.0e-15. X is sparse where S^{-1} is
+// full (dense_top_plan.hpp), so that the two read less, and are formed in less
+// time: refactorize + solve of a 100 x 60 grid, FP32, 2.37 ms with the values
+// formed on the host and no top, 7.1 with S^{-1}, 1.9 with X; 61 x 47 1.13 /
+// 2.36 / 0.92 ms. The price is a launch: icosphere(3), k = 3, FP32 53 us by
+// the block passes, 6.4 with S^{-1}, 10.4; icosphere(5) 66 / 40 / 44; but
+// icosphere(6), k = 128, FP32 342 / 225 / 202.
 //
-// Layout: S^{-1} (symmetric) in panels of 16 output rows, each contiguous:
-// the entry of output c and input rho is element
-//   (rho / G) * 64 V + ((rho % 4) * 16 + c % 16) * V + (rho % G) / 4
-// of panel c / 16, V = 16 bytes / element size, G = 4 V, inputs padded with
-// zeros to a multiple of 16. One 16-byte load per lane is then the A operand
-// of V successive 16x16x4 MFMA steps, and a panel is one contiguous stream
-// whatever n is.
+// Rounding: products are summed a few at a time, and those sums in FP64 (one
+// running FP32 sum lost a factor of 3 to 4).
+//
+// Layout, per direction: panels of 16 output rows, each contiguous; in a
+// panel, per 16 inputs (a unit), the entry of output c and input rho is element
+//   (rho / G) * 64 V + ((rho % 4) * 16 + c % 16) * V + (rho % G) / 4,
+// V = 16 bytes / element size, G = 4 V, zeros outside X. One 16-byte load per
+// lane is then the A operand of V successive 16x16x4 MFMA steps, and a panel
+// is one contiguous stream whatever its inputs are.
 #include <algorithm>
 
 #include "block_plan.hpp"
@@ -61,43 +65,27 @@ template <> struct Pack<double> {
     static __device__ __forceinline__ int row(int q, int v) { return q + 4 * v; }
 };
 
-// The panel a workgroup starts at, and its system's top.
+// The panel of a workgroup and its system's vectors.
 struct Top {
-    int row0, n, npad, panel, k;
+    int row0, n, panel, first, count, k;
     long long vbase;
     int64_t off;
 };
-// Consecutive workgroups go to different XCDs (round robin over 8): give each
-// XCD a run of consecutive panels, so that what neighbours share stays in one L2.
 __device__ __forceinline__ Top top_of(const DenseTopArgs &a) {
-    const int count = gridDim.x, per = count / 8, extra = count % 8, x = blockIdx.x % 8;
-    const int g = x * per + min(x, extra) + blockIdx.x / 8;
-    Top r;
-    if (!a.tiles) {   // one system: no record to load
-        r.row0 = a.row0;
-        r.n = a.n;
-        r.panel = g;
-        r.k = a.k;
-        r.vbase = 0;
-        r.off = 0;
-    } else {
-        const DenseTopTile t = a.tiles[g];
-        r.row0 = t.row0;
-        r.n = t.n;
-        r.panel = t.panel;
+    const DenseTopPanel t = a.panels[blockIdx.x];
+    Top r{t.row0, t.n, t.panel, t.first, t.count, a.k, 0, t.off};
+    if (a.sys_k) {
         r.k = a.sys_k[t.sys];
         r.vbase = a.sys_vbase[t.sys];
-        r.off = t.off;
     }
-    r.npad = (r.n + 15) / 16 * 16;
-    r.off += (int64_t)r.panel * r.npad * 16;
     return r;
 }
 
-// Output row c, column col: z (read by the backward pass) and row xrow of the solution.
+// Output row c, column col: the work vector (y or z) and row xrow of the solution.
 template <typename F>
 __device__ __forceinline__ void put(const DenseTopArgs &a, const Top &top, int c, int col, int xrow, F v) {
-    if (a.z) static_cast<F *>(a.z)[top.vbase + (long long)(top.row0 + c) * top.k + col] = v;
+    if (a.out) static_cast<F *>(a.out)[top.vbase + (long long)(top.row0 + c) * top.k + col] = v;
+    if (!a.x) return;
     const long long o = top.vbase + (long long)xrow * top.k + col;
     if (a.xmode == 0) {
         static_cast<F *>(a.x)[o] = v;
@@ -106,6 +94,11 @@ __device__ __forceinline__ void put(const DenseTopArgs &a, const Top &top, int c
         x64[o] = (a.xmode == 2 ? x64[o] : 0.0) + (double)v;
     }
 }
+
+// Where a product's inputs are: rows of the top in order from unit `first` on
+// (kRange), the units listed (kList), or, for a whole system's first product,
+// rows of b in the caller's order (kPerm).
+constexpr int kRange = 0, kList = 1, kPerm = 2;
 
 // Bounds-checked loads: a buffer of `bytes` bytes at p (uniform over the
 // wavefront), whose loads past the end return zero without touching memory.
@@ -130,52 +123,68 @@ struct Buffer {
 // the panel's groups of G inputs in turn. A chunk is kFly groups of every
 // wavefront: all its loads are in flight at once, and each register is loaded
 // for the next chunk as soon as it is used, while the next chunk's inputs go
-// to the other LDS buffer. Bound by streaming the panel; the launch's fixed
-// cost is about 4.5 us.
+// to the other LDS buffer. Bound by streaming the panel and, for the many
+// short panels, by the launch and a chain of four memory latencies.
 constexpr int kNarrowThreads = 1024;
 constexpr int kNarrowWaves = kNarrowThreads / kWave;
 constexpr int kFly = 6;
-template <typename F, int KT>
+template <typename F, int KT, int kIn>
 __global__ __launch_bounds__(kNarrowThreads) __attribute__((amdgpu_waves_per_eu(8))) void dense_narrow(DenseTopArgs a) {
     using P = Pack<F>;
     using Vec = typename P::Vec;
     constexpr int V = P::V, G = 4 * V;
     constexpr int kGroups = kFly * kNarrowWaves, kChunk = kGroups * G;
-    constexpr int kIn = kChunk * KT / kNarrowThreads;   // inputs a thread stages per chunk
+    constexpr int kStage = kChunk * KT / kNarrowThreads;   // inputs a thread stages per chunk
+    static_assert(kTopUnit * KT == kWave, "a wavefront stages one unit at a time");
     __shared__ __align__(16) F in[2][kChunk * KT];
     __shared__ double red[kNarrowWaves * 16 * KT];
     const Top top = top_of(a);
     const int k = top.k;
     if (k <= 0) return;
-    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-    const int ng = top.npad / G;
+    const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int ng = top.count * kTopUnit / G;
     constexpr unsigned kVec = sizeof(Vec);
-    const Buffer M(static_cast<const F *>(a.M) + top.off, (unsigned)top.npad * 16 * sizeof(F));
-    const Buffer src(static_cast<const F *>(a.in) + top.vbase + (long long)top.row0 * k,
-                     (unsigned)top.n * (unsigned)k * (unsigned)sizeof(F));
+    const Buffer M(static_cast<const F *>(a.M) + top.off, (unsigned)top.count * kTopUnitEntries * (unsigned)sizeof(F));
+    // Rows of the range that exist, and the inputs up to their end.
+    const int in0 = kIn == kList ? 0 : top.first * kTopUnit;
+    const int end = kIn == kList ? top.n : min(top.n, in0 + top.count * kTopUnit);
+    const Buffer src(static_cast<const F *>(a.in) + (kIn == kPerm ? 0 : top.vbase + (long long)top.row0 * k),
+                     (unsigned)(kIn == kPerm ? a.b_rows : end) * (unsigned)k * (unsigned)sizeof(F));
+    const Buffer rows(kIn == kPerm ? a.rows + top.row0 : nullptr, kIn == kPerm ? (unsigned)end * 4u : 0u);
     const unsigned m0 = (unsigned)tid * kVec;   // this lane's vector of group `wave`
     Vec mv[kFly];
 #pragma unroll
     for (int u = 0; u < kFly; ++u) mv[u] = M.at<Vec>(m0 + u * kNarrowWaves * kWave * kVec);
-    F st[kIn];
+    F st[kStage];
+    const int si = lane / KT, stt = lane % KT;   // row and right-hand side in a unit
+    const unsigned s0 = stt < k ? (unsigned)(si * k + stt) * (unsigned)sizeof(F) : 1u << 31;
     auto load_in = [&](int c0) {
 #pragma unroll
-        for (int q = 0; q < kIn; ++q) {
-            const int i = tid + q * kNarrowThreads, r = c0 + i / KT, t = i % KT;
-            st[q] = src.at<F>(t < k ? (unsigned)(r * k + t) * (unsigned)sizeof(F) : ~0u);
+        for (int q = 0; q < kStage; ++q) {
+            const int unit = c0 / kTopUnit + wave + q * kNarrowWaves;
+            if (kIn == kPerm) {
+                const int r = in0 + unit * kTopUnit + si;
+                const int row = rows.at<int>((unsigned)r * 4u);
+                st[q] = src.at<F>(stt < k && r < end ? (unsigned)(row * k + stt) * (unsigned)sizeof(F) : 1u << 31);
+            } else {
+                // (Units past the end: rows past the end of src.)
+                int r = in0 + unit * kTopUnit;
+                if (kIn == kList) r = unit < top.count ? a.units[top.first + unit] * kTopUnit : end;
+                st[q] = src.at<F>(s0 + (unsigned)(r * k) * (unsigned)sizeof(F));
+            }
         }
     };
     load_in(0);
     // The solution row of this thread's output, needed last.
     const int oc = top.panel * 16 + tid / KT, ot = tid % KT;
     const bool out = tid < 16 * KT && oc < top.n && ot < k;
-    const int xrow = out && a.perm ? a.perm[top.row0 + oc] : top.row0 + oc;
+    const int xrow = out && a.x ? a.perm[top.row0 + oc] : 0;
     double acc[KT];
 #pragma unroll
     for (int t = 0; t < KT; ++t) acc[t] = 0.0;
     for (int g0 = 0, buf = 0; g0 < ng; g0 += kGroups, buf ^= 1) {
 #pragma unroll
-        for (int q = 0; q < kIn; ++q) in[buf][tid + q * kNarrowThreads] = st[q];
+        for (int q = 0; q < kStage; ++q) in[buf][tid + q * kNarrowThreads] = st[q];
         __syncthreads();
         if (g0 + kGroups < ng) load_in((g0 + kGroups) * G);
 #pragma unroll
@@ -213,18 +222,14 @@ __global__ __launch_bounds__(kNarrowThreads) __attribute__((amdgpu_waves_per_eu(
 // More right-hand sides: a workgroup takes a panel and NT tiles of 16
 // right-hand sides, its 8 wavefronts split the inputs and add their partial
 // tiles through LDS. A streams from the panel, B from the input rows (out of
-// the L2: an XCD's workgroups read the same rows), D groups of inputs in
-// flight per wavefront. Bound by the latency of those streams, not by the
-// matrix cores. Two panels a workgroup with one group in flight and B loaded a
-// value at a time, against this: icosphere(6), k = 128, FP32 (top 3,488) 65 ->
-// 50 us, 511 x 389 grid, k = 17, FP64 (top 2,048) 39 -> 18 us, 48^3 grid,
-// k = 32, FP32 (top 6,256) 62 -> 56 us, a batch of 64 systems, k = 1 to 128,
-// FP32 159 -> 111 us; 33^3 grid, k = 5, FP64 (top 4,512) 63 -> 51 us. 16
-// wavefronts a workgroup measured the same.
+// the L2), D groups of inputs in flight per wavefront. Bound by the latency of
+// those streams, not by the matrix cores.
 constexpr int kWideThreads = 512;
 constexpr int kWideWaves = kWideThreads / kWave;
 constexpr int kOneTileFly = 5;   // D of one tile
-template <typename F, int NT, int D>
+// (A wavefront's groups, with those asked for ahead, fit two registers a lane.)
+static_assert(kTopMaxRows / (Pack<double>::V * 4 * kWideWaves) + 2 * kOneTileFly - 2 < 2 * kWave, "kTopMaxRows");
+template <typename F, int NT, int D, int kIn>
 __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top, int t0, double (*red)[kWave * 4]) {
     using P = Pack<F>;
     using Vec = typename P::Vec;
@@ -233,10 +238,27 @@ __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top
     const int k = top.k;
     const int lane = threadIdx.x % kWave, q = lane / 16, l = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const Buffer M(static_cast<const F *>(a.M) + top.off, (unsigned)top.npad * 16 * (unsigned)sizeof(F));
+    const Buffer M(static_cast<const F *>(a.M) + top.off, (unsigned)top.count * kTopUnitEntries * (unsigned)sizeof(F));
+    const int in0 = kIn == kList ? 0 : top.first * kTopUnit;
+    const int end = kIn == kList ? top.n : min(top.n, in0 + top.count * kTopUnit);
     const Buffer src(static_cast<const F *>(a.in) + top.vbase + (long long)top.row0 * k,
-                     (unsigned)top.n * (unsigned)k * (unsigned)sizeof(F));
-    const int ng = top.npad / G;
+                     (unsigned)end * (unsigned)k * (unsigned)sizeof(F));
+    const int ng = top.count * kTopUnit / G;
+    // First input row of this wavefront's i-th group (wave + 8 i): from the
+    // unit list held one entry a lane, or counted on. Past the last group: past
+    // the end of src.
+    int li[2];
+    if (kIn == kList)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int r = (wave + (lane + h * kWave) * kWideWaves) * G, unit = r / kTopUnit;
+            li[h] = unit < top.count ? a.units[top.first + unit] * kTopUnit + r % kTopUnit : top.n;
+        }
+    auto first_row = [&](int i) {
+        if (kIn == kRange) return in0 + (wave + i * kWideWaves) * G;
+        const int r0 = __builtin_amdgcn_readlane(li[0], i % kWave), r1 = __builtin_amdgcn_readlane(li[1], i % kWave);
+        return i < kWave ? r0 : r1;
+    };
     Vec m[D];
     // B of tile n, lane column l: right-hand side col0 + n, so that a lane's
     // tiles are one load of NT consecutive values. Lanes past the row's end
@@ -248,12 +270,13 @@ __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top
     F b[D][V][NT];
     constexpr int kPer = NT * (int)sizeof(F) <= 16 ? NT : 16 / (int)sizeof(F);   // values per load
     typedef F BVec __attribute__((ext_vector_type(kPer)));
-    auto load = [&](int d, int g) {
+    auto load = [&](int d, int i) {
         // (Groups past the end are past the end of both buffers: zero.)
-        m[d] = M.at<Vec>((unsigned)(g * kWave + lane) * (unsigned)sizeof(Vec));
+        m[d] = M.at<Vec>((unsigned)((wave + i * kWideWaves) * kWave + lane) * (unsigned)sizeof(Vec));
+        const int row = first_row(i);
 #pragma unroll
         for (int j = 0; j < V; ++j) {
-            const unsigned at = b0 + (unsigned)((g * G + 4 * j) * k) * (unsigned)sizeof(F);
+            const unsigned at = b0 + (unsigned)((row + 4 * j) * k) * (unsigned)sizeof(F);
 #pragma unroll
             for (int n = 0; n < NT; n += kPer) {
                 if constexpr (kPer == 1) {
@@ -268,11 +291,11 @@ __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top
     };
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-        load(d, wave + d * kWideWaves);
+        load(d, d);
         __builtin_amdgcn_sched_barrier(0);
     }
     double sum[NT][4] = {};
-    for (int g0 = wave; g0 < ng; g0 += D * kWideWaves) {
+    for (int i = 0; wave + i * kWideWaves < ng; i += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             // Two steps (8 products an entry) at a time, summed in FP64.
@@ -287,7 +310,7 @@ __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top
             // (The scheduler would gather the D loads at the loop's end, and
             // its head would wait for all of them.)
             __builtin_amdgcn_sched_barrier(0);
-            load(d, g0 + (D + d) * kWideWaves);
+            load(d, i + D + d);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -314,11 +337,11 @@ __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top
         double s = 0.0;
 #pragma unroll
         for (int w = 0; w < kHalf; ++w) s += red[w * NT + n][e];
-        if (c < top.n && col < k && col >= t0 + NT * l) put(a, top, c, col, a.perm ? a.perm[top.row0 + c] : top.row0 + c, (F)s);
+        if (c < top.n && col < k && col >= t0 + NT * l) put(a, top, c, col, a.x ? a.perm[top.row0 + c] : 0, (F)s);
     }
 }
 
-template <typename F, int NT, int D>
+template <typename F, int NT, int D, int kIn>
 __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(4))) void dense_wide(DenseTopArgs a) {
     __shared__ double red[kWideWaves / 2 * NT][kWave * 4];
     const Top top = top_of(a);
@@ -326,44 +349,52 @@ __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(4)
     if (t0 >= top.k) return;
     // A rest of one tile: a batch's systems differ in their right-hand sides.
     if (NT > 1 && top.k - t0 <= 16)
-        wide_tiles<F, 1, kOneTileFly>(a, top, t0, red);
+        wide_tiles<F, 1, kOneTileFly, kIn>(a, top, t0, red);
     else
-        wide_tiles<F, NT, D>(a, top, t0, red);
+        wide_tiles<F, NT, D, kIn>(a, top, t0, red);
 }
 
-__global__ void copy_words(uint32_t *dst, const uint32_t *src, size_t count) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < count; i += (size_t)gridDim.x * blockDim.x)
-        dst[i] = src[i];
+// dst row i = src row rows[i], k columns.
+template <typename F>
+__global__ void gather_rows_of(F *dst, const F *src, const int *rows, int n, int k) {
+    const size_t total = (size_t)n * k;
+    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x)
+        dst[e] = src[(size_t)rows[e / k] * k + e % k];
 }
 
 }  // namespace
 
-hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream) {
-    const size_t count = bytes / 4;
-    if (count == 0) return hipSuccess;
-    copy_words<<<dim3((unsigned)std::min<size_t>((count + 255) / 256, 4096)), 256, 0, stream>>>(
-        static_cast<uint32_t *>(dst), static_cast<const uint32_t *>(src), count);
+hipError_t launch_gather_rows(int float_bytes, void *dst, const void *src, const int *rows, int n, int k, hipStream_t stream) {
+    const size_t total = (size_t)n * k;
+    if (total == 0) return hipSuccess;
+    const dim3 grid((unsigned)std::min<size_t>((total + 255) / 256, 4096));
+    if (float_bytes == 4)
+        gather_rows_of<float><<<grid, 256, 0, stream>>>(static_cast<float *>(dst), static_cast<const float *>(src), rows, n, k);
+    else
+        gather_rows_of<double><<<grid, 256, 0, stream>>>(static_cast<double *>(dst), static_cast<const double *>(src), rows, n, k);
     return hipGetLastError();
 }
 
-hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int tiles, int max_k,
-                            hipStream_t stream) {
+template <typename F>
+static const void *dense_kernel(const DenseTopArgs &a, int max_k) {
+    if (max_k <= kNarrowTile)
+        return a.units  ? reinterpret_cast<const void *>(&dense_narrow<F, kNarrowTile, kList>)
+               : a.rows ? reinterpret_cast<const void *>(&dense_narrow<F, kNarrowTile, kPerm>)
+                        : reinterpret_cast<const void *>(&dense_narrow<F, kNarrowTile, kRange>);
+#define CHOLESPY_DENSE(NT, D)                                                 \
+    (a.units ? reinterpret_cast<const void *>(&dense_wide<F, NT, D, kList>)   \
+             : reinterpret_cast<const void *>(&dense_wide<F, NT, D, kRange>))
+    return max_k <= 16 ? CHOLESPY_DENSE(1, kOneTileFly) : max_k <= 32 ? CHOLESPY_DENSE(2, 3) : CHOLESPY_DENSE(4, 2);
+#undef CHOLESPY_DENSE
+}
+
+hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int panels, int max_k, hipStream_t stream) {
     DenseTopArgs a = args;
     void *p[] = {&a};
-    const void *kern;
-    if (max_k <= kNarrowTile) {
-        kern = float_bytes == 4 ? reinterpret_cast<const void *>(&dense_narrow<float, kNarrowTile>)
-                                : reinterpret_cast<const void *>(&dense_narrow<double, kNarrowTile>);
-        return hipLaunchKernel(kern, dim3(tiles), dim3(kNarrowThreads), p, 0, stream);
-    }
+    const void *kern = float_bytes == 4 ? dense_kernel<float>(a, max_k) : dense_kernel<double>(a, max_k);
+    if (max_k <= kNarrowTile) return hipLaunchKernel(kern, dim3(panels), dim3(kNarrowThreads), p, 0, stream);
     const int nt = max_k <= 16 ? 1 : (max_k <= 32 ? 2 : 4);
-#define CHOLESPY_DENSE(F)                                                    \
-    (nt == 1   ? reinterpret_cast<const void *>(&dense_wide<F, 1, kOneTileFly>) \
-     : nt == 2 ? reinterpret_cast<const void *>(&dense_wide<F, 2, 3>)        \
-               : reinterpret_cast<const void *>(&dense_wide<F, 4, 2>))
-    kern = float_bytes == 4 ? CHOLESPY_DENSE(float) : CHOLESPY_DENSE(double);
-#undef CHOLESPY_DENSE
-    return hipLaunchKernel(kern, dim3(tiles, (max_k + 16 * nt - 1) / (16 * nt)), dim3(kWideThreads), p, 0, stream);
+    return hipLaunchKernel(kern, dim3(panels, (max_k + 16 * nt - 1) / (16 * nt)), dim3(kWideThreads), p, 0, stream);
 }
 
 }  // namespace cholespy_amd

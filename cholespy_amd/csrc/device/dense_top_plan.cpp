@@ -1,0 +1,107 @@
+#include "dense_top_plan.hpp"
+
+#include <algorithm>
+
+namespace cholespy_amd {
+
+TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
+    TopLists L;
+    std::vector<int> pack_bwd;
+    int64_t fwd_units = 0, bwd_units = 0;
+    // The jobs of all blocks, by stage.
+    struct Pending {
+        TopLists::Job job;
+        int stage;
+    };
+    std::vector<Pending> pending;
+    std::vector<int> temps_of_stage;
+    for (const BlockPlan::TopBlock &top : P.tops) {
+        const int row0 = P.start[top.block], m = (int)top.parent.size(), sys = blk_sys ? (*blk_sys)[top.block] : 0;
+        const int np = (m + kTopUnit - 1) / kTopUnit, nt = (m + kTopTile - 1) / kTopTile, per = kTopTile / kTopUnit;
+        // has[p * np + q]: unit (p, q) of X holds a pair of an ancestor and its descendant.
+        std::vector<char> has((size_t)np * np, 0);
+        // (An ancestor among the same 16 columns marks the rest of the path.)
+        for (int j = 0; j < m; ++j)
+            for (int i = j; i >= 0; i = top.parent[i]) {
+                has[(size_t)(i / kTopUnit) * np + j / kTopUnit] = 1;
+                if (i > j && i / kTopUnit == j / kTopUnit) break;
+            }
+        std::vector<int> tile((size_t)nt * nt, -1);
+        for (int p = 0; p < np; ++p)
+            for (int q = 0; q <= p; ++q)
+                if (has[(size_t)p * np + q]) {
+                    int &t = tile[(size_t)(p / per) * nt + q / per];
+                    if (t < 0) t = L.tiles++;
+                }
+        const int map = (int)L.map.size();
+        L.map.push_back(nt);
+        L.map.insert(L.map.end(), tile.begin(), tile.end());
+        for (int c = 0; c < m; ++c) L.columns.push_back({c, row0, map});
+        auto code = [&](int p, int q) {
+            const int t = tile[(size_t)(p / per) * nt + q / per];
+            return t < 0 ? -1 : t * per * per + p % per * per + q % per;
+        };
+        // Panels. A row's descendants are consecutive under a postorder; any
+        // other numbering keeps the whole range from the lowest one on.
+        for (int p = 0; p < np; ++p) {
+            int lo = 0;
+            while (!has[(size_t)p * np + lo]) ++lo;
+            L.fwd.push_back({row0, m, p, sys, lo, p - lo + 1, fwd_units * kTopUnitEntries});
+            for (int q = lo; q <= p; ++q) L.pack.push_back(code(p, q));
+            fwd_units += p - lo + 1;
+            const int first = (int)L.units.size();
+            for (int r = p; r < np; ++r)
+                if (has[(size_t)r * np + p]) {
+                    L.units.push_back(r);
+                    pack_bwd.push_back(code(r, p));
+                }
+            const int count = (int)L.units.size() - first;
+            L.bwd.push_back({row0, m, p, sys, first, count, bwd_units * kTopUnitEntries});
+            bwd_units += count;
+        }
+        // Stages 2 s' (into temporaries) and 2 s' + 1 (back) of doubling s'.
+        for (int i = 0; i < nt; ++i) L.diagonals.push_back({tile[(size_t)i * nt + i], std::min(kTopTile, m - i * kTopTile)});
+        int stage = 0;
+        for (int s = 1; s < nt; s *= 2, stage += 2) {
+            if ((int)temps_of_stage.size() <= stage) temps_of_stage.resize((size_t)stage + 2, 0);
+            std::vector<int> temp((size_t)nt * nt, -1);
+            for (int half = 0; half < 2; ++half)
+                for (int g = 0; g + s < nt; g += 2 * s)
+                    for (int i = g + s; i < std::min(nt, g + 2 * s); ++i)
+                        for (int j = g; j < g + s; ++j) {
+                            const int out = tile[(size_t)i * nt + j];
+                            if (out < 0) continue;
+                            TopLists::Job job{out, (int)L.pairs.size(), 0};
+                            if (half == 0) job.out = temp[(size_t)i * nt + j] = temps_of_stage[(size_t)stage]++;
+                            const int k0 = half == 0 ? j : g + s, k1 = half == 0 ? g + s : i + 1;
+                            for (int k = k0; k < k1; ++k) {
+                                const int a = tile[(size_t)i * nt + k];
+                                const int b = half == 0 ? tile[(size_t)k * nt + j] : temp[(size_t)k * nt + j];
+                                if (a >= 0 && b >= 0) L.pairs.push_back({a, b});
+                            }
+                            job.count = (int)L.pairs.size() - job.first;
+                            pending.push_back({job, stage + half});
+                        }
+        }
+    }
+    L.entries = std::max(fwd_units, bwd_units) * kTopUnitEntries;
+    L.pack.resize((size_t)std::max(fwd_units, bwd_units), -1);
+    pack_bwd.resize(L.pack.size(), -1);
+    L.pack.insert(L.pack.end(), pack_bwd.begin(), pack_bwd.end());
+    auto longest = [](const DenseTopPanel &a, const DenseTopPanel &b) { return a.count > b.count; };
+    std::stable_sort(L.fwd.begin(), L.fwd.end(), longest);
+    std::stable_sort(L.bwd.begin(), L.bwd.end(), longest);
+    std::stable_sort(pending.begin(), pending.end(), [](const Pending &a, const Pending &b) {
+        return a.stage != b.stage ? a.stage < b.stage : a.job.count > b.job.count;
+    });
+    for (int t : temps_of_stage) L.temps = std::max(L.temps, t);
+    L.stages.assign(1, 0);
+    for (const Pending &q : pending) {
+        while ((int)L.stages.size() <= q.stage) L.stages.push_back((int)L.jobs.size());
+        L.jobs.push_back(q.job);
+    }
+    L.stages.push_back((int)L.jobs.size());
+    return L;
+}
+
+}  // namespace cholespy_amd

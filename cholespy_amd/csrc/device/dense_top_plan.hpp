@@ -1,0 +1,69 @@
+// Lists for the dense top blocks of a plan (host side): the panels of the two
+// products with X = L_TT^{-1} (dense_top.hip) and the tile products that form
+// X (block_inverse.hip).
+//
+// X_ij is nonzero only where row i is an ancestor of row j (or j itself) in
+// the elimination tree, so X is stored in the 16 x 16 units that hold such a
+// pair: 2,122 units of 16,290 for a 61 x 47 grid, 9,076 of 23,871 for the top
+// of icosphere(6), 55,732 of 76,636 for that of a 48^3 grid.
+#pragma once
+#include <cstdint>
+#include <vector>
+
+#include "block_plan.hpp"
+
+namespace cholespy_amd {
+
+constexpr int kTopUnit = 16;                          // rows and columns of a unit
+constexpr int kTopUnitEntries = kTopUnit * kTopUnit;
+constexpr int kTopTile = 64;                          // rows and columns of a tile of X while it is formed
+constexpr int kTopTileEntries = kTopTile * kTopTile;
+
+// One panel of 16 outputs of a product: count input units from unit `first`
+// on (w = X r: consecutive units of 16 rows), or those listed from position
+// `first` of TopLists::units on (z = X' w). Device record.
+struct DenseTopPanel {
+    int row0, n;      // first row of the top block and its rows
+    int panel, sys;
+    int first, count;
+    int64_t off;      // first element in the direction's array
+};
+
+struct TopLists {
+    std::vector<DenseTopPanel> fwd, bwd;   // longest first: the last workgroups to start are the short ones
+    std::vector<int> units;
+    int64_t entries = 0;                   // elements of one direction's array
+
+    // Forming X. A block is a square of 64 x 64 tiles, of which those with an
+    // ancestor pair exist; tile t is the kTopTileEntries column-major values
+    // at t. They start as L and become X in place: the diagonal tiles are
+    // inverted, then inverses of doubled size, X_21 = -X_22 (L_21 X_11), in
+    // stages of independent jobs: into temporary tiles (L_21 X_11), then back.
+    struct Column {
+        int c, row0, map;          // column c of the block from row0, its tile map at map
+    };
+    struct Diagonal {
+        int tile, rows;
+    };
+    struct Job {
+        int out, first, count;     // pairs [first, first + count); out: temporary tile (even stages) or tile (odd)
+    };
+    struct Pair {
+        int a, b;                  // even: tile, tile; odd: tile, temporary tile
+    };
+    int tiles = 0, temps = 0;
+    std::vector<Column> columns;
+    std::vector<int> map;          // per block: tiles across, then the tile of (i, j) at i * across + j, -1 = none
+    std::vector<Diagonal> diagonals;
+    std::vector<Job> jobs;
+    std::vector<Pair> pairs;
+    std::vector<int> stages;       // job ranges: stage s is [stages[s], stages[s + 1])
+    // Per unit of the fwd and then of the bwd array: tile * 16 + unit row in
+    // it * 4 + unit column (-1: no such tile, zeros).
+    std::vector<int> pack;
+};
+
+// blk_sys: the system of each block (null: one system).
+TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys);
+
+}  // namespace cholespy_amd

@@ -4,6 +4,7 @@
 #include <string>
 #include <vector>
 #include <hip/hip_runtime.h>
+#include "dense_top_plan.hpp"
 #include <stddef.h>
 #include <stdint.h>
 
@@ -142,27 +143,24 @@ const void *block_pass_kernel(int float_bytes, bool forward, int tile);
 hipError_t launch_block_pass(int float_bytes, bool forward, const BlockPassBuffers &buf, int grid,
                              QueueState &queues, hipStream_t stream);
 
-// Dense top blocks (dense_top.hip): z_T = S^{-1} r_T. One record per panel of
-// 16 outputs.
-struct DenseTopTile {
-    int row0, n;     // first row of the top block and its rows
-    int panel, sys;
-    int64_t off;     // the inverse's first element
-};
+// The two products of the dense top blocks (dense_top.hip), one workgroup per
+// panel (dense_top_plan.hpp): out = X in (units null) or out, x = X' in.
 struct DenseTopArgs {
-    const DenseTopTile *tiles;     // null: one system, whose top is the n rows from row0
-    int row0, n;
-    const void *M, *in;            // the inverses; r_T at rows row0.. of `in`
-    void *z, *x;                   // z may be null
-    const int *perm;               // solution row of each row; null: the row itself
+    const DenseTopPanel *panels;
+    const int *units;              // input units of X' (null: X)
+    const int *rows;               // first product of a whole system, up to 4 right-hand sides: `in` is b, whose
+    int b_rows;                    // row rows[r] (of b_rows) is plan row r; null: `in` is in plan order
+    const void *M, *in;
+    void *out, *x;                 // plan order (null: not stored); the solution (null: not stored)
+    const int *perm;               // solution row of each plan row
     int k, xmode;                  // xmode as in BlockPassBuffers
     const int *sys_k;              // batches (null for a single system)
     const long long *sys_vbase;
 };
-hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int tiles, int max_k,
-                            hipStream_t stream);
-// bytes (a multiple of 4) from src to dst, device to device, as a kernel.
-hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream);
+hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int panels, int max_k, hipStream_t stream);
+// dst row i := src row rows[i] (n rows of k values).
+hipError_t launch_gather_rows(int float_bytes, void *dst, const void *src, const int *rows, int n, int k,
+                              hipStream_t stream);
 
 // Mixed-precision refinement helpers (refine.hip).
 hipError_t launch_cast_to_f32(const double *in, float *out, size_t count, hipStream_t stream);

@@ -400,8 +400,8 @@ __global__ __launch_bounds__(kTaskThreads) void block_forward(BlockPassArgs<F> a
         }
         for (int t0 = 0; t0 < k; t0 += KT) {
             const int kt = min(KT, k - t0);
-            if (kind == 1 || kind == 4) {   // gather-only task: rows [first, last) of r_B to rbuf (top: y)
-                gather_partials(a, bv, pv, kind == 4 ? yv : rb, (F *)nullptr, a0, first, last, t0, kt, k, KT, KT, true);
+            if (kind == 1 || kind == 4) {   // gather-only task: rows [first, last) of r_B to rbuf (top: z)
+                gather_partials(a, bv, pv, kind == 4 ? zv : rb, (F *)nullptr, a0, first, last, t0, kt, k, KT, KT, true);
                 if (a.trace && tid == 0 && t0 == 0) a.trace[4 * (size_t)tk + 1] = wall_clock64();
                 continue;
             }

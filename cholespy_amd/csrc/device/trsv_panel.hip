@@ -678,8 +678,8 @@ void block_forward_panel(BlockPassArgs<F> a) {
         };
         const int nsp = split_count(task.nsplit), sidx = split_index(task.nsplit);
         const int srow = task.sbase + sidx * (last - first) - first;
-        if (kind == 1 || kind == 4) {   // gather-only task: rows [first, last) of r_B to rbuf (top: y)
-            gather_wide(a, stage, bv, pv, kind == 4 ? yv : rb, (F *)nullptr, a0, first, last, k, k, true);
+        if (kind == 1 || kind == 4) {   // gather-only task: rows [first, last) of r_B to rbuf (top: z)
+            gather_wide(a, stage, bv, pv, kind == 4 ? zv : rb, (F *)nullptr, a0, first, last, k, k, true);
             if (a.trace && tid == 0) a.trace[4 * (size_t)tk + 1] = wall_clock64();
         } else if (k > 0) {
             const int nT = (k + 15) / 16;

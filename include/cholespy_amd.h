@@ -269,7 +269,7 @@ int cholespy_probe_handoff(double *results, int count);
 int cholespy_solver_tune_report(const cholespy_gpu_solver *solver, char *report, size_t report_len);
 
 /* Block-plan statistics: info[0..count) = {blocks, dense entries of all
- * M_B (of a dense top, whose square inverse serves both passes, half),
+ * M_B and of a dense top's inverse (what one pass reads),
  * forward block levels, backward block levels, forward tasks, backward tasks,
  * partial slots, largest m + |R|, forward tasks and backward tasks of the
  * wide right-hand-side list}. No counterpart in the reference. */
