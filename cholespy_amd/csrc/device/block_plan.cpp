@@ -285,7 +285,7 @@ int automatic_max_block(int n, const std::vector<int> &parent) {
 
 // Block starts (then n): small whole subtrees, then chains (j and j + 1 share
 // a block when parent(j) = j + 1), capped at max_block; the last top_rows
-// rows are one block.
+// rows are one block per tree (trees one after another, each ending at its root).
 std::vector<int> partition_rows(int n, const std::vector<int> &parent, const std::vector<int> &size,
                                 const BlockPlanOptions &opt) {
     const int end = n - std::min(n, opt.top_rows);
@@ -309,7 +309,10 @@ std::vector<int> partition_rows(int n, const std::vector<int> &parent, const std
         while (e + 1 < end && parent[e] == e + 1 && e + 1 - j + 1 <= max_block) ++e;
         j = e + 1;
     }
-    if (end < n) start.push_back(end);
+    for (int t = end; t < n; ++t) {
+        start.push_back(t);
+        while (t + 1 < n && parent[t] >= 0) ++t;
+    }
     start.push_back(n);
     return start;
 }
@@ -543,21 +546,29 @@ DenseTop choose_dense_top(int n, const int *colptr, const int *rowidx, const Blo
         if (p >= 0) level[block_of[p]] = std::max(level[block_of[p]], level[b] + 1);
         levels = std::max(levels, level[b] + 1);
     }
-    // Per row: its ancestors with itself (the entries of its column of X:
-    // every ancestor of a top row is one too).
-    std::vector<int> depth((size_t)n);
-    for (int j = n - 1; j >= 0; --j) depth[j] = parent[j] < 0 ? 1 : depth[parent[j]] + 1;
-    // Per level: the rows of the blocks from it up and the entries of their X,
-    // and the entries of its own M_B.
-    std::vector<int64_t> rows((size_t)levels + 1, 0), inverse((size_t)levels + 1, 0), entries((size_t)levels, 0);
+    // Per row: its tree's root, and its ancestors with itself (the entries of
+    // its column of X: every ancestor of a top row is one too).
+    std::vector<int> root((size_t)n), depth((size_t)n);
+    for (int j = n - 1; j >= 0; --j) {
+        root[j] = parent[j] < 0 ? j : root[parent[j]];
+        depth[j] = parent[j] < 0 ? 1 : depth[parent[j]] + 1;
+    }
+    // Per level: the rows of the blocks from it up, their trees and the
+    // entries of their X, and the entries of its own M_B.
+    std::vector<int64_t> rows((size_t)levels + 1, 0), trees((size_t)levels + 1, 0), inverse((size_t)levels + 1, 0),
+        entries((size_t)levels, 0);
     for (int b = 0; b < nb; ++b) {
         const int64_t m = start[b + 1] - start[b], below = colptr[start[b + 1]] - colptr[start[b + 1] - 1] - 1;
         rows[level[b]] += m;
         entries[level[b]] += m * (m + 1) / 2 + m * below;   // (|R| >= the last column's rows below)
-        for (int i = start[b]; i < start[b + 1]; ++i) inverse[level[b]] += depth[i];
+        for (int i = start[b]; i < start[b + 1]; ++i) {
+            trees[level[b]] += parent[i] < 0;
+            inverse[level[b]] += depth[i];
+        }
     }
     for (int l = levels - 1; l >= 0; --l) {
         rows[l] += rows[l + 1];
+        trees[l] += trees[l + 1];
         inverse[l] += inverse[l + 1];
     }
     double passes = opt.pass_us;
@@ -565,7 +576,7 @@ DenseTop choose_dense_top(int n, const int *colptr, const int *rowidx, const Blo
     int cut = levels;
     double best = opt.top_forced ? std::numeric_limits<double>::infinity() : passes;
     const int64_t most = std::min<int64_t>(opt.top_max_rows, kTopMaxRows);
-    for (int l = levels - 1; l >= 0 && rows[l] <= most; --l) {
+    for (int l = levels - 1; l >= 0 && rows[l] <= most && trees[l] <= kTopMaxTrees; --l) {
         passes -= 2.0 * (opt.level_us + (double)entries[l] * float_bytes / opt.level_gbs * 1e-3);
         // X is stored twice, in 16 x 16 units: about 48 more entries a row than it has.
         const double stored = 2.0 * ((double)inverse[l] + 48.0 * (double)rows[l]);
@@ -582,6 +593,7 @@ DenseTop choose_dense_top(int n, const int *colptr, const int *rowidx, const Blo
         for (int b = 0; b < nb; ++b)
             if ((level[b] >= cut) == (pass == 1))
                 for (int i = start[b]; i < start[b + 1]; ++i) top.src.push_back(i);
+    std::stable_sort(top.src.end() - top.rows, top.src.end(), [&](int i, int j) { return root[i] < root[j]; });
     return top;
 }
 

@@ -89,9 +89,10 @@ struct BlockPlanOptions {
     // schedule.
     bool critical_order = true;
     // Rows of the dense top: the last top_rows rows of the factor (an
-    // ancestor-closed set: see choose_dense_top), one block, solved with the
-    // explicit inverse X of L's part between the two passes. 0 = none. The
-    // host fill does not form its values.
+    // ancestor-closed set: see choose_dense_top), one block per tree of the
+    // elimination forest among them, solved with the explicit inverse X of
+    // L's part between the two passes. 0 = none. The host fill does not form
+    // its values.
     int top_rows = 0;
     // What choose_dense_top weighs, in microseconds and GB/s: the two passes'
     // launches and leaf tasks, a level of a pass (its hand-offs, and its M_B
@@ -157,7 +158,7 @@ struct BlockPlan {
     // BlockPlanOptions' wide_* shape), leaf tasks first and last as well.
     std::vector<int> fwd_task_wide, bwd_task_wide;
     int n_leaf_fwd_wide = 0, n_leaf_bwd_wide = 0;
-    // Dense top blocks (none, or one per system). They have no
+    // Dense top blocks (none, or one per tree of a system's top). They have no
     // entries in mfwd / mbwd, no R rows and no backward tasks; their forward
     // tasks are gathers (kind 4) that leave r_B in z, for the products of
     // dense_top.hip. parent: the elimination tree among the block's rows
@@ -190,11 +191,14 @@ void fill_block_plan_values(BlockPlan &P, const int *colptr, const int *rowidx, 
 // The most rows of a dense top (dense_top.hip keeps a wavefront's input units
 // in two registers of a row).
 constexpr int kTopMaxRows = 7168;
+// The most trees a dense top may hold: each is a block with panels of its own.
+constexpr int kTopMaxTrees = 64;
 
 // The rows that are worth solving by an explicit inverse, and a numbering
 // that puts them last. src[r] = factor row at plan row r (the other rows keep
-// their order, then the top rows in order: a topological order of the
-// elimination tree, so L keeps its pattern under it); empty src: no top block. Blocks at forward level >= cut (in the partition that
+// their order, then the top rows tree by tree, each in order: a topological
+// order of the elimination forest, so L keeps its pattern under it); empty
+// src: no top block. Blocks at forward level >= cut (in the partition that
 // `opt` gives) are the top rows; the cut minimises the estimated time of the
 // levels below it and of the products with the inverse.
 struct DenseTop {

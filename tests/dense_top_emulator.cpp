@@ -9,7 +9,9 @@
 //     its block or array, or the panels do not cover the top's rows once;
 //   - the leaf tasks (of either list) do not fit the leaf kernels, do not come
 //     first (forward) and last (backward), or receive partial sums;
-//   - a top block has a backward task or a forward task that is no gather.
+//   - a top block has a backward task or a forward task that is no gather;
+//   - a NaN in the right-hand side of one tree of the elimination forest
+//     reaches the solution of another.
 //
 // Usage: dense_top_emulator FILE narrow|wide ROWS SHUFFLE
 // FILE as in plan_emulator.cpp; ROWS: the most rows of the top, whose levels
@@ -204,7 +206,7 @@ void check_leaves(const BlockPlan &P, const std::vector<int> &fwd, const std::ve
 }
 
 std::vector<double> solve(const BlockPlan &P, const TopLists &L, const std::vector<double> &xf, const std::vector<double> &xb,
-                          bool wide, const std::vector<double> &b) {
+                          bool wide, const std::vector<double> &b, bool nans) {
     const std::vector<int> &ft = wide ? P.fwd_task_wide : P.fwd_task, &bt = wide ? P.bwd_task_wide : P.bwd_task;
     std::vector<double> y((size_t)P.n, NAN), z((size_t)P.n, NAN), rbuf((size_t)P.n, NAN), part(P.rlist.size(), NAN),
         split((size_t)std::max(1, P.nsplit_rows), NAN);
@@ -279,7 +281,7 @@ std::vector<double> solve(const BlockPlan &P, const TopLists &L, const std::vect
                 zset[(size_t)a0 + first + i] = 1;
             }
     }
-    for (int i = 0; i < P.n; ++i) check(zset[i] && !std::isnan(z[i]), "a row of the solution is missing");
+    for (int i = 0; i < P.n; ++i) check(zset[i] && (nans || !std::isnan(z[i])), "a row of the solution is missing");
     return z;
 }
 
@@ -335,7 +337,7 @@ int run(const char *path, bool wide, int most, bool shuffle) {
         for (int p = f.cp[j] + 1; p < f.cp[j + 1]; ++p) ref[j] -= f.v[p] * ref[f.ri[p]];
         ref[j] /= f.v[f.cp[j]];
     }
-    const std::vector<double> z = solve(P, L, xf, xb, wide, b);
+    const std::vector<double> z = solve(P, L, xf, xb, wide, b, false);
     double err = 0.0, scale = 0.0;
     for (int i = 0; i < f.n; ++i) {
         err = std::max(err, std::fabs(z[i] - ref[i]));
@@ -343,8 +345,21 @@ int run(const char *path, bool wide, int most, bool shuffle) {
     }
     check(err <= 1e-10 * scale, "the solution differs from the sequential solve");
 
-    std::printf("ok n %d top %d in %zu blocks of %d, panels %zu units %lld tiles %d temps %d stages %zu err %.1e\n", f.n,
-                top.rows, P.tops.size(), P.nblocks, L.fwd.size(), (long long)(L.entries / kTopUnitEntries), L.tiles,
+    // One tree's right-hand side NaN: the other trees' solutions stay as they were.
+    std::vector<int> root((size_t)f.n);
+    std::set<int> trees;
+    for (int j = f.n - 1; j >= 0; --j) {
+        root[j] = f.cp[j + 1] - f.cp[j] > 1 ? root[f.ri[f.cp[j] + 1]] : j;
+        trees.insert(root[j]);
+    }
+    std::vector<double> bn = b;
+    for (int j = 0; j < f.n; ++j)
+        if (root[j] == root[f.n - 1]) bn[j] = NAN;
+    const std::vector<double> zn = solve(P, L, xf, xb, wide, bn, true);
+    for (int j = 0; j < f.n; ++j)
+        check(root[j] == root[f.n - 1] ? std::isnan(zn[j]) : zn[j] == z[j], "a NaN reaches another tree");
+    std::printf("ok n %d top %d in %zu blocks of %d, trees %zu, panels %zu units %lld tiles %d temps %d stages %zu err %.1e\n", f.n,
+                top.rows, P.tops.size(), P.nblocks, trees.size(), L.fwd.size(), (long long)(L.entries / kTopUnitEntries), L.tiles,
                 L.temps, L.stages.size() - 1, err / scale);
     return 0;
 }

@@ -85,3 +85,11 @@ def test_inverse_is_stored_where_it_is_nonzero(factors, emulator):
     """A 61 x 47 grid as one top: a dense square would take 180 x 180 units."""
     res = subprocess.run([str(emulator), str(factors["grid61x47"]), "narrow", "7168", "0"], capture_output=True, text=True)
     assert "top 2867" in res.stdout and " units 2122 tiles 264 " in res.stdout, res.stdout
+
+
+def test_forest_top_has_a_block_per_tree(factors, emulator):
+    res = subprocess.run([str(emulator), str(factors["forest"]), "narrow", "7168", "0"], capture_output=True, text=True)
+    assert "in 6 blocks of 6, trees 6" in res.stdout, res.stdout
+    # Too many trees for a top of all rows: fewer levels, or none.
+    res = subprocess.run([str(emulator), str(factors["dust"]), "narrow", "7168", "0"], capture_output=True, text=True)
+    assert "ok" in res.stdout and "top 470" not in res.stdout, res.stdout
