@@ -86,10 +86,15 @@ template <typename F, int NT, bool Forward> constexpr int batch_steps() {
 // (3 waves), 116 backward (4). FP32, up to 4 tiles: 4 waves forward, 5
 // backward. FP64 forward with up to 4 tiles: 3 waves (left alone the compiler
 // takes AGPRs and 2); with 8 tiles it would spill at more waves and keeps the
-// default; FP64 backward with up to 4 tiles fits 4 waves.
+// default; FP64 backward with up to 4 tiles: 3 waves. It fits 4 where a leaf
+// unit keeps one running sum, but that put the FP64 solve's error 9 to 13 %
+// above the workgroup tasks' (151 x 97 grid, k = 17: 3.96e-16 against 3.61e-16;
+// 3.61e-16 with two sums). 3 waves and two sums against 4 and one: 511 x 389
+// grid, k = 17 248 and 246 us, 311 x 189, k = 32 144 and 141, 33^3, k = 17 192
+// and 194, icosphere(6), k = 40 180 and 179; two sums at 4 waves spill: 254,
+// 145, 199, 181.
 template <typename F, int NT, bool Forward> constexpr int kMinWavesFor() {
     if (sizeof(F) == 4) return NT >= 8 ? 3 : 4;
-    if (!Forward) return NT <= 4 ? 4 : 1;
     return NT <= 4 ? 3 : 1;
 }
 // Backward tasks stage the R-row indices they read in LDS (up to this many).
@@ -521,7 +526,7 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int nsteps = (rows - first + 3) / 4, groups = (last - first + 15) / 16;
-    // In FP32 even and odd steps are summed apart (up to 40 steps of 4 rows:
+    // Even and odd steps are summed apart (up to 40 steps of 4 rows:
     // the rounding of one long running sum grows with its length).
     Acc acc[kGroups][NT], odd[kGroups][NT];
 #pragma unroll
@@ -567,7 +572,7 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
                     const F x = rho < rows && rho >= first + 16 * g + l ? from_bits<F>(av[d][u][g]) : F(0);
 #pragma unroll
                     for (int n = 0; n < NT; ++n) {
-                        Acc &sum = sizeof(F) == 4 && u % 2 ? odd[g][n] : acc[g][n];
+                        Acc &sum = u % 2 ? odd[g][n] : acc[g][n];
                         sum = Mfma<F>::step(x, b[n], sum);
                     }
                 }
@@ -586,7 +591,7 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
     for (int g = 0; g < kGroups; ++g)
 #pragma unroll
         for (int n = 0; n < NT; ++n)
-            if (sizeof(F) == 4) acc[g][n] += odd[g][n];
+            acc[g][n] += odd[g][n];
 #pragma unroll
     for (int g = 0; g < kGroups; ++g)
 #pragma unroll
