@@ -99,14 +99,15 @@ struct BlockPlanOptions {
     // at the rate the block tasks reach), and the products with X and X' (two
     // launches and X's entries at the rate they reach). Fitted to solves of
     // k = 3 over all cuts of eight systems, in us without a top and with what
-    // the rule takes: icosphere(5) FP32 65.5 -> 43.3 (2,640 rows), (6) FP32
-    // 93.0 -> 70.2 (5,274), (6) FP64 98.7 -> 77.5, (7) FP32 143.5 -> 146.3
-    // (5,109; k = 17 257 -> 227), (7) FP64 none (163.4; 169.6 with 2,886 rows,
-    // k = 17 288 and 270), 511 x 389 grid FP64 161.7 -> 156.2 (3,479; 161.7
-    // with 6,114), 200 x 150 grid FP64 78.3 -> 57.6 (5,455), 33^3 grid FP64
-    // 154.5 -> 126.5 (4,507), 48^3 grid FP32 243.3 -> 228.7 (6,241). More right-
-    // hand sides gain more from the same cuts. More rows than top_max_rows
-    // were hardly measured, and cost a refactorisation more than they give.
+    // the rule takes: icosphere(5) FP32 65.3 -> 43.0 (2,640 rows), (6) FP32
+    // 93.2 -> 66.2 (5,274), (6) FP64 99.3 -> 72.8, (7) FP32 144.1 -> 142.1
+    // (5,109; k = 17 258 -> 221), (7) FP64 none (163.6; 165.6 with 2,886 rows,
+    // k = 17 291 and 272), 511 x 389 grid FP64 162.1 -> 151.6 (3,479; 153.1
+    // with 6,114), 200 x 150 grid FP64 78.2 -> 51.6 (5,455), 33^3 grid FP64
+    // 154.8 -> 123.2 (4,507), 48^3 grid FP32 243.7 -> 230.9 (6,241). More right-
+    // hand sides gain more from the same cuts. Of tops of more rows than
+    // top_max_rows only 33^3 was measured (6,565: FP32 101.8 -> 95.6, FP64
+    // 123.2 -> 122.1): their inverse costs a refactorisation more.
     double pass_us = 25.0, level_us = 3.0, level_gbs = 4000.0, top_us = 12.0, top_gbs = 4000.0;
     int64_t top_max_rows = 6400;
     bool top_forced = false;   // a top wherever a cut fits top_max_rows, estimate or not

@@ -115,7 +115,9 @@ struct DeviceBlockPlan {
     void *mtop = nullptr;
     DenseTopPanel *top_fwd = nullptr, *top_bwd = nullptr;
     int *top_units = nullptr;
-    int n_top_panels = 0;
+    int n_top_fwd = 0, n_top_bwd = 0;
+    double *top_sums = nullptr;         // segment sums and arrivals (DenseTopArgs)
+    unsigned *top_arrived = nullptr;
     bool whole = false;
     DeviceTopLists tops;
     int *perm = nullptr;   // caller row of each plan row
@@ -129,6 +131,8 @@ struct DeviceBlockPlan {
         dev_free(top_fwd);
         dev_free(top_bwd);
         dev_free(top_units);
+        dev_free(top_sums);
+        dev_free(top_arrived);
         tops.release();
         dev_free(perm);
         dev_free(colptr);
@@ -366,7 +370,11 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mfwd), me * fb));
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mbwd), me * fb));
     HIP_TRY(dev_alloc(reinterpret_cast<char **>(&d.mtop), 2 * (size_t)tops.entries * fb));
-    d.n_top_panels = (int)tops.fwd.size();
+    d.n_top_fwd = (int)tops.fwd.size();
+    d.n_top_bwd = (int)tops.bwd.size();
+    HIP_TRY(dev_alloc(&d.top_sums, (size_t)tops.slots * kTopUnit * kMaxRhs));
+    HIP_TRY(dev_alloc(&d.top_arrived, (size_t)tops.slots * kTopArrivals));
+    HIP_TRY(hipMemset(d.top_arrived, 0, std::max<size_t>(1, (size_t)tops.slots * kTopArrivals) * sizeof(unsigned)));
     d.whole = !blk_sys && P.nblocks > 0 && (int)P.tops.size() == P.nblocks;
     HIP_TRY(upload(&d.top_fwd, tops.fwd.data(), tops.fwd.size()));
     HIP_TRY(upload(&d.top_bwd, tops.bwd.data(), tops.bwd.size()));
@@ -1002,6 +1010,8 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         top.panels = forward ? d.top_fwd : d.top_bwd;
         top.units = forward ? nullptr : d.top_units;
         top.M = static_cast<const char *>(d.mtop) + (forward ? 0 : half);
+        top.sums = d.top_sums;
+        top.arrived = d.top_arrived;
         top.in = forward ? w.z : w.y;
         top.out = forward ? w.y : d.whole ? nullptr : w.z;
         top.x = forward ? nullptr : x;
@@ -1018,12 +1028,12 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
             const hipError_t e = launch_gather_rows(fbytes, w.z, b, d.perm, s->n, k, st);
             if (e != hipSuccess) return e;
         }
-        return launch_dense_top(fbytes, top, d.n_top_panels, bf.max_k, st);
+        return launch_dense_top(fbytes, top, forward ? d.n_top_fwd : d.n_top_bwd, bf.max_k, st);
     };
     for (int pass = 0; pass < 2; ++pass) {
         if (only_pass >= 0 && pass != only_pass) continue;
         const bool forward = pass == 0;
-        if (d.n_top_panels > 0 && (!forward || d.whole)) HIP_TRY(dense_top(forward));
+        if (d.n_top_fwd > 0 && (!forward || d.whole)) HIP_TRY(dense_top(forward));
         if (d.whole) continue;
         const int tile = effective_tile(s, fbytes, bf.max_k);
         if (is_panel_tile(tile)) {
@@ -1052,7 +1062,7 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         bf.tile = tile;
         bf.leaf_queues = &s->queues[6 + (forward ? 1 : 0)];
         HIP_TRY(launch_block_pass(fbytes, forward, bf, grid, s->queues[4 + (forward ? 1 : 0)], st));
-        if (d.n_top_panels > 0 && forward) HIP_TRY(dense_top(true));
+        if (d.n_top_fwd > 0 && forward) HIP_TRY(dense_top(true));
     }
     return CHOLESPY_OK;
 }

@@ -19,8 +19,8 @@
 // time: refactorize + solve of a 100 x 60 grid, FP32, 2.37 ms with the values
 // formed on the host and no top, 7.1 with S^{-1}, 1.9 with X; 61 x 47 1.13 /
 // 2.36 / 0.92 ms. The price is a launch: icosphere(3), k = 3, FP32 53 us by
-// the block passes, 6.4 with S^{-1}, 10.4; icosphere(5) 66 / 40 / 44; but
-// icosphere(6), k = 128, FP32 342 / 225 / 202.
+// the block passes, 6.4 with S^{-1}, 10.4; icosphere(5) 65 / 40 / 43; but
+// icosphere(6), k = 128, FP32 342 / 225 / 189.
 //
 // Rounding: products are summed a few at a time, and those sums in FP64 (one
 // running FP32 sum lost a factor of 3 to 4).
@@ -67,13 +67,13 @@ template <> struct Pack<double> {
 
 // The panel of a workgroup and its system's vectors.
 struct Top {
-    int row0, n, panel, first, count, k;
+    int row0, n, panel, first, count, seg, nseg, slot, k;
     long long vbase;
     int64_t off;
 };
 __device__ __forceinline__ Top top_of(const DenseTopArgs &a) {
     const DenseTopPanel t = a.panels[blockIdx.x];
-    Top r{t.row0, t.n, t.panel, t.first, t.count, a.k, 0, t.off};
+    Top r{t.row0, t.n, t.panel, t.first, t.count, t.seg, t.nseg, t.slot, a.k, 0, t.off};
     if (a.sys_k) {
         r.k = a.sys_k[t.sys];
         r.vbase = a.sys_vbase[t.sys];
@@ -93,6 +93,34 @@ __device__ __forceinline__ void put(const DenseTopArgs &a, const Top &top, int c
         double *x64 = static_cast<double *>(a.x);
         x64[o] = (a.xmode == 2 ? x64[o] : 0.0) + (double)v;
     }
+}
+
+// Segment sums (panels of more than kTopSegment units): a segment publishes
+// its sums (put_sum), and the one that arrives last, whichever that is, finds
+// all of them complete and adds them in segment order (sum_of). Nobody waits
+// for another workgroup. The stores and loads are agent-scope ones, each
+// store complete before its workgroup's arrival is counted.
+__device__ __forceinline__ double *sum_at(const DenseTopArgs &a, const Top &top, int seg, int row, int col) {
+    return a.sums + ((size_t)(top.slot + seg) * kTopUnit + row) * kMaxRhs + col;
+}
+__device__ __forceinline__ void put_sum(const DenseTopArgs &a, const Top &top, int row, int col, double s) {
+    publish(sum_at(a, top, top.seg, row, col), s);
+}
+__device__ __forceinline__ bool arrives_last(const DenseTopArgs &a, const Top &top, int tile, int *last) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned *n = a.arrived + (size_t)top.slot * kTopArrivals + tile;
+        *last = __hip_atomic_fetch_add(n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)top.nseg - 1;
+        if (*last) __hip_atomic_store(n, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    return *last != 0;
+}
+__device__ __forceinline__ double sum_of(const DenseTopArgs &a, const Top &top, int row, int col) {
+    double s = 0.0;
+    for (int seg = 0; seg < top.nseg; ++seg) s += from_bits<double>(load_bits(sum_at(a, top, seg, row, col)));
+    return s;
 }
 
 // Where a product's inputs are: rows of the top in order from unit `first` on
@@ -120,7 +148,7 @@ struct Buffer {
 };
 
 // Up to KT right-hand sides: one workgroup per panel, its 16 wavefronts take
-// the panel's groups of G inputs in turn. A chunk is kFly groups of every
+// the panel's (or the segment's) groups of G inputs in turn. A chunk is kFly groups of every
 // wavefront: all its loads are in flight at once, and each register is loaded
 // for the next chunk as soon as it is used, while the next chunk's inputs go
 // to the other LDS buffer. Bound by streaming the panel and, for the many
@@ -138,6 +166,7 @@ __global__ __launch_bounds__(kNarrowThreads) __attribute__((amdgpu_waves_per_eu(
     static_assert(kTopUnit * KT == kWave, "a wavefront stages one unit at a time");
     __shared__ __align__(16) F in[2][kChunk * KT];
     __shared__ double red[kNarrowWaves * 16 * KT];
+    __shared__ int last;
     const Top top = top_of(a);
     const int k = top.k;
     if (k <= 0) return;
@@ -211,12 +240,16 @@ __global__ __launch_bounds__(kNarrowThreads) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
         for (int t = 0; t < KT; ++t) red[(wave * 16 + lane) * KT + t] = acc[t];
     __syncthreads();
-    if (out) {
-        double s = 0.0;
+    double s = 0.0;
+    if (out)
 #pragma unroll
         for (int w = 0; w < kNarrowWaves; ++w) s += red[w * 16 * KT + tid];
-        put(a, top, oc, ot, xrow, (F)s);
+    if (top.nseg > 1) {
+        if (out) put_sum(a, top, tid / KT, ot, s);
+        if (!arrives_last(a, top, 0, &last)) return;
+        if (out) s = sum_of(a, top, tid / KT, ot);
     }
+    if (out) put(a, top, oc, ot, xrow, (F)s);
 }
 
 // More right-hand sides: a workgroup takes a panel and NT tiles of 16
@@ -230,7 +263,7 @@ constexpr int kOneTileFly = 5;   // D of one tile
 // (A wavefront's groups, with those asked for ahead, fit two registers a lane.)
 static_assert(kTopMaxRows / (Pack<double>::V * 4 * kWideWaves) + 2 * kOneTileFly - 2 < 2 * kWave, "kTopMaxRows");
 template <typename F, int NT, int D, int kIn>
-__device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top, int t0, double (*red)[kWave * 4]) {
+__device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top, int t0, double (*red)[kWave * 4], int *last) {
     using P = Pack<F>;
     using Vec = typename P::Vec;
     using Acc = typename P::Acc;
@@ -337,21 +370,30 @@ __device__ __forceinline__ void wide_tiles(const DenseTopArgs &a, const Top &top
         double s = 0.0;
 #pragma unroll
         for (int w = 0; w < kHalf; ++w) s += red[w * NT + n][e];
-        if (c < top.n && col < k && col >= t0 + NT * l) put(a, top, c, col, a.x ? a.perm[top.row0 + c] : 0, (F)s);
+        if (c >= top.n || col >= k || col < t0 + NT * l) continue;
+        if (top.nseg > 1) put_sum(a, top, c - top.panel * 16, col, s);
+        else put(a, top, c, col, a.x ? a.perm[top.row0 + c] : 0, (F)s);
+    }
+    if (top.nseg == 1 || !arrives_last(a, top, t0 / 16, last)) return;
+    const int width = min(16 * NT, k - t0);
+    for (int e = threadIdx.x; e < kTopUnit * width; e += kWideThreads) {
+        const int row = e / width, col = t0 + e % width, c = top.panel * 16 + row;
+        if (c < top.n) put(a, top, c, col, a.x ? a.perm[top.row0 + c] : 0, (F)sum_of(a, top, row, col));
     }
 }
 
 template <typename F, int NT, int D, int kIn>
 __global__ __launch_bounds__(kWideThreads) __attribute__((amdgpu_waves_per_eu(4))) void dense_wide(DenseTopArgs a) {
     __shared__ double red[kWideWaves / 2 * NT][kWave * 4];
+    __shared__ int last;
     const Top top = top_of(a);
     const int t0 = blockIdx.y * NT * 16;
     if (t0 >= top.k) return;
     // A rest of one tile: a batch's systems differ in their right-hand sides.
     if (NT > 1 && top.k - t0 <= 16)
-        wide_tiles<F, 1, kOneTileFly, kIn>(a, top, t0, red);
+        wide_tiles<F, 1, kOneTileFly, kIn>(a, top, t0, red, &last);
     else
-        wide_tiles<F, NT, D, kIn>(a, top, t0, red);
+        wide_tiles<F, NT, D, kIn>(a, top, t0, red, &last);
 }
 
 // dst row i = src row rows[i], k columns.

@@ -8,6 +8,22 @@ TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
     TopLists L;
     std::vector<int> pack_bwd;
     int64_t fwd_units = 0, bwd_units = 0;
+    int slots[2] = {0, 0};
+    // A panel's segments, as even as they go.
+    auto push = [&](bool fwd, DenseTopPanel p) {
+        const int count = p.count, first = p.first;
+        const int64_t off = p.off;
+        p.nseg = (count + kTopSegment - 1) / kTopSegment;
+        p.slot = p.nseg > 1 ? slots[fwd] : 0;
+        if (p.nseg > 1) slots[fwd] += p.nseg;
+        for (p.seg = 0; p.seg < p.nseg; ++p.seg) {
+            const int lo = (int)((int64_t)count * p.seg / p.nseg), hi = (int)((int64_t)count * (p.seg + 1) / p.nseg);
+            p.first = first + lo;
+            p.count = hi - lo;
+            p.off = off + (int64_t)lo * kTopUnitEntries;
+            (fwd ? L.fwd : L.bwd).push_back(p);
+        }
+    };
     // The jobs of all blocks, by stage.
     struct Pending {
         TopLists::Job job;
@@ -46,7 +62,7 @@ TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
         for (int p = 0; p < np; ++p) {
             int lo = 0;
             while (!has[(size_t)p * np + lo]) ++lo;
-            L.fwd.push_back({row0, m, p, sys, lo, p - lo + 1, fwd_units * kTopUnitEntries});
+            push(true, {row0, m, p, sys, lo, p - lo + 1, 0, 1, 0, 0, fwd_units * kTopUnitEntries});
             for (int q = lo; q <= p; ++q) L.pack.push_back(code(p, q));
             fwd_units += p - lo + 1;
             const int first = (int)L.units.size();
@@ -56,7 +72,7 @@ TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
                     pack_bwd.push_back(code(r, p));
                 }
             const int count = (int)L.units.size() - first;
-            L.bwd.push_back({row0, m, p, sys, first, count, bwd_units * kTopUnitEntries});
+            push(false, {row0, m, p, sys, first, count, 0, 1, 0, 0, bwd_units * kTopUnitEntries});
             bwd_units += count;
         }
         // Stages 2 s' (into temporaries) and 2 s' + 1 (back) of doubling s'.
@@ -84,6 +100,7 @@ TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
                         }
         }
     }
+    L.slots = std::max(slots[0], slots[1]);
     L.entries = std::max(fwd_units, bwd_units) * kTopUnitEntries;
     L.pack.resize((size_t)std::max(fwd_units, bwd_units), -1);
     pack_bwd.resize(L.pack.size(), -1);

@@ -19,19 +19,31 @@ constexpr int kTopUnitEntries = kTopUnit * kTopUnit;
 constexpr int kTopTile = 64;                          // rows and columns of a tile of X while it is formed
 constexpr int kTopTileEntries = kTopTile * kTopTile;
 
-// One panel of 16 outputs of a product: count input units from unit `first`
-// on (w = X r: consecutive units of 16 rows), or those listed from position
-// `first` of TopLists::units on (z = X' w). Device record.
+// Panels of more units than this are split among several workgroups: one
+// streams 20 to 30 KB a microsecond, and the panels near the root have every
+// row of the top as input. First product, whole panels against segments:
+// icosphere(6), k = 16, FP64 (330 units) 27.3 -> 13.9 us, k = 128, FP32 43.0 ->
+// 28.1, 33^3 grid, k = 5, FP64 24.9 -> 18.6, icosphere(7), k = 3, FP32 16.4 ->
+// 13.0. (Twice the wavefronts a workgroup instead: 28.1, 42.0, 26.7.)
+constexpr int kTopSegment = 96;
+
+// One panel of 16 outputs of a product, or one of its segments: count input
+// units from unit `first` on (w = X r: consecutive units of 16 rows), or those
+// listed from position `first` of TopLists::units on (z = X' w). Segment `seg`
+// of nseg leaves its sums in slot + seg of the segment sums; the last one to
+// finish adds them up in order. Device record.
 struct DenseTopPanel {
     int row0, n;      // first row of the top block and its rows
     int panel, sys;
     int first, count;
+    int seg, nseg, slot, reserved;
     int64_t off;      // first element in the direction's array
 };
 
 struct TopLists {
     std::vector<DenseTopPanel> fwd, bwd;   // longest first: the last workgroups to start are the short ones
     std::vector<int> units;
+    int slots = 0;                         // segment sums (the more of the two directions)
     int64_t entries = 0;                   // elements of one direction's array
 
     // Forming X. A block is a square of 64 x 64 tiles, of which those with an

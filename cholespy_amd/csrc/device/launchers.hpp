@@ -151,12 +151,15 @@ struct DenseTopArgs {
     const int *rows;               // first product of a whole system, up to 4 right-hand sides: `in` is b, whose
     int b_rows;                    // row rows[r] (of b_rows) is plan row r; null: `in` is in plan order
     const void *M, *in;
+    double *sums;                  // segment sums: 16 rows of kMaxRhs a slot
+    unsigned *arrived;             // per slot and 16 right-hand sides, zero between launches
     void *out, *x;                 // plan order (null: not stored); the solution (null: not stored)
     const int *perm;               // solution row of each plan row
     int k, xmode;                  // xmode as in BlockPassBuffers
     const int *sys_k;              // batches (null for a single system)
     const long long *sys_vbase;
 };
+constexpr int kTopArrivals = 128 / 16;   // counters per slot
 hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int panels, int max_k, hipStream_t stream);
 // dst row i := src row rows[i] (n rows of k values).
 hipError_t launch_gather_rows(int float_bytes, void *dst, const void *src, const int *rows, int n, int k,

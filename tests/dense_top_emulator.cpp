@@ -157,16 +157,20 @@ void form_inverse(const Factor &f, const BlockPlan &P, const TopLists &L, std::v
 // The product of one direction: out = X in or X' in on the top rows.
 void product(const TopLists &L, bool forward, const std::vector<double> &x, const std::vector<double> &in,
              std::vector<double> &out) {
-    std::set<int> rows;
+    std::set<int> rows, slots;
+    std::set<std::pair<int, int>> segments;
+    for (const auto &c : L.columns) out[(size_t)c.row0 + c.c] = 0.0;
     int longest = 1 << 30;
     for (const DenseTopPanel &p : forward ? L.fwd : L.bwd) {
-        check(p.count > 0 && p.count <= longest, "panels longest first");
+        check(p.count > 0 && p.count <= kTopSegment && p.count <= longest, "panels longest first");
+        check(p.seg >= 0 && p.seg < p.nseg && segments.insert({p.row0 + p.panel * kTopUnit, p.seg}).second, "a segment twice");
+        if (p.nseg > 1) check(p.slot >= 0 && p.slot + p.nseg <= L.slots && slots.insert(p.slot + p.seg).second, "a slot twice");
         longest = p.count;
         check(p.off >= 0 && p.off + (int64_t)p.count * kTopUnitEntries <= L.entries, "a panel outside its array");
         for (int o = 0; o < kTopUnit; ++o) {
             const int c = p.panel * kTopUnit + o;
             if (c >= p.n) continue;
-            check(rows.insert(p.row0 + c).second, "a top row in two panels");
+            if (p.seg == 0) check(rows.insert(p.row0 + c).second, "a top row in two panels");
             double s = 0.0;
             for (int u = 0; u < p.count; ++u) {
                 const int unit = forward ? p.first + u : L.units[(size_t)p.first + u];
@@ -175,9 +179,11 @@ void product(const TopLists &L, bool forward, const std::vector<double> &x, cons
                     if (unit * kTopUnit + i < p.n)
                         s += x[(size_t)p.off + (size_t)(u * kTopUnit + o) * kTopUnit + i] * in[(size_t)p.row0 + unit * kTopUnit + i];
             }
-            out[(size_t)p.row0 + c] = s;
+            out[(size_t)p.row0 + c] += s;
         }
     }
+    for (const DenseTopPanel &p : forward ? L.fwd : L.bwd)
+        for (int q = 0; q < p.nseg; ++q) check(segments.count({p.row0 + p.panel * kTopUnit, q}) == 1, "a segment is missing");
     size_t n = 0;
     for (const auto &c : L.columns) n += (size_t)(c.c >= 0);
     check(rows.size() == n, "panels cover the top rows");
