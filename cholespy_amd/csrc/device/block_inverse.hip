@@ -22,6 +22,7 @@
 #include "block_inverse.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 #include <vector>
 
 #include "common.hpp"
@@ -354,17 +355,26 @@ __global__ void cast_factor(int64_t nnz, const double *val, const int *csr_src, 
     }
 }
 
-// Device memory that lives for one fill.
+// Work memory of one group of a fill, within CHOLESPY_FILL_MIB if that is set.
 struct Arena {
     std::vector<void *> held;
+    size_t left = bound();
+    static size_t bound() {
+        const char *e = std::getenv("CHOLESPY_FILL_MIB");
+        return e ? (size_t)std::max(0, std::atoi(e)) << 20 : ~size_t(0);
+    }
     ~Arena() {
         for (void *p : held) (void)hipFree(p);
     }
     template <typename T>
     hipError_t get(T **p, size_t count) {
         void *q = nullptr;
+        *p = nullptr;
+        if (count * sizeof(T) > left) return hipErrorOutOfMemory;
+        left -= count * sizeof(T);
         const hipError_t e = hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T));
         if (e == hipSuccess) held.push_back(q);
+        else (void)hipGetLastError();   // (not for the next launch to report)
         *p = static_cast<T *>(q);
         return e;
     }

@@ -60,7 +60,9 @@ struct DeviceTopLists {
 
 // Fills mfwd and mbwd (offsets P.moff) and the top blocks' mtop (X, then X',
 // tops.entries elements each). small: device list of the n_small blocks of up
-// to 64 rows that are not top blocks.
+// to 64 rows that are not top blocks. Work memory that cannot be had, or more
+// of it at a time than CHOLESPY_FILL_MIB allows, ends in
+// hipErrorOutOfMemory, by then with some values overwritten.
 hipError_t fill_block_plan_on_device(const BlockPlan &P, const InverseArgs &args, const int *small, int n_small,
                                      const DeviceTopLists &tops, int float_bytes, void *mfwd, void *mbwd, void *mtop);
 // The blocks of P that `small` lists.

@@ -79,7 +79,9 @@ template <typename T>
 hipError_t dev_alloc(T **p, size_t count) {
     *p = nullptr;
     if (count == 0) count = 1;
-    return hipMalloc(reinterpret_cast<void **>(p), count * sizeof(T));
+    const hipError_t e = hipMalloc(reinterpret_cast<void **>(p), count * sizeof(T));
+    if (e != hipSuccess) (void)hipGetLastError();   // (not for the next launch to report)
+    return e;
 }
 
 template <typename T>
@@ -171,7 +173,10 @@ struct cholespy_gpu_solver {
     int fbytes = 4;
     int64_t nnz = 0;
     int device = 0;
-    bool uploaded = false;
+    // planned: the pattern and the plan's structure are on the device;
+    // uploaded: their values are, whole. A fill that fails part way leaves
+    // planned alone, and solves refuse until values are uploaded again.
+    bool planned = false, uploaded = false;
     bool analysed[2] = {false, false};   // [0] = upper (L'), [1] = lower (L)
     int n_levels[2] = {0, 0};
 
@@ -322,6 +327,7 @@ std::vector<int> device_tasks(const BlockPlan &P, const std::vector<int> &tasks,
 int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<int> &perm,
                 const std::vector<int64_t> &colptr, const std::vector<int> &src, const std::vector<int> *blk_sys) {
     DeviceBlockPlan &d = s->plan;
+    s->planned = s->uploaded = false;
     d.release();
     d.nblocks = P.nblocks;
     d.nslots = P.rptr[P.nblocks];
@@ -391,6 +397,7 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
     for (auto &row : s->grid_blocks)
         for (int &g : row) g = 0;
     s->buffers_path = -1;
+    s->planned = true;
     return CHOLESPY_OK;
 }
 
@@ -413,8 +420,13 @@ struct DeviceTemp {
 // compressed columns (rowidx and val: device).
 int fill_plan_values(cholespy_gpu_solver *s, const BlockPlan &P, const int *rowidx, const double *val) {
     DeviceBlockPlan &d = s->plan;
+    s->uploaded = false;
     const InverseArgs args{d.colptr, rowidx, val, d.src, d.rank, d.start, d.rptr, d.rlist, d.moff};
-    HIP_TRY(fill_block_plan_on_device(P, args, d.small, d.n_small, d.tops, s->fbytes, d.mfwd, d.mbwd, d.mtop));
+    try {
+        HIP_TRY(fill_block_plan_on_device(P, args, d.small, d.n_small, d.tops, s->fbytes, d.mfwd, d.mbwd, d.mtop));
+    } catch (const std::exception &ex) {
+        return fail(CHOLESPY_ERR_HIP, ex.what());
+    }
     return CHOLESPY_OK;
 }
 
@@ -423,8 +435,11 @@ int fill_plan_values(cholespy_gpu_solver *s, const BlockPlan &P, const int *rowi
 int upload_values(cholespy_gpu_solver *s, const double *val) {
     DeviceTemp tval;
     HIP_TRY(tval.put(val, (size_t)s->nnz));
+    s->uploaded = false;
     HIP_TRY(launch_cast_factor(s->fbytes, s->nnz, tval.as<double>(), s->csr_src, s->lvals, s->uvals));
-    return fill_plan_values(s, s->host_plan, s->ucols, tval.as<double>());
+    const int rc = fill_plan_values(s, s->host_plan, s->ucols, tval.as<double>());
+    s->uploaded = rc == CHOLESPY_OK;
+    return rc;
 }
 
 // Whether plans may have a dense top (CHOLESPY_DENSE_TOP: its most rows, and
@@ -464,18 +479,17 @@ BlockPlan plan_structure(int n, const int *colptr, const int *rowidx, BlockPlanO
 // Plans the uploaded pattern with base options `base` and uploads the
 // structure (the values follow).
 int plan_system(cholespy_gpu_solver *s, const BlockPlanOptions &base) {
-    BlockPlan P;
-    std::vector<int> src;
     try {
-        P = plan_structure(s->n, s->host_colptr.data(), s->host_rowidx.data(), plan_options(base), s->fbytes, src);
+        std::vector<int> src;
+        BlockPlan P = plan_structure(s->n, s->host_colptr.data(), s->host_rowidx.data(), plan_options(base), s->fbytes, src);
+        std::vector<int> perm((size_t)s->n);
+        for (int r = 0; r < s->n; ++r) perm[(size_t)r] = s->host_perm[(size_t)src[(size_t)r]];
+        const int rc = upload_plan(s, P, perm, std::vector<int64_t>(s->host_colptr.begin(), s->host_colptr.end()), src);
+        if (rc != CHOLESPY_OK) return rc;
+        s->host_plan = std::move(P);
     } catch (const std::exception &ex) {
         return fail(CHOLESPY_ERR_INVALID_ARGUMENT, ex.what());
     }
-    std::vector<int> perm((size_t)s->n);
-    for (int r = 0; r < s->n; ++r) perm[(size_t)r] = s->host_perm[(size_t)src[(size_t)r]];
-    const int rc = upload_plan(s, P, perm, std::vector<int64_t>(s->host_colptr.begin(), s->host_colptr.end()), src);
-    if (rc != CHOLESPY_OK) return rc;
-    s->host_plan = std::move(P);
     s->plan_base = base;
     return CHOLESPY_OK;
 }
@@ -694,7 +708,7 @@ int cholespy_solver_upload_factor(cholespy_gpu_solver *s, const int *perm, const
             }
     }
     const size_t fb = (size_t)s->fbytes;
-    s->uploaded = false;
+    s->planned = s->uploaded = false;
     dev_free(s->lrowptr);
     dev_free(s->lcols);
     dev_free(s->lvals);
@@ -723,7 +737,6 @@ int cholespy_solver_upload_factor(cholespy_gpu_solver *s, const int *perm, const
     if (rc != CHOLESPY_OK) return rc;
     rc = upload_values(s, val);
     if (rc != CHOLESPY_OK) return rc;
-    s->uploaded = true;
     s->buffers_path = -1;
     return CHOLESPY_OK;
 }
@@ -756,7 +769,7 @@ int cholespy_normalize_input(int n, int64_t nnz, const void *ii, const void *jj,
 int cholespy_solver_refactor(cholespy_gpu_solver *s, const double *val, int64_t nnz) {
     if (!s || !val) return fail(CHOLESPY_ERR_INVALID_ARGUMENT, "null argument");
     if (s->is_batch) return fail(CHOLESPY_ERR_INVALID_ARGUMENT, "refactor is not available for batches");
-    if (!s->uploaded) return fail(CHOLESPY_ERR_STATE, "refactor called before upload_factor");
+    if (!s->planned) return fail(CHOLESPY_ERR_STATE, "refactor called before upload_factor");
     if (nnz != s->nnz) return fail(CHOLESPY_ERR_INVALID_ARGUMENT, "nnz does not match the uploaded factor");
     for (int j = 0; j < s->n; ++j) {
         const double d = val[s->host_colptr[j]];
@@ -1150,6 +1163,7 @@ int cholespy_solver_upload_matrix(cholespy_gpu_solver *s, const int *colptr, con
                 vals[next[j]++] = val[p];
             }
     }
+    s->has_matrix = false;
     dev_free(s->arowptr);
     dev_free(s->acols);
     dev_free(s->avals);
@@ -1176,6 +1190,7 @@ int refined_impl(cholespy_gpu_solver *s, int k, const double *b, double *x, int 
     if (!s) return fail(CHOLESPY_ERR_INVALID_ARGUMENT, "null solver");
     if (s->fbytes != 4) return fail(CHOLESPY_ERR_INVALID_ARGUMENT, "refined solves need a float32 solver");
     if (!s->has_matrix) return fail(CHOLESPY_ERR_STATE, "refined solve called before upload_matrix");
+    if (!s->uploaded) return fail(CHOLESPY_ERR_STATE, "solve called before the factor was uploaded");
     if (k > kMaxRhs) return fail(CHOLESPY_ERR_INVALID_ARGUMENT, "The number of RHS should be less than 128.");
     if (k < 0 || iterations < 0) return fail(CHOLESPY_ERR_INVALID_ARGUMENT, "negative argument");
     if (k == 0 || s->n == 0) return CHOLESPY_OK;
@@ -1951,6 +1966,7 @@ extern "C" int cholespy_solver_autotune(cholespy_gpu_solver *s, const double *va
     best.path = s->path;
     best.fused = s->fused_leaves;
     best.queues = s->queues[4].nq;
+    const TuneConfig initial = best;
     double best_ms = 0;
     auto finish = [&](const char *how, int evaluated, double default_ms) {
         std::string r = std::string(how) + " " + format_config(best);
@@ -2057,9 +2073,12 @@ extern "C" int cholespy_solver_autotune(cholespy_gpu_solver *s, const double *va
     (void)hipDeviceSynchronize();
     (void)hipFree(b);
     (void)hipFree(x);
-    if (rc != CHOLESPY_OK) return rc;
-    rc = apply_config(s, val, k, best);
-    if (rc != CHOLESPY_OK) return rc;
+    if (rc == CHOLESPY_OK) rc = apply_config(s, val, k, best);
+    if (rc != CHOLESPY_OK) {   // back to the plan the call found, if that can be had
+        const std::string why = g_error;
+        (void)apply_config(s, val, k, initial);
+        return fail(rc, why);
+    }
     if (!(flags & 2)) cache_store(path, key, best, best_ms);
     return finish("tuned", evaluated, default_ms);
 }
