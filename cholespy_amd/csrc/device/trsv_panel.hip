@@ -621,6 +621,22 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
     }
 }
 
+// One unit; the task's timeline is that of its first right-hand sides. (A
+// forward unit gathers nothing, a backward one waits as it multiplies: the
+// second stamp is the first.)
+template <typename F, bool FORWARD>
+__device__ __forceinline__ void traced_leaf_unit(const BlockPassArgs<F> &a, const Task &task, const VecMap &vm, int tk, int t0,
+                                                 int *rowidx) {
+    const bool traced = a.leaf_trace && t0 == 0 && threadIdx.x % kWave == 0;
+    if (traced) a.leaf_trace[4 * (size_t)tk] = a.leaf_trace[4 * (size_t)tk + 1] = wall_clock64();
+    if (FORWARD) leaf_forward_unit<F>(a, task, vm, t0);
+    else leaf_backward_unit<F>(a, task, vm, t0, rowidx);
+    if (traced) {
+        a.leaf_trace[4 * (size_t)tk + 2] = wall_clock64();
+        a.leaf_trace[4 * (size_t)tk + 3] = blockIdx.x;
+    }
+}
+
 // Takes units until this wavefront's queue is exhausted, the next one
 // requested while a unit runs (trsv_blocks.hip leaf_phase).
 template <typename F, bool FORWARD>
@@ -634,10 +650,7 @@ __device__ __forceinline__ void leaf_phase_wide(const BlockPassArgs<F> &a, int *
         const Task task = load_task_at(a.leaf_task, t / a.leaf_chunks);
         const VecMap vm = vec_map(a, task);
         const int t0 = t % a.leaf_chunks * kLeafTiles * 16;
-        if (t0 < vm.k) {
-            if (FORWARD) leaf_forward_unit<F>(a, task, vm, t0);
-            else leaf_backward_unit<F>(a, task, vm, t0, lds + wave * kLeafMaxRows);
-        }
+        if (t0 < vm.k) traced_leaf_unit<F, FORWARD>(a, task, vm, t / a.leaf_chunks, t0, FORWARD ? nullptr : lds + wave * kLeafMaxRows);
         t = __builtin_amdgcn_readfirstlane(next);
     }
 }
@@ -1048,9 +1061,7 @@ void leaf_units(BlockPassArgs<F> a) {
     const Task task = load_task_at(a.leaf_task, (int)(u / a.leaf_chunks));
     const VecMap vm = vec_map(a, task);
     const int t0 = (int)(u % a.leaf_chunks) * kLeafTiles * 16;
-    if (t0 >= vm.k) return;
-    if (FORWARD) leaf_forward_unit<F>(a, task, vm, t0);
-    else leaf_backward_unit<F>(a, task, vm, t0, rowidx + wave * kLeafMaxRows);
+    if (t0 < vm.k) traced_leaf_unit<F, FORWARD>(a, task, vm, (int)(u / a.leaf_chunks), t0, rowidx + (FORWARD ? 0 : wave * kLeafMaxRows));
 }
 
 }  // namespace

@@ -306,8 +306,9 @@ int cholespy_entry_gradient(int n, int64_t nnz, const int *rows, const int *cols
 /* Task timeline of the block passes (diagnostics; no counterpart in the
  * reference). With tracing on, every block-pass launch records per task
  * {start, end of the gather phase, end, workgroup} as 100 MHz wall-clock
- * ticks; get_trace copies min(words, 4 * tasks) words of the last forward
- * (forward = 1) or backward pass. */
+ * ticks (a leaf task run for many right-hand sides: of its first 32); get_trace
+ * copies min(words, 4 * tasks) words of the last forward (forward = 1) or
+ * backward pass. A system whose rows are all top rows runs no tasks. */
 int cholespy_solver_set_trace(cholespy_gpu_solver *solver, int enable);
 int cholespy_solver_get_trace(const cholespy_gpu_solver *solver, int forward, uint64_t *out,
                               int64_t words);
