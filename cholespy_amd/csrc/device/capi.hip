@@ -1770,6 +1770,11 @@ uint64_t fnv1a(uint64_t h, const void *p, size_t bytes) {
     return h;
 }
 
+// Part of the key: raised when kernels or plans change so that what was timed
+// before need not be the best any more (a small system's rows schedule against
+// the dense top, say).
+constexpr int kTunePlans = 3;
+
 std::string tune_key(const cholespy_gpu_solver *s, int k) {
     uint64_t h = 1469598103934665603ull;
     h = fnv1a(h, &s->n, sizeof(s->n));
@@ -1785,8 +1790,8 @@ std::string tune_key(const cholespy_gpu_solver *s, int k) {
         if (colon != std::string::npos) arch.resize(colon);
     }
     char buf[160];
-    std::snprintf(buf, sizeof buf, "%016llx-n%d-f%d-t%d-%s-cu%d", (unsigned long long)h, s->n, s->fbytes * 8,
-                  block_tile(s->fbytes, k), arch.c_str(), cus);
+    std::snprintf(buf, sizeof buf, "%016llx-n%d-f%d-t%d-%s-cu%d-p%d", (unsigned long long)h, s->n, s->fbytes * 8,
+                  block_tile(s->fbytes, k), arch.c_str(), cus, kTunePlans);
     return buf;
 }
 
