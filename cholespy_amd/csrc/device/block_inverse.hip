@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <limits>
 #include <vector>
 
 #include "common.hpp"
@@ -258,16 +259,15 @@ __global__ __launch_bounds__(kThreads) void top_products(const TopLists::Job *jo
                 out[wi + 16 * x + (lane >> 4) + 4 * v + (wj + 16 * y + (lane & 15)) * kTopTile] = alpha * total[x][y][v];
 }
 
-// One unit a workgroup: units [0, gridDim.x / 2) of X, then as many of X'.
+// One unit a workgroup, of X (fwd) or X'.
 template <typename F>
-__global__ __launch_bounds__(kTopUnitEntries) void top_pack(const int *pack, const double *D, F *dst) {
+__global__ __launch_bounds__(kTopUnitEntries) void top_pack(const int *pack, const double *D, F *dst, bool fwd) {
     constexpr int V = 16 / (int)sizeof(F), G = 4 * V;
     const int code = pack[blockIdx.x], tid = threadIdx.x;
     const int lane = tid % (64 * V) / V, c = lane % 16, rho = tid / (64 * V) * G + tid % V * 4 + lane / 16;
     double v = 0.0;
     if (code >= 0) {
         const int i0 = code / 4 % 4 * kTopUnit, j0 = code % 4 * kTopUnit;
-        const bool fwd = blockIdx.x < gridDim.x / 2;
         v = D[(int64_t)(code / 16) * kTopTileEntries + i0 + (fwd ? c : rho) + (j0 + (fwd ? rho : c)) * kTopTile];
     }
     dst[(int64_t)blockIdx.x * kTopUnitEntries + tid] = (F)v;
@@ -358,11 +358,7 @@ __global__ void cast_factor(int64_t nnz, const double *val, const int *csr_src, 
 // Work memory of one group of a fill, within CHOLESPY_FILL_MIB if that is set.
 struct Arena {
     std::vector<void *> held;
-    size_t left = bound();
-    static size_t bound() {
-        const char *e = std::getenv("CHOLESPY_FILL_MIB");
-        return e ? (size_t)std::max(0, std::atoi(e)) << 20 : ~size_t(0);
-    }
+    int64_t left = std::getenv("CHOLESPY_FILL_MIB") ? fill_work_bytes() : std::numeric_limits<int64_t>::max();
     ~Arena() {
         for (void *p : held) (void)hipFree(p);
     }
@@ -370,8 +366,8 @@ struct Arena {
     hipError_t get(T **p, size_t count) {
         void *q = nullptr;
         *p = nullptr;
-        if (count * sizeof(T) > left) return hipErrorOutOfMemory;
-        left -= count * sizeof(T);
+        if ((int64_t)(count * sizeof(T)) > left) return hipErrorOutOfMemory;
+        left -= (int64_t)(count * sizeof(T));
         const hipError_t e = hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T));
         if (e == hipSuccess) held.push_back(q);
         else (void)hipGetLastError();   // (not for the next launch to report)
@@ -391,6 +387,18 @@ struct Arena {
         const hipError_t e_ = (expr);      \
         if (e_ != hipSuccess) return e_;   \
     } while (0)
+
+// launch(first, grid) over [lo, hi) in grids that a launch takes (fewer than
+// 2^32 threads).
+template <typename Launch>
+hipError_t in_grids(int64_t lo, int64_t hi, Launch launch) {
+    constexpr int64_t kMost = int64_t(1) << 22;
+    for (; lo < hi; lo += kMost) {
+        launch(lo, (unsigned)std::min(kMost, hi - lo));
+        INV_TRY(hipGetLastError());
+    }
+    return hipSuccess;
+}
 
 // The blocks `large` of P through dense work arrays.
 template <typename F>
@@ -490,29 +498,37 @@ hipError_t fill_large(const BlockPlan &P, const InverseArgs &args, const std::ve
     return hipDeviceSynchronize();   // the work arrays are freed on return
 }
 
-// The top blocks' X and X'.
+// The top blocks' X and X', group by group.
 template <typename F>
 hipError_t fill_tops(const InverseArgs &args, const DeviceTopLists &t, F *mtop) {
-    Arena arena;
-    double *D = nullptr, *T = nullptr;
-    INV_TRY(arena.get(&D, (size_t)t.tiles * kTopTileEntries));
-    INV_TRY(arena.get(&T, (size_t)t.temps * kTopTileEntries));
-    INV_TRY(hipMemsetAsync(D, 0, (size_t)t.tiles * kTopTileEntries * sizeof(double), nullptr));
-    top_scatter<<<dim3((unsigned)t.n_columns), 64>>>(args, t.columns, t.map, D);
-    INV_TRY(hipGetLastError());
-    top_diagonals<<<dim3((unsigned)t.n_diagonals), kThreads>>>(t.diagonals, D);
-    INV_TRY(hipGetLastError());
-    for (size_t s = 0; s + 1 < t.stages.size(); ++s) {
-        const int count = t.stages[s + 1] - t.stages[s];
-        if (count == 0) continue;
-        const bool even = s % 2 == 0;
-        top_products<<<dim3((unsigned)count), kThreads>>>(t.jobs + t.stages[s], t.pairs, D, even ? D : T, even ? T : D,
-                                                          even ? 1.0 : -1.0);
-        INV_TRY(hipGetLastError());
+    for (const TopLists::Group &g : t.groups) {
+        Arena arena;
+        double *D = nullptr, *T = nullptr;
+        INV_TRY(arena.get(&D, (size_t)g.tiles * kTopTileEntries));
+        INV_TRY(arena.get(&T, (size_t)g.temps * kTopTileEntries));
+        INV_TRY(hipMemsetAsync(D, 0, (size_t)g.tiles * kTopTileEntries * sizeof(double), nullptr));
+        INV_TRY(in_grids(g.columns[0], g.columns[1], [&](int64_t lo, unsigned grid) {
+            top_scatter<<<dim3(grid), 64>>>(args, t.columns + lo, t.map, D);
+        }));
+        INV_TRY(in_grids(g.diagonals[0], g.diagonals[1], [&](int64_t lo, unsigned grid) {
+            top_diagonals<<<dim3(grid), kThreads>>>(t.diagonals + lo, D);
+        }));
+        for (size_t s = 0; s + 1 < g.stages.size(); ++s) {
+            const bool even = s % 2 == 0;
+            INV_TRY(in_grids(g.stages[s], g.stages[s + 1], [&](int64_t lo, unsigned grid) {
+                top_products<<<dim3(grid), kThreads>>>(t.jobs + lo, t.pairs, D, even ? D : T, even ? T : D, even ? 1.0 : -1.0);
+            }));
+        }
+        const int64_t units = t.entries / kTopUnitEntries;
+        INV_TRY(in_grids(g.fwd_units[0], g.fwd_units[1], [&](int64_t lo, unsigned grid) {
+            top_pack<F><<<dim3(grid), kTopUnitEntries>>>(t.pack + lo, D, mtop + lo * kTopUnitEntries, true);
+        }));
+        INV_TRY(in_grids(units + g.bwd_units[0], units + g.bwd_units[1], [&](int64_t lo, unsigned grid) {
+            top_pack<F><<<dim3(grid), kTopUnitEntries>>>(t.pack + lo, D, mtop + lo * kTopUnitEntries, false);
+        }));
+        INV_TRY(hipDeviceSynchronize());   // the work arrays are freed
     }
-    top_pack<F><<<dim3((unsigned)(2 * (t.entries / kTopUnitEntries))), kTopUnitEntries>>>(t.pack, D, mtop);
-    INV_TRY(hipGetLastError());
-    return hipDeviceSynchronize();   // the work arrays are freed on return
+    return hipSuccess;
 }
 
 template <typename F>
@@ -521,25 +537,23 @@ hipError_t fill(const BlockPlan &P, const InverseArgs &args, const int *small, i
     std::vector<int> large;
     for (int b = 0; b < P.nblocks; ++b)
         if (!P.is_top(b) && P.start[b + 1] - P.start[b] > kSmall) large.push_back(b);
-    if (n_small > 0) {
-        small_blocks<F><<<dim3((unsigned)n_small), kThreads>>>(args, small, mfwd, mbwd);
-        INV_TRY(hipGetLastError());
-    }
-    // In groups whose work arrays take up to 4 GiB.
-    constexpr size_t kGroup = size_t(1) << 29;
+    INV_TRY(in_grids(0, n_small, [&](int64_t lo, unsigned grid) {
+        small_blocks<F><<<dim3(grid), kThreads>>>(args, small + lo, mfwd, mbwd);
+    }));
+    const size_t most = (size_t)fill_work_bytes() / sizeof(double);
     for (size_t lo = 0; lo < large.size();) {
         size_t hi = lo, words = 0;
         std::vector<int> group;
         for (; hi < large.size(); ++hi) {
             const size_t m = P.start[large[hi] + 1] - P.start[large[hi]], R = P.rptr[large[hi] + 1] - P.rptr[large[hi]];
             words += 3 * m * m + 2 * R * m;
-            if (hi > lo && words > kGroup) break;
+            if (hi > lo && words > most) break;
             group.push_back(large[hi]);
         }
         INV_TRY(fill_large<F>(P, args, group, mfwd, mbwd));
         lo = hi;
     }
-    if (tops.n_columns > 0) INV_TRY(fill_tops<F>(args, tops, mtop));
+    INV_TRY(fill_tops<F>(args, tops, mtop));
     return hipDeviceSynchronize();
 }
 
@@ -567,13 +581,14 @@ hipError_t DeviceTopLists::upload(const TopLists &l) {
     INV_TRY(put(&diagonals, l.diagonals));
     INV_TRY(put(&jobs, l.jobs));
     INV_TRY(put(&pairs, l.pairs));
-    n_columns = (int)l.columns.size();
-    n_diagonals = (int)l.diagonals.size();
-    tiles = l.tiles;
-    temps = l.temps;
     entries = l.entries;
-    stages = l.stages;
+    groups = l.groups;
     return hipSuccess;
+}
+
+int64_t fill_work_bytes() {
+    const char *e = std::getenv("CHOLESPY_FILL_MIB");
+    return e ? std::min<int64_t>(kTopWorkBytes, (int64_t)std::max(0, std::atoi(e)) << 20) : kTopWorkBytes;
 }
 
 std::vector<int> small_block_list(const BlockPlan &P) {

@@ -44,16 +44,15 @@ struct InversePack {
 };
 
 // Device copies of the lists that form the top blocks' inverses
-// (dense_top_plan.hpp), the stages on the host.
+// (dense_top_plan.hpp), the groups on the host.
 struct DeviceTopLists {
     TopLists::Column *columns = nullptr;
     int *map = nullptr, *pack = nullptr;
     TopLists::Diagonal *diagonals = nullptr;
     TopLists::Job *jobs = nullptr;
     TopLists::Pair *pairs = nullptr;
-    int n_columns = 0, n_diagonals = 0, tiles = 0, temps = 0;
     int64_t entries = 0;           // elements of one direction's array
-    std::vector<int> stages;
+    std::vector<TopLists::Group> groups;
     void release();
     hipError_t upload(const TopLists &lists);
 };
@@ -65,6 +64,9 @@ struct DeviceTopLists {
 // hipErrorOutOfMemory, by then with some values overwritten.
 hipError_t fill_block_plan_on_device(const BlockPlan &P, const InverseArgs &args, const int *small, int n_small,
                                      const DeviceTopLists &tops, int float_bytes, void *mfwd, void *mbwd, void *mtop);
+// The work memory a fill takes at a time where one block does not need more:
+// 4 GiB, or what CHOLESPY_FILL_MIB allows.
+int64_t fill_work_bytes();
 // The blocks of P that `small` lists.
 std::vector<int> small_block_list(const BlockPlan &P);
 

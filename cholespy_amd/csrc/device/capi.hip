@@ -345,7 +345,7 @@ int upload_plan(cholespy_gpu_solver *s, const BlockPlan &P, const std::vector<in
     d.levels_fwd = d.levels_bwd = 0;
     for (int v : P.level_fwd) d.levels_fwd = std::max(d.levels_fwd, v + 1);
     for (int v : P.level_bwd) d.levels_bwd = std::max(d.levels_bwd, v + 1);
-    const TopLists tops = top_lists(P, blk_sys);
+    const TopLists tops = top_lists(P, blk_sys, fill_work_bytes());
     d.m_entries = P.moff[P.nblocks] + tops.entries;
     s->plan_copy[0] = P.start;
     s->plan_copy[1] = P.rptr;

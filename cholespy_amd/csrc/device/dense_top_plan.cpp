@@ -4,7 +4,7 @@
 
 namespace cholespy_amd {
 
-TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
+TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys, int64_t work_bytes) {
     TopLists L;
     std::vector<int> pack_bwd;
     int64_t fwd_units = 0, bwd_units = 0;
@@ -24,13 +24,41 @@ TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
             (fwd ? L.fwd : L.bwd).push_back(p);
         }
     };
-    // The jobs of all blocks, by stage.
+    // The jobs of the group's blocks, by stage.
     struct Pending {
         TopLists::Job job;
         int stage;
     };
     std::vector<Pending> pending;
     std::vector<int> temps_of_stage;
+    TopLists::Group group;
+    auto open = [&]() {
+        group = TopLists::Group();
+        group.columns[0] = (int)L.columns.size();
+        group.diagonals[0] = (int)L.diagonals.size();
+        group.fwd_units[0] = fwd_units;
+        group.bwd_units[0] = bwd_units;
+        pending.clear();
+        temps_of_stage.clear();
+    };
+    auto close = [&]() {
+        group.columns[1] = (int)L.columns.size();
+        group.diagonals[1] = (int)L.diagonals.size();
+        group.fwd_units[1] = fwd_units;
+        group.bwd_units[1] = bwd_units;
+        for (int t : temps_of_stage) group.temps = std::max(group.temps, t);
+        std::stable_sort(pending.begin(), pending.end(), [](const Pending &a, const Pending &b) {
+            return a.stage != b.stage ? a.stage < b.stage : a.job.count > b.job.count;
+        });
+        group.stages.assign(1, (int)L.jobs.size());
+        for (const Pending &q : pending) {
+            while ((int)group.stages.size() <= q.stage) group.stages.push_back((int)L.jobs.size());
+            L.jobs.push_back(q.job);
+        }
+        group.stages.push_back((int)L.jobs.size());
+        L.groups.push_back(group);
+    };
+    open();
     for (const BlockPlan::TopBlock &top : P.tops) {
         const int row0 = P.start[top.block], m = (int)top.parent.size(), sys = blk_sys ? (*blk_sys)[top.block] : 0;
         const int np = (m + kTopUnit - 1) / kTopUnit, nt = (m + kTopTile - 1) / kTopTile, per = kTopTile / kTopUnit;
@@ -43,12 +71,19 @@ TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
                 if (i > j && i / kTopUnit == j / kTopUnit) break;
             }
         std::vector<int> tile((size_t)nt * nt, -1);
+        int count = 0;
         for (int p = 0; p < np; ++p)
             for (int q = 0; q <= p; ++q)
-                if (has[(size_t)p * np + q]) {
-                    int &t = tile[(size_t)(p / per) * nt + q / per];
-                    if (t < 0) t = L.tiles++;
-                }
+                if (has[(size_t)p * np + q] && tile[(size_t)(p / per) * nt + q / per] < 0)
+                    tile[(size_t)(p / per) * nt + q / per] = count++;
+        // (Temporaries: at most the tiles below the diagonal.)
+        if (group.tiles > 0 && (int64_t)2 * (group.tiles + count) * kTopTileEntries * 8 > work_bytes) {
+            close();
+            open();
+        }
+        for (int &t : tile)
+            if (t >= 0) t += group.tiles;
+        group.tiles += count;
         const int map = (int)L.map.size();
         L.map.push_back(nt);
         L.map.insert(L.map.end(), tile.begin(), tile.end());
@@ -100,6 +135,7 @@ TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
                         }
         }
     }
+    if (group.tiles > 0) close();
     L.slots = std::max(slots[0], slots[1]);
     L.entries = std::max(fwd_units, bwd_units) * kTopUnitEntries;
     L.pack.resize((size_t)std::max(fwd_units, bwd_units), -1);
@@ -108,16 +144,6 @@ TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys) {
     auto longest = [](const DenseTopPanel &a, const DenseTopPanel &b) { return a.count > b.count; };
     std::stable_sort(L.fwd.begin(), L.fwd.end(), longest);
     std::stable_sort(L.bwd.begin(), L.bwd.end(), longest);
-    std::stable_sort(pending.begin(), pending.end(), [](const Pending &a, const Pending &b) {
-        return a.stage != b.stage ? a.stage < b.stage : a.job.count > b.job.count;
-    });
-    for (int t : temps_of_stage) L.temps = std::max(L.temps, t);
-    L.stages.assign(1, 0);
-    for (const Pending &q : pending) {
-        while ((int)L.stages.size() <= q.stage) L.stages.push_back((int)L.jobs.size());
-        L.jobs.push_back(q.job);
-    }
-    L.stages.push_back((int)L.jobs.size());
     return L;
 }
 

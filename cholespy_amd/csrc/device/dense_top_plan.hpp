@@ -63,19 +63,28 @@ struct TopLists {
     struct Pair {
         int a, b;                  // even: tile, tile; odd: tile, temporary tile
     };
-    int tiles = 0, temps = 0;
+    // Blocks in groups whose work arrays stay within a bound (a block alone may
+    // pass it); tiles and temporaries are counted from zero in each.
+    struct Group {
+        int tiles = 0, temps = 0;
+        int columns[2], diagonals[2];        // ranges of the lists below
+        int64_t fwd_units[2], bwd_units[2];
+        std::vector<int> stages;             // job ranges: stage s is [stages[s], stages[s + 1])
+    };
+    std::vector<Group> groups;
     std::vector<Column> columns;
     std::vector<int> map;          // per block: tiles across, then the tile of (i, j) at i * across + j, -1 = none
     std::vector<Diagonal> diagonals;
     std::vector<Job> jobs;
     std::vector<Pair> pairs;
-    std::vector<int> stages;       // job ranges: stage s is [stages[s], stages[s + 1])
     // Per unit of the fwd and then of the bwd array: tile * 16 + unit row in
     // it * 4 + unit column (-1: no such tile, zeros).
     std::vector<int> pack;
 };
 
-// blk_sys: the system of each block (null: one system).
-TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys);
+constexpr int64_t kTopWorkBytes = int64_t(4) << 30;
+
+// blk_sys: the system of each block (null: one system). work_bytes: a group's bound.
+TopLists top_lists(const BlockPlan &P, const std::vector<int> *blk_sys, int64_t work_bytes = kTopWorkBytes);
 
 }  // namespace cholespy_amd

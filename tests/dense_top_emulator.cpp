@@ -13,10 +13,11 @@
 //   - a NaN in the right-hand side of one tree of the elimination forest
 //     reaches the solution of another.
 //
-// Usage: dense_top_emulator FILE narrow|wide ROWS SHUFFLE
+// Usage: dense_top_emulator FILE narrow|wide ROWS SHUFFLE MIB
 // FILE as in plan_emulator.cpp; ROWS: the most rows of the top, whose levels
 // are then always worth it; SHUFFLE != 0: the factor renumbered first by a
-// random topological order (no postorder).
+// random topological order (no postorder); MIB: the work
+// arrays' bound, in groups.
 #include "block_plan.hpp"
 #include "dense_top_plan.hpp"
 
@@ -89,69 +90,81 @@ std::vector<int> random_topological(const Factor &f) {
 }
 
 // X in both packed arrays, unit by unit: element [unit][output][input].
-void form_inverse(const Factor &f, const BlockPlan &P, const TopLists &L, std::vector<double> &xf, std::vector<double> &xb) {
-    std::vector<double> D((size_t)L.tiles * kTopTileEntries, 0.0), T((size_t)L.temps * kTopTileEntries, NAN);
-    auto at = [](std::vector<double> &v, int tile, int i, int j) -> double & {
-        return v[(size_t)tile * kTopTileEntries + i + (size_t)j * kTopTile];
-    };
-    for (const auto &c : L.columns)
-        for (int p = f.cp[c.row0 + c.c]; p < f.cp[c.row0 + c.c + 1]; ++p) {
-            const int i = f.ri[p] - c.row0, nt = L.map[c.map];
-            check(i / kTopTile < nt, "an entry of a top column lies below its block");
-            const int tile = L.map[c.map + 1 + i / kTopTile * nt + c.c / kTopTile];
-            check(tile >= 0 && tile < L.tiles, "an entry of L has no tile");
-            at(D, tile, i % kTopTile, c.c % kTopTile) = f.v[p];
-        }
-    for (const auto &d : L.diagonals) {
-        std::vector<double> X((size_t)kTopTileEntries, 0.0);
-        for (int c = 0; c < d.rows; ++c)
-            for (int i = c; i < d.rows; ++i) {
-                double s = i == c ? 1.0 : 0.0;
-                for (int j = c; j < i; ++j) s -= at(D, d.tile, i, j) * X[(size_t)j + (size_t)c * kTopTile];
-                X[(size_t)i + (size_t)c * kTopTile] = s / at(D, d.tile, i, i);
-            }
-        std::copy(X.begin(), X.end(), D.begin() + (size_t)d.tile * kTopTileEntries);
-    }
-    for (size_t s = 0; s + 1 < L.stages.size(); ++s) {
-        const bool even = s % 2 == 0;
-        std::vector<double> &B = even ? D : T, &C = even ? T : D;
-        std::vector<std::pair<int, std::vector<double>>> results;   // a stage's jobs are independent
-        for (int q = L.stages[s]; q < L.stages[s + 1]; ++q) {
-            const auto &job = L.jobs[q];
-            check(job.out >= 0 && job.out < (even ? L.temps : L.tiles), "a job's result has no place");
-            std::vector<double> out((size_t)kTopTileEntries, 0.0);
-            for (int p = job.first; p < job.first + job.count; ++p) {
-                const auto &pr = L.pairs[p];
-                check(pr.a >= 0 && pr.a < L.tiles && pr.b >= 0 && pr.b < (even ? L.tiles : L.temps), "a pair's tile");
-                for (int j = 0; j < kTopTile; ++j)
-                    for (int k = 0; k < kTopTile; ++k) {
-                        const double b = at(B, pr.b, k, j);
-                        if (b != 0.0)
-                            for (int i = 0; i < kTopTile; ++i) out[(size_t)i + (size_t)j * kTopTile] += at(D, pr.a, i, k) * b;
-                    }
-            }
-            if (!even)
-                for (double &v : out) v = -v;
-            results.push_back({job.out, out});
-        }
-        for (auto &r : results) std::copy(r.second.begin(), r.second.end(), C.begin() + (size_t)r.first * kTopTileEntries);
-    }
+void form_inverse(const Factor &f, const TopLists &L, std::vector<double> &xf, std::vector<double> &xb) {
     const size_t units = (size_t)(L.entries / kTopUnitEntries);
     check(L.pack.size() == 2 * units, "one pack code a unit");
-    xf.assign(units * kTopUnitEntries, 0.0);
-    xb.assign(units * kTopUnitEntries, 0.0);
-    for (size_t u = 0; u < 2 * units; ++u) {
-        const int code = L.pack[u];
-        if (code < 0) continue;
-        check(code / 16 < L.tiles, "a unit's tile");
-        for (int o = 0; o < kTopUnit; ++o)
-            for (int i = 0; i < kTopUnit; ++i) {
-                const int r0 = code / 4 % 4 * kTopUnit, c0 = code % 4 * kTopUnit;
-                if (u < units) xf[(u * kTopUnit + o) * kTopUnit + i] = at(D, code / 16, r0 + o, c0 + i);
-                else xb[((u - units) * kTopUnit + o) * kTopUnit + i] = at(D, code / 16, r0 + i, c0 + o);
+    xf.assign(units * kTopUnitEntries, NAN);
+    xb.assign(units * kTopUnitEntries, NAN);
+    int columns = 0, diagonals = 0, jobs = 0;
+    int64_t fwd = 0, bwd = 0;
+    for (const TopLists::Group &g : L.groups) {
+        check(g.columns[0] == columns && g.diagonals[0] == diagonals && g.stages.front() == jobs && g.fwd_units[0] == fwd &&
+                  g.bwd_units[0] == bwd,
+              "groups follow one another");
+        columns = g.columns[1], diagonals = g.diagonals[1], jobs = g.stages.back(), fwd = g.fwd_units[1], bwd = g.bwd_units[1];
+        std::vector<double> D((size_t)g.tiles * kTopTileEntries, 0.0), T((size_t)g.temps * kTopTileEntries, NAN);
+        auto at = [](std::vector<double> &v, int tile, int i, int j) -> double & {
+            return v[(size_t)tile * kTopTileEntries + i + (size_t)j * kTopTile];
+        };
+        for (int q = g.columns[0]; q < g.columns[1]; ++q) {
+            const auto &c = L.columns[q];
+            for (int p = f.cp[c.row0 + c.c]; p < f.cp[c.row0 + c.c + 1]; ++p) {
+                const int i = f.ri[p] - c.row0, nt = L.map[c.map];
+                check(i / kTopTile < nt, "an entry of a top column lies below its block");
+                const int tile = L.map[c.map + 1 + i / kTopTile * nt + c.c / kTopTile];
+                check(tile >= 0 && tile < g.tiles, "an entry of L has no tile");
+                at(D, tile, i % kTopTile, c.c % kTopTile) = f.v[p];
+            }
+        }
+        for (int q = g.diagonals[0]; q < g.diagonals[1]; ++q) {
+            const auto &d = L.diagonals[q];
+            std::vector<double> X((size_t)kTopTileEntries, 0.0);
+            for (int c = 0; c < d.rows; ++c)
+                for (int i = c; i < d.rows; ++i) {
+                    double s = i == c ? 1.0 : 0.0;
+                    for (int j = c; j < i; ++j) s -= at(D, d.tile, i, j) * X[(size_t)j + (size_t)c * kTopTile];
+                    X[(size_t)i + (size_t)c * kTopTile] = s / at(D, d.tile, i, i);
+                }
+            std::copy(X.begin(), X.end(), D.begin() + (size_t)d.tile * kTopTileEntries);
+        }
+        for (size_t s = 0; s + 1 < g.stages.size(); ++s) {
+            const bool even = s % 2 == 0;
+            std::vector<double> &B = even ? D : T, &C = even ? T : D;
+            std::vector<std::pair<int, std::vector<double>>> results;   // a stage's jobs are independent
+            for (int q = g.stages[s]; q < g.stages[s + 1]; ++q) {
+                const auto &job = L.jobs[q];
+                check(job.out >= 0 && job.out < (even ? g.temps : g.tiles), "a job's result has no place");
+                std::vector<double> out((size_t)kTopTileEntries, 0.0);
+                for (int p = job.first; p < job.first + job.count; ++p) {
+                    const auto &pr = L.pairs[p];
+                    check(pr.a >= 0 && pr.a < g.tiles && pr.b >= 0 && pr.b < (even ? g.tiles : g.temps), "a pair's tile");
+                    for (int j = 0; j < kTopTile; ++j)
+                        for (int k = 0; k < kTopTile; ++k) {
+                            const double b = at(B, pr.b, k, j);
+                            if (b != 0.0)
+                                for (int i = 0; i < kTopTile; ++i) out[(size_t)i + (size_t)j * kTopTile] += at(D, pr.a, i, k) * b;
+                        }
+                }
+                if (!even)
+                    for (double &v : out) v = -v;
+                results.push_back({job.out, out});
+            }
+            for (auto &r : results) std::copy(r.second.begin(), r.second.end(), C.begin() + (size_t)r.first * kTopTileEntries);
+        }
+        for (int dir = 0; dir < 2; ++dir)
+            for (int64_t u = (dir ? g.bwd_units : g.fwd_units)[0]; u < (dir ? g.bwd_units : g.fwd_units)[1]; ++u) {
+                const int code = L.pack[(size_t)u + dir * units];
+                check(code < 16 * g.tiles, "a unit's tile");
+                for (int o = 0; o < kTopUnit; ++o)
+                    for (int i = 0; i < kTopUnit; ++i) {
+                        const int r0 = code / 4 % 4 * kTopUnit, c0 = code % 4 * kTopUnit;
+                        (dir ? xb : xf)[((size_t)u * kTopUnit + o) * kTopUnit + i] =
+                            code < 0 ? 0.0 : dir ? at(D, code / 16, r0 + i, c0 + o) : at(D, code / 16, r0 + o, c0 + i);
+                    }
             }
     }
-    (void)P;
+    check(columns == (int)L.columns.size() && diagonals == (int)L.diagonals.size() && jobs == (int)L.jobs.size(),
+          "groups cover the lists");
 }
 
 // The product of one direction: out = X in or X' in on the top rows.
@@ -291,7 +304,7 @@ std::vector<double> solve(const BlockPlan &P, const TopLists &L, const std::vect
     return z;
 }
 
-int run(const char *path, bool wide, int most, bool shuffle) {
+int run(const char *path, bool wide, int most, bool shuffle, int mib) {
     Factor f;
     FILE *fh = std::fopen(path, "rb");
     check(fh != nullptr, "cannot open the factor file");
@@ -324,9 +337,19 @@ int run(const char *path, bool wide, int most, bool shuffle) {
     }
     BlockPlan P = build_block_plan_structure(f.n, f.cp.data(), f.ri.data(), opt);
     fill_block_plan_values(P, f.cp.data(), f.ri.data(), f.v.data(), 1);
-    const TopLists L = top_lists(P, nullptr);
+    const TopLists L = top_lists(P, nullptr, (int64_t)mib << 20);
+    int tiles = 0, temps = 0;
+    size_t stages = 0;
+    for (const TopLists::Group &g : L.groups) {
+        std::set<int> blocks;
+        for (int q = g.columns[0]; q < g.columns[1]; ++q) blocks.insert(L.columns[q].row0);
+        check(blocks.size() == 1 || (int64_t)(g.tiles + g.temps) * kTopTileEntries * 8 <= (int64_t)mib << 20, "a group's bound");
+        tiles += g.tiles;
+        temps = std::max(temps, g.temps);
+        stages = std::max(stages, g.stages.size() - 1);
+    }
     std::vector<double> xf, xb;
-    form_inverse(f, P, L, xf, xb);
+    form_inverse(f, L, xf, xb);
     check_leaves(P, P.fwd_task, P.bwd_task, P.n_leaf_fwd, P.n_leaf_bwd);
     check_leaves(P, P.fwd_task_wide, P.bwd_task_wide, P.n_leaf_fwd_wide, P.n_leaf_bwd_wide);
 
@@ -364,21 +387,21 @@ int run(const char *path, bool wide, int most, bool shuffle) {
     const std::vector<double> zn = solve(P, L, xf, xb, wide, bn, true);
     for (int j = 0; j < f.n; ++j)
         check(root[j] == root[f.n - 1] ? std::isnan(zn[j]) : zn[j] == z[j], "a NaN reaches another tree");
-    std::printf("ok n %d top %d in %zu blocks of %d, trees %zu, panels %zu units %lld tiles %d temps %d stages %zu err %.1e\n", f.n,
-                top.rows, P.tops.size(), P.nblocks, trees.size(), L.fwd.size(), (long long)(L.entries / kTopUnitEntries), L.tiles,
-                L.temps, L.stages.size() - 1, err / scale);
+    std::printf("ok n %d top %d in %zu blocks of %d, trees %zu, panels %zu units %lld tiles %d temps %d stages %zu groups %zu err %.1e\n", f.n,
+                top.rows, P.tops.size(), P.nblocks, trees.size(), L.fwd.size(), (long long)(L.entries / kTopUnitEntries), tiles,
+                temps, stages, L.groups.size(), err / scale);
     return 0;
 }
 
 }  // namespace
 
 int main(int argc, char **argv) {
-    if (argc != 5) {
-        std::fprintf(stderr, "usage: %s FILE narrow|wide ROWS SHUFFLE\n", argv[0]);
+    if (argc != 6) {
+        std::fprintf(stderr, "usage: %s FILE narrow|wide ROWS SHUFFLE MIB\n", argv[0]);
         return 2;
     }
     try {
-        return run(argv[1], std::strcmp(argv[2], "wide") == 0, std::atoi(argv[3]), std::atoi(argv[4]) != 0);
+        return run(argv[1], std::strcmp(argv[2], "wide") == 0, std::atoi(argv[3]), std::atoi(argv[4]) != 0, std::atoi(argv[5]));
     } catch (const Failure &e) {
         std::printf("FAIL %s\n", e.what.c_str());
     } catch (const std::exception &e) {

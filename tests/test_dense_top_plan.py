@@ -74,8 +74,8 @@ def factors(tmp_path_factory):
 @pytest.mark.parametrize("rows", [0, 1, 15, 64, 200, 900, 7168])
 @pytest.mark.parametrize("case", sorted(CASES))
 def test_top_schedule_and_inverse(case, rows, shuffle, factors, emulator):
-    for kind in ("narrow", "wide"):
-        res = subprocess.run([str(emulator), str(factors[case]), kind, str(rows), str(shuffle)], capture_output=True,
+    for kind, mib in (("narrow", 4096), ("wide", 4)):
+        res = subprocess.run([str(emulator), str(factors[case]), kind, str(rows), str(shuffle), str(mib)], capture_output=True,
                              text=True, timeout=120)
         assert res.returncode == 0, (case, kind, rows, shuffle, res.stdout + res.stderr)
         print(kind, res.stdout.strip())
@@ -83,13 +83,19 @@ def test_top_schedule_and_inverse(case, rows, shuffle, factors, emulator):
 
 def test_inverse_is_stored_where_it_is_nonzero(factors, emulator):
     """A 61 x 47 grid as one top: a dense square would take 180 x 180 units."""
-    res = subprocess.run([str(emulator), str(factors["grid61x47"]), "narrow", "7168", "0"], capture_output=True, text=True)
+    res = subprocess.run([str(emulator), str(factors["grid61x47"]), "narrow", "7168", "0", "4096"], capture_output=True, text=True)
     assert "top 2867" in res.stdout and " units 2122 tiles 264 " in res.stdout, res.stdout
 
 
 def test_forest_top_has_a_block_per_tree(factors, emulator):
-    res = subprocess.run([str(emulator), str(factors["forest"]), "narrow", "7168", "0"], capture_output=True, text=True)
+    res = subprocess.run([str(emulator), str(factors["forest"]), "narrow", "7168", "0", "4096"], capture_output=True, text=True)
     assert "in 6 blocks of 6, trees 6" in res.stdout, res.stdout
     # Too many trees for a top of all rows: fewer levels, or none.
-    res = subprocess.run([str(emulator), str(factors["dust"]), "narrow", "7168", "0"], capture_output=True, text=True)
+    res = subprocess.run([str(emulator), str(factors["dust"]), "narrow", "7168", "0", "4096"], capture_output=True, text=True)
     assert "ok" in res.stdout and "top 470" not in res.stdout, res.stdout
+
+
+def test_groups_of_bounded_work(factors, emulator):
+    """32 KiB a tile, twice: the forest's six trees in several groups, each within 8 MiB."""
+    res = subprocess.run([str(emulator), str(factors["forest"]), "narrow", "7168", "0", "8"], capture_output=True, text=True)
+    assert res.returncode == 0 and " groups 2 " in res.stdout or " groups 3 " in res.stdout, res.stdout

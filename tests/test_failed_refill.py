@@ -73,3 +73,22 @@ def test_failed_autotune(monkeypatch, tmp_path):
     monkeypatch.delenv("CHOLESPY_FILL_MIB")
     s.refactorize(torch.tensor(v, device=DEV))
     _right(s, n, np.float32)
+
+
+@pytest.mark.parametrize("cls,dtype", [(CholeskySolverF, np.float32), (CholeskySolverD, np.float64)])
+def test_refill_in_groups(cls, dtype, monkeypatch):
+    """Less work memory than all blocks together take: one group after another
+    (the tops of three unconnected parts, and the large blocks below them)."""
+    monkeypatch.setenv("CHOLESPY_FILL_MIB", "48")
+    n, values, rows, cols = 0, [], [], []
+    for m in (9, 21, 24):
+        v, idx = workloads.grid3d_laplacian(m, 1.0)
+        values.append(v)
+        rows.append(idx[0] + n)
+        cols.append(idx[1] + n)
+        n += m ** 3
+    s = cls(n, *(torch.tensor(np.concatenate(a), device=DEV) for a in (rows, cols, values)), MatrixType.COO)
+    assert (s._plan_arrays()["fwd_task"][:, 3] == 4).any()
+    _right(s, n, dtype)
+    s.refactorize(torch.tensor(np.concatenate(values), device=DEV))
+    _right(s, n, dtype)
