@@ -434,9 +434,16 @@ hipError_t launch_dense_top(int float_bytes, const DenseTopArgs &args, int panel
     DenseTopArgs a = args;
     void *p[] = {&a};
     const void *kern = float_bytes == 4 ? dense_kernel<float>(a, max_k) : dense_kernel<double>(a, max_k);
-    if (max_k <= kNarrowTile) return hipLaunchKernel(kern, dim3(panels), dim3(kNarrowThreads), p, 0, stream);
     const int nt = max_k <= 16 ? 1 : (max_k <= 32 ? 2 : 4);
-    return hipLaunchKernel(kern, dim3(panels, (max_k + 16 * nt - 1) / (16 * nt)), dim3(kWideThreads), p, 0, stream);
+    constexpr int kMost = 1 << 21;   // (a launch takes fewer than 2^32 threads)
+    for (int lo = 0; lo < panels; lo += kMost, a.panels += kMost) {
+        const unsigned grid = (unsigned)std::min(kMost, panels - lo);
+        const hipError_t e = max_k <= kNarrowTile
+                                 ? hipLaunchKernel(kern, dim3(grid), dim3(kNarrowThreads), p, 0, stream)
+                                 : hipLaunchKernel(kern, dim3(grid, (max_k + 16 * nt - 1) / (16 * nt)), dim3(kWideThreads), p, 0, stream);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace cholespy_amd

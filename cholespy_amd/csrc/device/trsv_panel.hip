@@ -1100,8 +1100,17 @@ static hipError_t launch_leaf_impl(bool forward, const BlockPassArgs<F> &args, h
     void *p[] = {&a};
     const void *kern = forward ? reinterpret_cast<const void *>(&leaf_units<F, true>)
                                : reinterpret_cast<const void *>(&leaf_units<F, false>);
-    const long long per = kTaskThreads / kWave, units = (long long)a.n_leaf * a.leaf_chunks;
-    return hipLaunchKernel(kern, dim3((unsigned)((units + per - 1) / per)), dim3(kTaskThreads), p, 0, stream);
+    // (A launch takes fewer than 2^32 threads: up to 2^24 units.)
+    const int per = kTaskThreads / kWave, most = (1 << 24) / a.leaf_chunks;
+    for (int left = args.n_leaf; left > 0; left -= most) {
+        a.n_leaf = std::min(left, most);
+        const hipError_t e = hipLaunchKernel(kern, dim3((unsigned)((a.n_leaf * a.leaf_chunks + per - 1) / per)), dim3(kTaskThreads),
+                                             p, 0, stream);
+        if (e != hipSuccess) return e;
+        a.leaf_task += (size_t)a.n_leaf * kDevTaskInts;
+        if (a.leaf_trace) a.leaf_trace += 4 * (size_t)a.n_leaf;
+    }
+    return hipSuccess;
 }
 hipError_t launch_panel_leaf_f32(bool forward, const BlockPassArgs<float> &a, hipStream_t stream) {
     return launch_leaf_impl<float>(forward, a, stream);
