@@ -176,16 +176,17 @@ struct BlockPlan {
     int64_t nnz_l = 0;
 };
 
-// Builds the plan from L in compressed-column form (rows ascending,
-// diagonal first), postordered so that parent(j) > j.
+// Builds the plan, with its values, from L in compressed-column form (rows
+// ascending, diagonal first), postordered so that parent(j) > j. The CPU checks
+// of the schedule run on it; a solver forms the values on the GPU
+// (block_inverse.hip).
 BlockPlan build_block_plan(int n, const int *colptr, const int *rowidx, const double *val,
                            const BlockPlanOptions &opt);
 
 // The two halves of build_block_plan. The structure (blocks, R rows, slots,
-// levels, tasks) depends only on the pattern of L; fill_block_plan_values
-// (re)computes mfwd / mbwd for the values val of L with that pattern, on up
-// to `threads` host threads (0 = hardware count, at most 16). A numeric
-// refactorisation keeps the structure and refills the values.
+// levels, tasks) depends only on the pattern of L and is kept over numeric
+// refactorisations; fill_block_plan_values computes mfwd / mbwd, but for top
+// blocks, on up to `threads` host threads (0 = hardware count, at most 16).
 BlockPlan build_block_plan_structure(int n, const int *colptr, const int *rowidx, const BlockPlanOptions &opt);
 void fill_block_plan_values(BlockPlan &P, const int *colptr, const int *rowidx, const double *val, int threads);
 

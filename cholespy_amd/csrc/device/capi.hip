@@ -1052,8 +1052,9 @@ int solve_blocks(cholespy_gpu_solver *s, int k, const void *b, void *x, hipStrea
         if (is_panel_tile(tile)) {
             bf.ntasks = forward ? d.n_fwd_tasks_wide : d.n_bwd_tasks_wide;
             // Leaf units carry two tiles of 16 right-hand sides: for one tile
-            // the workgroups' own tasks stay (33^3 grid, k = 5, FP64: 139 us,
-            // 148 with units; icosphere(6), k = 8, FP32 80 and 90).
+            // the workgroups' own tasks stay (solves back to back, with a dense
+            // top of 4,512 and 3,488 rows: 33^3 grid, k = 5, FP64 139 us, 148 with
+            // units; icosphere(6), k = 8, FP32 80 and 90).
             const bool units = s->leaf_kernels && bf.max_k > 16;
             bf.n_leaf = units ? (forward ? d.n_leaf_fwd_wide : d.n_leaf_bwd_wide) : 0;
             bf.task = forward ? d.ftask_wide : d.btask_wide;
@@ -1395,9 +1396,11 @@ int cholespy_batch_finalize(cholespy_gpu_solver *s) {
     if (ns >= 8 && !std::getenv("CHOLESPY_SPLIT_GATHER")) opt.split_gather = 257;
     if (ns >= 8) opt.wide_list = false;
     // Levels of many systems overlap, so a dense top pays only where it ends
-    // the long unsplit tasks of each system's last levels: 64 grid systems, n
-    // 1k-20k, k 1-128: 1153 us without one, 1021 / 973 / 956 / 976 / 1051 us
-    // with up to 600 / 800 / 1000 / 1200 / 1600 rows.
+    // the long unsplit tasks of each system's last levels. No top, then up to
+    // 600 / 800 / 1000 / 1200 / 1600 / 3000 rows: 64 grid systems, n 1k-20k, k
+    // 1-128, FP32 759, 681 / 620 / 595 / 602 / 622 / 602 us; 256 of them, k
+    // 1-64, 1156, 1123 / 1130 / 1168 / 1106 / 1163 / 1209; 12 of n 2k-12k, k
+    // 1-8, FP64 123, 97 / 98 / 93 / 93 / 89 / 91.
     if (ns >= 8) opt.top_max_rows = 1000;
     std::vector<BlockPlan> plans((size_t)ns);
     std::vector<std::vector<int>> srcs((size_t)ns);
