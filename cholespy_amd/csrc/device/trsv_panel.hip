@@ -86,15 +86,10 @@ template <typename F, int NT, bool Forward> constexpr int batch_steps() {
 // (3 waves), 116 backward (4). FP32, up to 4 tiles: 4 waves forward, 5
 // backward. FP64 forward with up to 4 tiles: 3 waves (left alone the compiler
 // takes AGPRs and 2); with 8 tiles it would spill at more waves and keeps the
-// default; FP64 backward with up to 4 tiles: 3 waves. It fits 4 where a leaf
-// unit keeps one running sum, but that put the FP64 solve's error 9 to 13 %
-// above the workgroup tasks' (151 x 97 grid, k = 17: 3.96e-16 against 3.61e-16;
-// 3.61e-16 with two sums). 3 waves and two sums against 4 and one: 511 x 389
-// grid, k = 17 248 and 246 us, 311 x 189, k = 32 144 and 141, 33^3, k = 17 192
-// and 194, icosphere(6), k = 40 180 and 179; two sums at 4 waves spill: 254,
-// 145, 199, 181.
+// default; FP64 backward with up to 4 tiles fits 4 waves.
 template <typename F, int NT, bool Forward> constexpr int kMinWavesFor() {
     if (sizeof(F) == 4) return NT >= 8 ? 3 : 4;
+    if (!Forward) return NT <= 4 ? 4 : 1;
     return NT <= 4 ? 3 : 1;
 }
 // Backward tasks stage the R-row indices they read in LDS (up to this many).
@@ -526,8 +521,14 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int nsteps = (rows - first + 3) / 4, groups = (last - first + 15) / 16;
-    // Even and odd steps are summed apart (up to 40 steps of 4 rows:
-    // the rounding of one long running sum grows with its length).
+    // The steps run from the last rows up: M_B's largest entries, those near
+    // its diagonal, are added last, so that the sums before them round at their
+    // own small size. Downwards the FP64 solve's error was 9 to 13 % above that
+    // of the workgroup tasks (151 x 97 grid, k = 17: 3.96e-16 against 3.61e-16;
+    // upwards 3.43e-16), FP32's 1.07e-7 against 8.4e-8, at the same times. (Two
+    // sums in FP64 gave 3.61e-16 but spilled, or took a wave a SIMD: 64^3 grid,
+    // k = 32, backward 708 us against 632.) In FP32 even and odd steps are summed
+    // apart as well.
     Acc acc[kGroups][NT], odd[kGroups][NT];
 #pragma unroll
     for (int g = 0; g < kGroups; ++g)
@@ -539,6 +540,7 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
 #pragma unroll
     for (int n = 0; n < NT; ++n) tc[n] = min(t0 + 16 * n + l, k - 1);
     U av[2][kFly][kGroups], bb[2][kFly][NT];
+    auto rho_of = [&](int s) { return rows - 4 * (s + 1) + q; };
     auto vrow = [&](int rho) {
         const int zr = lds_int(rowidx, max(rho - m, 0));   // (y rows: not used)
         return rho < m ? yv + (long long)(a0 + rho) * k : zv + (long long)zr * k;
@@ -546,7 +548,7 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
     auto load = [&](int d, int s0) {
 #pragma unroll
         for (int u = 0; u < kFly; ++u) {
-            const int rho = min(first + 4 * (s0 + u) + q, rows - 1);
+            const int rho = max(rho_of(s0 + u), first);
 #pragma unroll
             for (int g = 0; g < kGroups; ++g) av[d][u][g] = as_bits(M[(unsigned)bwd_off32(m, rho, cc[g])]);
             const F *src = vrow(rho);
@@ -559,20 +561,20 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
         asm volatile("" : "+v"(s1));   // addresses computed again, not kept
         // (y rows never hold the sentinel.)
         settle<F>(bb[d], a.status, a.qa,
-                  [&](int u, int n) { return vrow(min(first + 4 * (s1 + u) + q, rows - 1)) + tc[n]; });
+                  [&](int u, int n) { return vrow(max(rho_of(s1 + u), first)) + tc[n]; });
 #pragma unroll
         for (int u = 0; u < kFly; ++u) {
-            const int rho = first + 4 * (s0 + u) + q;
+            const int rho = rho_of(s0 + u);
             F b[NT];
 #pragma unroll
-            for (int n = 0; n < NT; ++n) b[n] = rho < rows ? from_bits<F>(bb[d][u][n]) : F(0);
+            for (int n = 0; n < NT; ++n) b[n] = rho >= first ? from_bits<F>(bb[d][u][n]) : F(0);
 #pragma unroll
             for (int g = 0; g < kGroups; ++g)
                 if (g < groups) {
-                    const F x = rho < rows && rho >= first + 16 * g + l ? from_bits<F>(av[d][u][g]) : F(0);
+                    const F x = rho >= first + 16 * g + l ? from_bits<F>(av[d][u][g]) : F(0);
 #pragma unroll
                     for (int n = 0; n < NT; ++n) {
-                        Acc &sum = u % 2 ? odd[g][n] : acc[g][n];
+                        Acc &sum = sizeof(F) == 4 && u % 2 ? odd[g][n] : acc[g][n];
                         sum = Mfma<F>::step(x, b[n], sum);
                     }
                 }
@@ -591,7 +593,7 @@ __device__ __forceinline__ void leaf_backward_unit(const BlockPassArgs<F> &a, co
     for (int g = 0; g < kGroups; ++g)
 #pragma unroll
         for (int n = 0; n < NT; ++n)
-            acc[g][n] += odd[g][n];
+            if (sizeof(F) == 4) acc[g][n] += odd[g][n];
 #pragma unroll
     for (int g = 0; g < kGroups; ++g)
 #pragma unroll
