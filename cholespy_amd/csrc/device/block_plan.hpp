@@ -104,11 +104,12 @@ struct BlockPlanOptions {
     // (5,109; k = 17 258 -> 221), (7) FP64 none (163.6; 165.6 with 2,886 rows,
     // k = 17 291 and 272), 511 x 389 grid FP64 162.1 -> 151.6 (3,479; 153.1
     // with 6,114), 200 x 150 grid FP64 78.2 -> 51.6 (5,455), 33^3 grid FP64
-    // 154.8 -> 123.2 (4,507), 48^3 grid FP32 243.7 -> 230.9 (6,241). More right-
+    // 154.8 -> 123.2 (4,507), 48^3 grid FP32 243.7 -> 230.9 (6,241);
+    // k = 32, 64^3 grid (5,514) FP32 1035 -> 996, FP64 1412 -> 1375. More right-
     // hand sides gain more from the same cuts. Of tops of more rows than
     // top_max_rows only 33^3 was measured (6,565: FP32 101.8 -> 95.6, FP64
     // 123.2 -> 122.1): their inverse costs a refactorisation more.
-    double pass_us = 25.0, level_us = 3.0, level_gbs = 4000.0, top_us = 12.0, top_gbs = 4000.0;
+    double pass_us = 25.0, level_us = 3.0, level_gbs = 4000.0, top_us = 10.5, top_gbs = 4000.0;
     int64_t top_max_rows = 6400;
     bool top_forced = false;   // a top wherever a cut fits top_max_rows, estimate or not
     // Host threads for the dense block inverses (0 = hardware count, at most
