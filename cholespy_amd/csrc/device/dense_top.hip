@@ -14,7 +14,7 @@
 // two triangular ones keep the residual of the block passes. ||b - A x|| /
 // ||b||, k = 3, block passes / S^{-1} / X'(X r): 61 x 47 grid, shift 1e-4,
 // FP64 2.9e-16 / 3.6e-15 / 3.4e-16, FP32 1.4e-7 / 7.8e-7 / 9.7e-8; 16^3 grid,
-// kappa 1e6, FP64 3.2e-16 / 1.5e-12 / 1.0e-15. X is sparse where S^{-1} is
+// kappa 1e6, FP64 3.4e-16 / 1.5e-12 / 1.0e-15. X is sparse where S^{-1} is
 // full (dense_top_plan.hpp), so that the two read less, and are formed in less
 // time: refactorize + solve of a 100 x 60 grid, FP32, 2.37 ms with the values
 // formed on the host and no top, 7.1 with S^{-1}, 1.9 with X; 61 x 47 1.13 /
